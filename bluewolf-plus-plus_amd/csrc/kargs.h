@@ -17,12 +17,13 @@ typedef struct {
   const int32_t *idx_in;
   float *maxv;
   int32_t *argmax;
-  float *dgamma; /* rmsnorm_grad partials */
-  float *dbeta;
+  float *part_v;    /* axis 0: [bands][cols] partial maxima ... */
+  uint32_t *part_i; /* ... and their row indices */
   uint32_t rows;
   uint32_t cols;
   uint32_t ld;
   float eps;
+  uint32_t bands;
 } BwppRowArgs;
 
 /* GEMM: C = op(A)·op(B) (+bias) (->SiLU); see gemm.hip. */

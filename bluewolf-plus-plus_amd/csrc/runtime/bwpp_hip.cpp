@@ -76,9 +76,10 @@ struct BwppHip {
   hipFunction_t row_maxgrad_idx_v4 = nullptr;
   hipFunction_t row_maskgrad = nullptr;
   hipFunction_t col_maskgrad = nullptr;
-  hipFunction_t col_max = nullptr;
-  hipFunction_t col_maxgrad = nullptr;
-  hipFunction_t col_mask = nullptr;
+  hipFunction_t col_max_band = nullptr, col_max_final = nullptr;
+  hipFunction_t col_mask_apply[2] = {}, col_maxgrad_apply[2] = {};  // [16-byte rows]
+  hipFunction_t col_maxgrad = nullptr;                               // no workspace
+  hipFunction_t col_mask = nullptr;                                  // no workspace
   // bwpp_gemm_<bf16|f32>_t<TA><TB>_<e|f>: [dtype][ta][tb][full]
   hipFunction_t gemm[2][2][2][2] = {};
   hipFunction_t gemm_bf16_w8[2][2] = {};  // 8-wave full-tile bf16: [ta][tb]
@@ -117,6 +118,16 @@ struct BwppHip {
   // reuse across calls is safe.
   void *ws = nullptr;
   size_t ws_bytes = 0;
+  // Split scratch: partials of operators that also have a path without
+  // them.  One fixed allocation of kSplitBytes on first use, never moved
+  // (so captured plans stay valid whatever runs later), freed by
+  // bwpp_hip_destroy.  See split_scratch.
+  void *split = nullptr;
+  bool split_off = false;          // not available (again): callers take their other path
+  bool split_used = false;         // work on the current stream may use it
+  hipEvent_t split_ev = nullptr;   // recorded behind the last use when the stream changed ...
+  bool split_wait = false;         // ... which the next use waits for
+  bool plan_capture = false;  // bwpp_hip_plan_capture is recording this handle's launches
   // Device address of this device's scratch array (bwpp_scratch.hip), for
   // the allocation-free entry point; NULL with scratch_why set if the
   // lookup failed.
@@ -164,6 +175,38 @@ BwppHipStatus bwpp_hip_set_error(BwppHip *h, BwppHipStatus s, const char *fmt, .
 
 const void *bwpp_hip_workspace(const BwppHip *h) { return h ? h->ws : nullptr; }
 
+void bwpp_hip_set_plan_capture(BwppHip *h, bool on) { h->plan_capture = on; }
+
+void bwpp_hip_split_enter(BwppHip *h) {
+  if (h->split_wait) {
+    (void)hipStreamWaitEvent(h->stream, h->split_ev, 0);
+    h->split_wait = false;
+  }
+  h->split_used = h->split != nullptr;
+}
+
+namespace {
+
+// The stream changes: an event behind the old one's use of the split
+// scratch, which the next use waits for (and not the new stream itself,
+// which may be recording a graph that does not use it).
+void split_leave(BwppHip *h) {
+  if (!h->split_used) return;
+  (void)hipSetDevice(h->device);
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  bool ok = hipStreamIsCapturing(h->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+  if (ok && !h->split_ev) ok = hipEventCreateWithFlags(&h->split_ev, hipEventDisableTiming) == hipSuccess;
+  if (ok) ok = hipEventRecord(h->split_ev, h->stream) == hipSuccess;
+  if (!ok) {  // that use cannot be ordered from here: no further use
+    (void)hipGetLastError();
+    h->split_off = true;
+  }
+  h->split_wait = ok;
+  h->split_used = false;
+}
+
+}  // namespace
+
 namespace {
 
 BwppHipStatus resolve(BwppHip *h, const std::string &name, hipFunction_t *out) {
@@ -207,8 +250,12 @@ BwppHipStatus resolve_all(BwppHip *h) {
   } singles[] = {
       {"bwpp_row_maxgrad_idx", &h->row_maxgrad_idx}, {"bwpp_row_maxgrad_idx_v4", &h->row_maxgrad_idx_v4},
       {"bwpp_row_maskgrad", &h->row_maskgrad},       {"bwpp_col_maskgrad", &h->col_maskgrad},
-      {"bwpp_col_max", &h->col_max},                 {"bwpp_col_maxgrad", &h->col_maxgrad},
-      {"bwpp_col_mask", &h->col_mask},
+      {"bwpp_col_max_band", &h->col_max_band},       {"bwpp_col_max_final", &h->col_max_final},
+      {"bwpp_col_mask_apply", &h->col_mask_apply[0]},
+      {"bwpp_col_mask_apply_v4", &h->col_mask_apply[1]},
+      {"bwpp_col_maxgrad_apply", &h->col_maxgrad_apply[0]},
+      {"bwpp_col_maxgrad_apply_v4", &h->col_maxgrad_apply[1]},
+      {"bwpp_col_maxgrad", &h->col_maxgrad},         {"bwpp_col_mask", &h->col_mask},
       {"bwpp_silu_grad", &h->silu_grad},             {"bwpp_softmax_grad", &h->softmax_grad},
       {"bwpp_rmsnorm_grad", &h->rmsnorm_grad},       {"bwpp_col_partials_sum", &h->col_partials_sum},
       {"bwpp_reduce_sum_rows", &h->reduce_sum_rows}, {"bwpp_reduce_sum_cols", &h->reduce_sum_cols},
@@ -308,6 +355,32 @@ std::string library_dir() {
   return ".";
 }
 
+constexpr size_t kSplitBytes = 64u << 20;
+
+// `bytes` of the handle's split scratch, or NULL where the caller has to
+// take its path without one: more than it holds, no device memory, or a
+// capture that the caller records itself (such a graph may be replayed on
+// any stream beside this handle's other work, which the scratch does not
+// allow; a plan's graph is replayed on the handle's stream, after one eager
+// run, which has allocated it).
+void *split_scratch(BwppHip *h, size_t bytes) {
+  if (bytes > kSplitBytes || h->split_off) return nullptr;
+  if (h->plan_capture) return h->split;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(h->stream, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (st != hipStreamCaptureStatusNone) return nullptr;
+  if (!h->split && hipMalloc(&h->split, kSplitBytes) != hipSuccess) {
+    (void)hipGetLastError();
+    h->split = nullptr;
+    h->split_off = true;
+  }
+  if (h->split) bwpp_hip_split_enter(h);
+  return h->split;
+}
+
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 BwppHipStatus enter(BwppHip *h) {
@@ -404,6 +477,40 @@ BwppHipStatus check_rows(BwppHip *h, uint32_t rows, uint32_t cols, uint32_t ld) 
 
 }  // namespace
 
+namespace {
+
+// Blocks of the axis-0 kernels: 64 columns (or 64 chunks of four) wide, and
+// enough bands of rows to give every CU eight 4-wave blocks, each band at
+// least 32 rows (one trip of a wave's eight loads): at 4096 x 4096, 64 x 32
+// blocks (13.3 us; 64 x 1, no second pass, would be 64 blocks on 256 CUs).
+// Fewer than 64 rows stay in one band and one launch.
+uint32_t col_bands(const BwppHip *h, uint32_t rows, uint32_t cols) {
+  const uint64_t blocks = ((uint64_t)cols + 63) / 64, want = 8ull * (uint64_t)(h->cus > 0 ? h->cus : 256);
+  const uint64_t by_rows = std::max<uint64_t>(1, rows / 32u);
+  return (uint32_t)std::min<uint64_t>(std::min<uint64_t>(std::max<uint64_t>(1, want / blocks), by_rows), 512);
+}
+
+// Column maxima into a.maxv / a.argmax (either may be NULL); `part`: 8 *
+// bands * cols bytes, used when bands > 1.
+BwppHipStatus col_max_launch(BwppHip *h, BwppRowArgs a, uint32_t bands, void *part) {
+  a.bands = bands;
+  a.part_v = static_cast<float *>(part);
+  a.part_i = reinterpret_cast<uint32_t *>(a.part_v + (size_t)bands * a.cols);
+  const uint32_t gx = (uint32_t)(((uint64_t)a.cols + 63) / 64);
+  BwppHipStatus s = launch(h, h->col_max_band, gx, bands, 1, 256, a);
+  if (s != BWPP_HIP_OK || bands == 1) return s;
+  return launch(h, h->col_max_final, gx, 1, 1, 256, a);
+}
+
+BwppHipStatus col_apply_launch(BwppHip *h, hipFunction_t (&f)[2], const BwppRowArgs &a, bool vec) {
+  const uint64_t gx = vec ? ((uint64_t)a.cols + 255) / 256 : ((uint64_t)a.cols + 63) / 64;
+  const uint64_t want = 8ull * (uint64_t)(h->cus > 0 ? h->cus : 256);
+  const uint64_t gy = std::min<uint64_t>(std::max<uint64_t>(1, want / gx), ((uint64_t)a.rows + 15) / 16);
+  return launch(h, f[vec ? 1 : 0], (uint32_t)gx, (uint32_t)gy, 1, 256, a);
+}
+
+}  // namespace
+
 extern "C" {
 
 const char *bwpp_hip_status_string(BwppHipStatus s) {
@@ -483,10 +590,12 @@ BwppHipStatus bwpp_hip_create(BwppHip **out, int device, const char *code_object
 
 void bwpp_hip_destroy(BwppHip *h) {
   if (!h) return;
-  if (h->ws) {
+  if (h->ws || h->split) {
     (void)hipSetDevice(h->device);
     (void)hipStreamSynchronize(h->stream);
-    (void)hipFree(h->ws);
+    if (h->ws) (void)hipFree(h->ws);
+    if (h->split) (void)hipFree(h->split);
+    if (h->split_ev) (void)hipEventDestroy(h->split_ev);
   }
   for (hipModule_t m : h->modules) (void)hipModuleUnload(m);
   delete h;
@@ -496,6 +605,7 @@ BwppHipStatus bwpp_hip_set_stream(BwppHip *h, void *hip_stream) {
   if (!h) return BWPP_HIP_ERR_INVALID_ARG;
   const hipStream_t ns = (hipStream_t)hip_stream;
   if (ns == h->stream) return BWPP_HIP_OK;
+  split_leave(h);
   if (h->ws) {
     // The workspace (split-K partial planes, attention D rows, column
     // partials) is ordered on the handle's stream.  Work still queued on the
@@ -672,7 +782,10 @@ BwppHipStatus bwpp_hip_dispatch_reduce_max(BwppHip *h, const float *x, float *ma
   a.ld = ld;
   if (p.axis == 0) {
     if (p.cols == 0) return BWPP_HIP_OK;
-    return launch(h, h->col_max, (p.cols + 255) / 256, 1, 1, 256, a);
+    uint32_t bands = col_bands(h, p.rows, p.cols);
+    void *part = bands > 1 ? split_scratch(h, (size_t)bands * p.cols * 8u) : nullptr;
+    if (!part) bands = 1;
+    return col_max_launch(h, a, bands, part);
   }
   if (p.rows == 0) return BWPP_HIP_OK;
   if (p.cols == 0) return launch(h, h->row_gen[ROW_MAX], p.rows, 1, 1, 256, a);
@@ -692,7 +805,17 @@ BwppHipStatus bwpp_hip_dispatch_reduce_max_mask(BwppHip *h, const float *x, floa
   a.rows = p.rows;
   a.cols = p.cols;
   a.ld = ld;
-  if (p.axis == 0) return launch(h, h->col_mask, (p.cols + 255) / 256, 1, 1, 256, a);
+  if (p.axis == 0) {
+    const uint32_t bands = col_bands(h, p.rows, p.cols);
+    float *m = static_cast<float *>(split_scratch(h, (size_t)p.cols * 4u + (size_t)bands * p.cols * 8u));
+    if (!m) return launch(h, h->col_mask, (p.cols + 255) / 256, 1, 1, 256, a);
+    BwppRowArgs r = a;
+    r.maxv = m;
+    if ((s = col_max_launch(h, r, bands, m + p.cols)) != BWPP_HIP_OK) return s;
+    a.part_v = m;
+    return col_apply_launch(h, h->col_mask_apply, a,
+                            aligned16(x) && aligned16(mask) && p.cols % 4 == 0 && ld % 4 == 0);
+  }
   return row_dispatch(h, ROW_MASK, a, aligned16(x) && aligned16(mask) && (ld % 4 == 0));
 }
 
@@ -731,7 +854,18 @@ BwppHipStatus bwpp_hip_dispatch_reduce_max_grad_argmax(BwppHip *h, const float *
   a.rows = p.rows;
   a.cols = p.cols;
   a.ld = ld;
-  if (p.axis == 0) return launch(h, h->col_maxgrad, (p.cols + 255) / 256, 1, 1, 256, a);
+  if (p.axis == 0) {
+    if (!argmax) {
+      const uint32_t bands = col_bands(h, p.rows, p.cols);
+      int32_t *idx = static_cast<int32_t *>(split_scratch(h, (size_t)p.cols * 4u + (size_t)bands * p.cols * 8u));
+      if (!idx) return launch(h, h->col_maxgrad, (p.cols + 255) / 256, 1, 1, 256, a);
+      BwppRowArgs r = a;
+      r.argmax = idx;
+      if ((s = col_max_launch(h, r, bands, idx + p.cols)) != BWPP_HIP_OK) return s;
+      a.idx_in = idx;
+    }
+    return col_apply_launch(h, h->col_maxgrad_apply, a, aligned16(dx) && p.cols % 4 == 0 && ld % 4 == 0);
+  }
   if (argmax) {
     const bool vec = aligned16(dx) && (ld % 4 == 0);
     return launch(h, vec ? h->row_maxgrad_idx_v4 : h->row_maxgrad_idx, stream_grid(p.rows), 1, 1, 256, a);

@@ -452,10 +452,12 @@ extern "C" BwppHipStatus bwpp_hip_plan_capture(BwppHipPlan *p) {
   if (hipStreamSynchronize(st) != hipSuccess) return perr(p, BWPP_HIP_ERR_HIP, "stream synchronize failed");
   hipError_t e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return perr(p, BWPP_HIP_ERR_HIP, "hipStreamBeginCapture: %s", hipGetErrorString(e));
+  bwpp_hip_set_plan_capture(p->h, true);
   for (const Op &op : p->ops) {
     s = run_op(*p, op);
     if (s != BWPP_HIP_OK) break;
   }
+  bwpp_hip_set_plan_capture(p->h, false);
   hipGraph_t g = nullptr;
   e = hipStreamEndCapture(st, &g);
   if (s != BWPP_HIP_OK) {
@@ -482,6 +484,7 @@ extern "C" BwppHipStatus bwpp_hip_plan_replay(BwppHipPlan *p) {
     return perr(p, BWPP_HIP_ERR_INVALID_ARG,
                 "the handle's workspace was reallocated after capture (a larger op ran on it): capture again");
   hipStream_t st = static_cast<hipStream_t>(bwpp_hip_get_stream(p->h));
+  bwpp_hip_split_enter(p->h);
   hipError_t e = hipGraphLaunch(p->exec, st);
   if (e != hipSuccess) return perr(p, BWPP_HIP_ERR_HIP, "hipGraphLaunch: %s", hipGetErrorString(e));
   return BWPP_HIP_OK;
