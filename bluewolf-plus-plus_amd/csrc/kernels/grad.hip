@@ -51,8 +51,106 @@ extern "C" __global__ __launch_bounds__(256) void bwpp_silu_grad(const BwppGradA
     g.out[i] = silu_grad1(g.a[i], g.b[i]);
 }
 
-// Row-wise softmax_grad: one block per row (grid-stride); the dot product is
-// reduced in fp32 across the block, the second pass re-reads the row (L2).
+// Columns of a row that thread g of its group of GT threads holds in chunk
+// j, element e: runs of four (VEC: 128-bit accesses), or every GT-th column
+// (rows at any 4-byte address: 4-byte accesses, still 256 contiguous bytes
+// per wave and instruction).
+template <int GT, bool VEC>
+__device__ __forceinline__ uint32_t elem_col(int g, int j, int e) {
+  return VEC ? 4u * (uint32_t)(j * GT + g) + (uint32_t)e : (uint32_t)((4 * j + e) * GT + g);
+}
+
+// One thread's share of a row, v[4 j + e] = p[elem_col(j, e)]; columns past
+// the end re-read the last ones (callers zero or skip them), so the loads
+// issue without branches.
+template <int VPT, int GT, bool VEC, bool NT = true>
+__device__ __forceinline__ void load_share(float (&v)[4 * VPT], const float *p, int g, uint32_t cols) {
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    if constexpr (VEC) {
+      const uint32_t c = elem_col<GT, VEC>(g, j, 0);
+      const float *q = p + (c < cols ? c : cols - 4u);
+      const float4 t = NT ? load_nt4(q) : *reinterpret_cast<const float4 *>(q);
+      v[4 * j] = t.x, v[4 * j + 1] = t.y, v[4 * j + 2] = t.z, v[4 * j + 3] = t.w;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t c = elem_col<GT, VEC>(g, j, e);
+        v[4 * j + e] = p[c < cols ? c : cols - 1u];
+      }
+    }
+  }
+}
+template <int VPT, int GT, bool VEC, bool NT = true>
+__device__ __forceinline__ void store_share(float *p, const float (&v)[4 * VPT], int g, uint32_t cols) {
+#pragma unroll
+  for (int j = 0; j < VPT; ++j) {
+    if constexpr (VEC) {
+      const uint32_t c = elem_col<GT, VEC>(g, j, 0);
+      const float4 t = make_float4(v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]);
+      if (c < cols) {
+        if constexpr (NT) store_nt4(p + c, t);
+        else *reinterpret_cast<float4 *>(p + c) = t;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t c = elem_col<GT, VEC>(g, j, e);
+        if (c < cols) p[c] = v[4 * j + e];
+      }
+    }
+  }
+}
+
+// Row-wise softmax_grad with the row in registers: y and dy are read once.
+// WPR waves share a row (WPR = 1: four rows per block, no barrier); the
+// block holds one group of rows, so blocks overlap each other's loads and
+// reductions.  4096 x 4096: re-reading the row for the second pass with
+// 4-byte loads took 50.5 us, this 32.0 us (201 MB at 6.3 TB/s).
+template <int VPT, int WPR, bool VEC>
+__device__ __forceinline__ void softmax_grad_reg(const BwppGradArgs &g) {
+  constexpr int GT = 64 * WPR, kBlock = WPR >= 4 ? GT : 256;
+  __shared__ float red[kBlock / 64];
+  const int tid = (int)threadIdx.x, gi = tid % GT, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t row = blockIdx.x * (uint32_t)(kBlock / GT) + (uint32_t)(wave / WPR);
+  const uint32_t r = row < g.rows ? row : g.rows - 1u;
+  float y[4 * VPT], d[4 * VPT];
+  load_share<VPT, GT, VEC>(y, g.a + (size_t)r * g.ld, gi, g.cols);
+  load_share<VPT, GT, VEC>(d, g.b + (size_t)r * g.ld, gi, g.cols);
+  float dot = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4 * VPT; ++i)
+    if (elem_col<GT, VEC>(gi, i / 4, i % 4) < g.cols) dot += d[i] * y[i];
+  dot = wave_sum(dot);
+  if constexpr (WPR > 1) {
+    if ((tid & 63) == 0) red[wave] = dot;
+    __syncthreads();
+    dot = red[wave / WPR * WPR];
+#pragma unroll
+    for (int w = 1; w < WPR; ++w) dot += red[wave / WPR * WPR + w];
+  }
+  if (row >= g.rows) return;
+#pragma unroll
+  for (int i = 0; i < 4 * VPT; ++i) y[i] = y[i] * (d[i] - dot);
+  store_share<VPT, GT, VEC>(g.out + (size_t)row * g.ld, y, gi, g.cols);
+}
+
+#define BWPP_SOFTMAX_GRAD(VPT, WPR)                                                                \
+  extern "C" __global__ __launch_bounds__(WPR >= 4 ? 64 * WPR : 256) void                           \
+      bwpp_softmax_grad_v##VPT##_w##WPR(const BwppGradArgs g) {                                     \
+    softmax_grad_reg<VPT, WPR, true>(g);                                                           \
+  }                                                                                                \
+  extern "C" __global__ __launch_bounds__(WPR >= 4 ? 64 * WPR : 256) void                           \
+      bwpp_softmax_grad_v##VPT##_w##WPR##_u(const BwppGradArgs g) {                                 \
+    softmax_grad_reg<VPT, WPR, false>(g);                                                          \
+  }
+// Keep this list in sync with kGradCfgs in runtime/bwpp_hip.cpp.
+#define BWPP_GRAD_ALL_CFG(MAC) MAC(1, 1) MAC(2, 1) MAC(4, 1) MAC(2, 4) MAC(2, 8) MAC(4, 8)
+BWPP_GRAD_ALL_CFG(BWPP_SOFTMAX_GRAD)
+BWPP_SOFTMAX_GRAD(8, 8)
+
+// Longer rows: one block per row (grid-stride); the second pass re-reads
+// the row (L2).
 extern "C" __global__ __launch_bounds__(256) void bwpp_softmax_grad(const BwppGradArgs g) {
   __shared__ float red[4];
   for (uint32_t r = blockIdx.x; r < g.rows; r += gridDim.x) {
@@ -104,18 +202,166 @@ extern "C" __global__ __launch_bounds__(256) void bwpp_mean_square_final(const B
   if (threadIdx.x == 0) g.out2[0] = acc * (g.s_loss ? *g.s_loss : 1.0f);
 }
 
-// Row-wise rmsnorm_grad with per-block column partials of dgamma / dbeta
-// (summed by bwpp_col_partials_sum).  gamma NULL means 1; with g.acc,
-// dx = acc + the gradient (the residual branch's gradient added in the same
-// pass; acc may be dx itself, each element being read before it is written
-// by the same thread).
+// rmsnorm_grad with the row in registers: x, dy (and acc) are read once,
+// WPR waves share a row, and a block strides over rows with the next row's
+// loads in flight while it reduces the current one; the dgamma / dbeta
+// column sums stay in registers and leave once per block as a partial row
+// (summed by bwpp_col_partials_sum; rows that share a block with WPR = 1
+// first meet in LDS).  The two row sums take one barrier: the LDS slots
+// alternate between rows.  gamma NULL means 1; with g.acc, dx = acc + the
+// gradient (acc may be dx itself: a thread has read its acc elements before
+// it writes them).  4096 x 4096 with dgamma and dbeta: two passes over the
+// row and per-element LDS accumulators took 148 us, this 31.4 us (201 MB
+// and 8 MB of partials).
+//
+// No contraction anywhere in the row's arithmetic: with plain roundings
+// every copy of the code gives the same bits, and dx = acc + gradient is
+// exactly the two ops.
+template <int VPT, int WPR, bool VEC>
+__device__ __forceinline__ void rmsnorm_grad_reg(const BwppGradArgs &g) {
+#pragma clang fp contract(off)
+  constexpr int GT = 64 * WPR, kBlock = WPR >= 4 ? GT : 256, kRows = kBlock / GT, E = 4 * VPT;
+  // One wave per row (rows of at most 1024 columns): no prefetch, the block's
+  // other rows cover the latency, and cached accesses, such rows mostly being
+  // a layer's own, just written (4096 x 1024: 14.5 us; with prefetch and
+  // non-temporal accesses 15.3).
+  constexpr bool kPrefetch = WPR > 1 && (VEC || VPT < 4), kNT = WPR > 1;
+  __shared__ float red[2][2][kBlock / 64];
+  extern __shared__ float colacc[];  // [kRows][2][cols] when partials are requested and kRows > 1
+  const int tid = (int)threadIdx.x, gi = tid % GT, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t sub = (uint32_t)(wave / WPR), cols = g.cols;
+  const bool parts = g.part_g != nullptr, has_acc = g.acc != nullptr;
+  float gm[E], ag[E], ab[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    gm[i] = 1.0f;
+    ag[i] = ab[i] = 0.0f;
+  }
+  if (g.gamma) load_share<VPT, GT, VEC, false>(gm, g.gamma, gi, cols);
+  struct Row {
+    float x[E], d[E], a[E];
+  };
+  auto load = [&](uint32_t row, Row &v) {
+    const size_t at = (size_t)(row < g.rows ? row : g.rows - 1u) * g.ld;
+    load_share<VPT, GT, VEC, kNT>(v.x, g.a + at, gi, cols);
+    load_share<VPT, GT, VEC, kNT>(v.d, g.b + at, gi, cols);
+    if (has_acc) load_share<VPT, GT, VEC, kNT>(v.a, g.acc + at, gi, cols);
+  };
+  auto process = [&](uint32_t row, Row &v, int slot) {
+    const bool valid = row < g.rows;
+    float ss = 0.0f, t = 0.0f;
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      if (!valid || elem_col<GT, VEC>(gi, i / 4, i % 4) >= cols) v.x[i] = v.d[i] = 0.0f;
+      ss += v.x[i] * v.x[i];
+      t += v.x[i] * gm[i] * v.d[i];
+    }
+    ss = wave_sum(ss);
+    t = wave_sum(t);
+    if constexpr (WPR > 1) {
+      if ((tid & 63) == 0) {
+        red[slot][0][wave] = ss;
+        red[slot][1][wave] = t;
+      }
+      __syncthreads();
+      const int w0 = wave / WPR * WPR;
+      ss = red[slot][0][w0];
+      t = red[slot][1][w0];
+#pragma unroll
+      for (int w = 1; w < WPR; ++w) {
+        ss += red[slot][0][w0 + w];
+        t += red[slot][1][w0 + w];
+      }
+    }
+    const float inv = 1.0f / sqrtf(ss / (float)cols + g.eps);
+    const float mdot = inv * t / (float)cols;  // mean(xhat * gamma * dy)
+    float o[E];
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const float h = v.x[i] * inv;
+      o[i] = inv * (gm[i] * v.d[i] - h * mdot);
+      o[i] = has_acc ? v.a[i] + o[i] : o[i];  // acc: a separate rounded add
+      ag[i] += v.d[i] * h;
+      ab[i] += v.d[i];
+    }
+    if (valid) store_share<VPT, GT, VEC, kNT>(g.out + (size_t)row * g.ld, o, gi, cols);
+  };
+  const uint32_t ngroups = (g.rows + kRows - 1) / kRows;
+  uint32_t grp = blockIdx.x;
+  if constexpr (!kPrefetch) {
+    for (int slot = 0; grp < ngroups; grp += gridDim.x, slot ^= 1) {
+      Row v;
+      load(grp * kRows + sub, v);
+      process(grp * kRows + sub, v, slot);
+    }
+  } else if (grp < ngroups) {
+    // Two rows per trip so that the buffers alternate without copies; the
+    // last row of a block is processed on a path of its own, so that inside
+    // the loop the next row's loads are issued unconditionally.
+    Row ra, rb;
+    load(grp * kRows + sub, ra);
+    for (;;) {
+      uint32_t next = grp + gridDim.x;
+      if (next >= ngroups) {
+        process(grp * kRows + sub, ra, 0);
+        break;
+      }
+      load(next * kRows + sub, rb);
+      process(grp * kRows + sub, ra, 0);
+      grp = next;
+      next = grp + gridDim.x;
+      if (next >= ngroups) {
+        process(grp * kRows + sub, rb, 1);
+        break;
+      }
+      load(next * kRows + sub, ra);
+      process(grp * kRows + sub, rb, 1);
+      grp = next;
+    }
+  }
+  if (!parts) return;  // block-uniform
+  if constexpr (kRows == 1) {
+    store_share<VPT, GT, VEC>(g.part_g + (size_t)blockIdx.x * cols, ag, gi, cols);
+    store_share<VPT, GT, VEC>(g.part_b + (size_t)blockIdx.x * cols, ab, gi, cols);
+  } else {
+    float *mine = colacc + (size_t)sub * 2 * cols;
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const uint32_t c = elem_col<GT, VEC>(gi, i / 4, i % 4);
+      if (c < cols) {
+        mine[c] = ag[i];
+        mine[cols + c] = ab[i];
+      }
+    }
+    __syncthreads();
+    for (uint32_t c = threadIdx.x; c < cols; c += kBlock) {
+      float sg = 0.0f, sb = 0.0f;
+#pragma unroll
+      for (int w = 0; w < kRows; ++w) {
+        sg += colacc[(size_t)w * 2 * cols + c];
+        sb += colacc[(size_t)w * 2 * cols + cols + c];
+      }
+      g.part_g[(size_t)blockIdx.x * cols + c] = sg;
+      g.part_b[(size_t)blockIdx.x * cols + c] = sb;
+    }
+  }
+}
+
+#define BWPP_RMSNORM_GRAD(VPT, WPR)                                                                \
+  extern "C" __global__ __launch_bounds__(WPR >= 4 ? 64 * WPR : 256) void                           \
+      bwpp_rmsnorm_grad_v##VPT##_w##WPR(const BwppGradArgs g) {                                     \
+    rmsnorm_grad_reg<VPT, WPR, true>(g);                                                           \
+  }                                                                                                \
+  extern "C" __global__ __launch_bounds__(WPR >= 4 ? 64 * WPR : 256) void                           \
+      bwpp_rmsnorm_grad_v##VPT##_w##WPR##_u(const BwppGradArgs g) {                                 \
+    rmsnorm_grad_reg<VPT, WPR, false>(g);                                                          \
+  }
+BWPP_GRAD_ALL_CFG(BWPP_RMSNORM_GRAD)
+
+// Rows of more than 8192 columns (no partials there): one block per row,
+// the row read twice.
 extern "C" __global__ __launch_bounds__(256) void bwpp_rmsnorm_grad(const BwppGradArgs g) {
   __shared__ float red[4];
-  extern __shared__ float colacc[];  // [2][cols] when partials are requested
-  const bool parts = g.part_g != nullptr;
-  if (parts)
-    for (uint32_t c = threadIdx.x; c < 2 * g.cols; c += 256) colacc[c] = 0.0f;
-  __syncthreads();
   for (uint32_t r = blockIdx.x; r < g.rows; r += gridDim.x) {
     const float *x = g.a + (size_t)r * g.ld;
     const float *dy = g.b + (size_t)r * g.ld;
@@ -143,156 +389,9 @@ extern "C" __global__ __launch_bounds__(256) void bwpp_rmsnorm_grad(const BwppGr
       } else {
         dx[c] = v;
       }
-      if (parts) {
-        colacc[c] += d * xh;
-        colacc[g.cols + c] += d;
-      }
-    }
-  }
-  if (parts) {
-    __syncthreads();
-    for (uint32_t c = threadIdx.x; c < g.cols; c += 256) {
-      g.part_g[(size_t)blockIdx.x * g.cols + c] = colacc[c];
-      g.part_b[(size_t)blockIdx.x * g.cols + c] = colacc[g.cols + c];
     }
   }
 }
-
-// rmsnorm_grad for 16-byte rows of at most 256 * VPT columns: one wave per
-// row (lane l owns float4 chunks l, l + 64, ...), so the two row sums are
-// wave reductions with no block barrier inside the row loop; the block's 4
-// waves stride over rows, each keeping its dgamma / dbeta column sums in
-// registers, and combine them once through LDS at the end into the block's
-// partial row (summed by bwpp_col_partials_sum).  Same arithmetic as
-// bwpp_rmsnorm_grad.  A row's loads (x, dy and acc) are all issued before
-// its first use; chunks past the row end re-read the row's last chunk and
-// are zeroed where they are used.
-template <int VPT>
-__device__ __forceinline__ void rmsnorm_grad_wave(const BwppGradArgs &g) {
-  extern __shared__ float colacc[];  // [4 waves][2][cols] when partials are requested
-  // wave is uniform: through readfirstlane the row pointers stay in SGPRs.
-  const int lane = (int)threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const uint32_t cols = g.cols;
-  const bool parts = g.part_g != nullptr;
-  float4 gm[VPT], ag[VPT], ab[VPT];
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) {
-    const uint32_t c = 4u * (uint32_t)(lane + 64 * j);
-    gm[j] = make_float4(1.f, 1.f, 1.f, 1.f);
-    if (g.gamma && c < cols) gm[j] = *reinterpret_cast<const float4 *>(g.gamma + c);
-    ag[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-    ab[j] = ag[j];
-  }
-  // One row's operands: x, dy and (when accumulating) acc.  acc is either
-  // dx itself or disjoint from it, so reading it ahead of the row's stores
-  // is exact: a lane reads each acc element before it writes that element.
-  struct Row {
-    float4 x[VPT], d[VPT], a[VPT];
-  };
-  const bool has_acc = g.acc != nullptr;
-  auto load = [&](uint32_t r, Row &v) {
-    const float *x = g.a + (size_t)r * g.ld;
-    const float *dy = g.b + (size_t)r * g.ld;
-    const float *ac = g.acc + (size_t)r * g.ld;
-#pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-      const uint32_t c = 4u * (uint32_t)(lane + 64 * j);
-      const uint32_t cc = c < cols ? c : cols - 4u;
-      v.x[j] = *reinterpret_cast<const float4 *>(x + cc);
-      v.d[j] = *reinterpret_cast<const float4 *>(dy + cc);
-      if (has_acc) v.a[j] = *reinterpret_cast<const float4 *>(ac + cc);
-    }
-  };
-  auto process = [&](uint32_t r, Row &v) {
-    // No contraction anywhere in the row's arithmetic: the compiler may
-    // duplicate this body (with / without acc) and would be free to fuse
-    // different products in each copy; with plain roundings every copy
-    // gives the same bits, and dx = acc + gradient is exactly the two ops.
-#pragma clang fp contract(off)
-    float *dx = g.out + (size_t)r * g.ld;
-    float ss = 0.0f, t = 0.0f;
-#pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-      // Zero the re-read chunks past the row end (component-wise selects:
-      // a float4-valued ?: can go through memory).
-      const bool in = 4u * (uint32_t)(lane + 64 * j) < cols;
-      auto keep = [in](float4 q) {
-        return make_float4(in ? q.x : 0.f, in ? q.y : 0.f, in ? q.z : 0.f, in ? q.w : 0.f);
-      };
-      v.x[j] = keep(v.x[j]);
-      v.d[j] = keep(v.d[j]);
-      ss += (v.x[j].x * v.x[j].x + v.x[j].y * v.x[j].y) + (v.x[j].z * v.x[j].z + v.x[j].w * v.x[j].w);
-      t += (v.x[j].x * gm[j].x * v.d[j].x + v.x[j].y * gm[j].y * v.d[j].y) +
-           (v.x[j].z * gm[j].z * v.d[j].z + v.x[j].w * gm[j].w * v.d[j].w);
-    }
-    ss = wave_sum(ss);
-    t = wave_sum(t);
-    const float inv = 1.0f / sqrtf(ss / (float)cols + g.eps);
-    const float mdot = inv * t / (float)cols;  // mean(xhat * gamma * dy)
-#pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-      const uint32_t c = 4u * (uint32_t)(lane + 64 * j);
-      if (c >= cols) continue;
-      float4 h, o;
-      h.x = v.x[j].x * inv;
-      h.y = v.x[j].y * inv;
-      h.z = v.x[j].z * inv;
-      h.w = v.x[j].w * inv;
-      o.x = inv * (gm[j].x * v.d[j].x - h.x * mdot);
-      o.y = inv * (gm[j].y * v.d[j].y - h.y * mdot);
-      o.z = inv * (gm[j].z * v.d[j].z - h.z * mdot);
-      o.w = inv * (gm[j].w * v.d[j].w - h.w * mdot);
-      o.x = has_acc ? v.a[j].x + o.x : o.x;  // acc: a separate rounded add
-      o.y = has_acc ? v.a[j].y + o.y : o.y;
-      o.z = has_acc ? v.a[j].z + o.z : o.z;
-      o.w = has_acc ? v.a[j].w + o.w : o.w;
-      *reinterpret_cast<float4 *>(dx + c) = o;
-      ag[j].x += v.d[j].x * h.x;
-      ag[j].y += v.d[j].y * h.y;
-      ag[j].z += v.d[j].z * h.z;
-      ag[j].w += v.d[j].w * h.w;
-      ab[j].x += v.d[j].x;
-      ab[j].y += v.d[j].y;
-      ab[j].z += v.d[j].z;
-      ab[j].w += v.d[j].w;
-    }
-  };
-  Row ra;
-  for (uint32_t r = blockIdx.x * 4u + (uint32_t)wave; r < g.rows; r += gridDim.x * 4u) {
-    load(r, ra);
-    process(r, ra);
-  }
-  if (!parts) return;  // block-uniform
-  float *mine = colacc + (size_t)wave * 2 * cols;
-#pragma unroll
-  for (int j = 0; j < VPT; ++j) {
-    const uint32_t c = 4u * (uint32_t)(lane + 64 * j);
-    if (c < cols) {
-      *reinterpret_cast<float4 *>(mine + c) = ag[j];
-      *reinterpret_cast<float4 *>(mine + cols + c) = ab[j];
-    }
-  }
-  __syncthreads();
-  for (uint32_t c = threadIdx.x; c < cols; c += 256) {
-    float sg = 0.0f, sb = 0.0f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      sg += colacc[(size_t)w * 2 * cols + c];
-      sb += colacc[(size_t)w * 2 * cols + cols + c];
-    }
-    g.part_g[(size_t)blockIdx.x * cols + c] = sg;
-    g.part_b[(size_t)blockIdx.x * cols + c] = sb;
-  }
-}
-
-#define BWPP_RMSNORM_GRAD_WAVE(VPT)                                                                 \
-  extern "C" __global__ __launch_bounds__(256) void bwpp_rmsnorm_grad_w##VPT(const BwppGradArgs g) { \
-    rmsnorm_grad_wave<VPT>(g);                                                                      \
-  }
-BWPP_RMSNORM_GRAD_WAVE(1)
-BWPP_RMSNORM_GRAD_WAVE(2)
-BWPP_RMSNORM_GRAD_WAVE(4)
-BWPP_RMSNORM_GRAD_WAVE(8)
 
 // out[c] = sum_p part[p][c] for the two partial arrays (dgamma, dbeta); the
 // outputs may be NULL.  A block owns 16 columns: thread (g, c) of 16 x 16
@@ -353,16 +452,35 @@ extern "C" __global__ __launch_bounds__(256) void bwpp_reduce_sum_rows(const Bwp
   }
 }
 
-// reduce_sum over rows (axis 0): column partials over row bands (blockIdx.y)
-// into part_g, then bwpp_col_partials_sum.
+// reduce_sum over rows (axis 0): a block owns 64 columns x one band of rows
+// (blockIdx.y), its 4 waves every fourth row with 8 rows' loads in flight;
+// the band sums go to part_g for bwpp_col_partials_sum, or with one band to
+// out.  4096 x 4096: 36.4 us with a serial walk of 64-row bands, 13.2 us
+// so.
 extern "C" __global__ __launch_bounds__(256) void bwpp_reduce_sum_cols(const BwppGradArgs g) {
-  const uint32_t c = blockIdx.x * 256u + threadIdx.x;
-  if (c >= g.cols) return;
-  const uint32_t band = (g.rows + gridDim.y - 1) / gridDim.y;
-  const uint32_t r0 = blockIdx.y * band, r1 = min(g.rows, r0 + band);
+  __shared__ float red[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t c = blockIdx.x * 64u + (uint32_t)lane;
+  const uint64_t band = ((uint64_t)g.rows + gridDim.y - 1) / gridDim.y;
+  const uint64_t r0 = band * blockIdx.y, r1 = min((uint64_t)g.rows, r0 + band);
   float s = 0.0f;
-  for (uint32_t r = r0; r < r1; ++r) s += g.a[(size_t)r * g.ld + c];
-  g.part_g[(size_t)blockIdx.y * g.cols + c] = s;
+  if (c < g.cols) {
+    const float *x = g.a + c;
+    uint64_t r = r0 + (uint64_t)wave;
+    for (; r + 28 < r1; r += 32) {
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = x[(r + 4 * i) * g.ld];
+      s += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    }
+    for (; r < r1; r += 4) s += x[r * g.ld];
+  }
+  red[wave][lane] = s;
+  __syncthreads();
+  if (wave != 0 || c >= g.cols) return;
+  s = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+  if (gridDim.y > 1) g.part_g[(size_t)blockIdx.y * g.cols + c] = s;
+  else g.out[c] = s;
 }
 
 // Binary elementwise with broadcasting of b, and broadcast itself (op 4:

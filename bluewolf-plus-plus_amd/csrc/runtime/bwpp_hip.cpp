@@ -49,6 +49,10 @@ const RowCfg kRowCfgs[kRowNCfg] = {{1, 1}, {2, 1}, {4, 1}, {8, 1}, {16, 1}, {2, 
 inline uint32_t row_capacity(const RowCfg &c) { return 256u * (uint32_t)c.wpr * (uint32_t)c.vpt; }
 inline uint32_t row_block(const RowCfg &c) { return c.wpr >= 4 ? 64u * (uint32_t)c.wpr : 256u; }
 inline uint32_t row_rows_per_block(const RowCfg &c) { return row_block(c) / (64u * (uint32_t)c.wpr); }
+// Row-in-register gradient kernels (grad.hip, BWPP_GRAD_ALL_CFG); the last
+// one exists for softmax_grad only.
+constexpr int kGradNCfg = 7;
+const RowCfg kGradCfgs[kGradNCfg] = {{1, 1}, {2, 1}, {4, 1}, {2, 4}, {2, 8}, {4, 8}, {8, 8}};
 int find_cfg(int vpt, int wpr) {
   for (int i = 0; i < kRowNCfg; ++i)
     if (kRowCfgs[i].vpt == vpt && kRowCfgs[i].wpr == wpr) return i;
@@ -109,7 +113,8 @@ struct BwppHip {
   hipFunction_t attn_f32_dsum[2] = {}, attn_f32_dkdv_ds[2][2] = {}, attn_f32_dq_ds[2][2] = {};
   uint64_t attn_ds_max = 8ull << 30;  // BWPP_ATTN_BWD_DS_MB: largest dS^T workspace in bytes (0: scheme off)
   hipFunction_t attn_conv_to_f32 = nullptr, attn_conv_to_bf16 = nullptr;  // bf16 <-> fp32 operand copies
-  hipFunction_t rmsnorm_grad_w[4] = {};  // wave-per-row rmsnorm_grad, 256 / 512 / 1024 / 2048 columns
+  hipFunction_t rmsnorm_grad_reg[kGradNCfg - 1][2] = {};  // [kGradCfgs][16-byte rows]
+  hipFunction_t softmax_grad_reg[kGradNCfg][2] = {};
   hipFunction_t silu_grad = nullptr, softmax_grad = nullptr, rmsnorm_grad = nullptr, col_partials_sum = nullptr,
                 reduce_sum_rows = nullptr, reduce_sum_cols = nullptr, elementwise = nullptr,
                 mean_square_part = nullptr, mean_square_final = nullptr, copy_multi = nullptr;
@@ -262,8 +267,6 @@ BwppHipStatus resolve_all(BwppHip *h) {
       {"bwpp_mean_square_part", &h->mean_square_part}, {"bwpp_mean_square_final", &h->mean_square_final},
       {"bwpp_copy_multi", &h->copy_multi},
       {"bwpp_elementwise", &h->elementwise},         {"bwpp_gemm_f32_splitk_reduce", &h->gemm_f32_reduce},
-      {"bwpp_rmsnorm_grad_w1", &h->rmsnorm_grad_w[0]}, {"bwpp_rmsnorm_grad_w2", &h->rmsnorm_grad_w[1]},
-      {"bwpp_rmsnorm_grad_w4", &h->rmsnorm_grad_w[2]}, {"bwpp_rmsnorm_grad_w8", &h->rmsnorm_grad_w[3]},
       {"bwpp_attn_conv_bf16_to_f32", &h->attn_conv_to_f32}, {"bwpp_attn_conv_f32_to_bf16", &h->attn_conv_to_bf16},
       {"bwpp_attn_bwd_bf16_mfma_d128_dkdv_w8", &h->attn_bf16_dkdv_w8[0]},
       {"bwpp_attn_bwd_bf16_mfma_d128_causal_dkdv_w8", &h->attn_bf16_dkdv_w8[1]},
@@ -287,6 +290,14 @@ BwppHipStatus resolve_all(BwppHip *h) {
   };
   for (auto &e : singles)
     if ((s = resolve(h, e.name, e.slot)) != BWPP_HIP_OK) return s;
+  for (int c = 0; c < kGradNCfg; ++c)
+    for (int vec = 0; vec < 2; ++vec) {
+      const std::string n = "_v" + std::to_string(kGradCfgs[c].vpt) + "_w" + std::to_string(kGradCfgs[c].wpr) +
+                            (vec ? "" : "_u");
+      if ((s = resolve(h, "bwpp_softmax_grad" + n, &h->softmax_grad_reg[c][vec])) != BWPP_HIP_OK) return s;
+      if (c < kGradNCfg - 1 && (s = resolve(h, "bwpp_rmsnorm_grad" + n, &h->rmsnorm_grad_reg[c][vec])) != BWPP_HIP_OK)
+        return s;
+    }
   for (int dt = 0; dt < 2; ++dt)
     for (int ta = 0; ta < 2; ++ta)
       for (int tb = 0; tb < 2; ++tb)
@@ -1570,6 +1581,15 @@ BwppHipStatus ensure_ws(BwppHip *h, size_t bytes) {
   return BWPP_HIP_OK;
 }
 
+// Smallest of the first n kGradCfgs that holds a row of `cols`, or -1: one
+// wave per row up to 1024 columns (no barrier), then as many waves as keep
+// the row at two chunks a thread, then more chunks.
+int grad_cfg(uint32_t cols, int n) {
+  for (int c = 0; c < n; ++c)
+    if (row_capacity(kGradCfgs[c]) >= cols) return c;
+  return -1;
+}
+
 uint32_t row_grid(const BwppHip *h, uint32_t rows) {
   const uint32_t cap = h->cus > 0 ? 8u * (uint32_t)h->cus : 2048u;
   return rows < cap ? rows : cap;
@@ -1632,7 +1652,12 @@ extern "C" BwppHipStatus bwpp_hip_dispatch_softmax_grad(BwppHip *h, const float 
   g.rows = p.rows;
   g.cols = p.cols;
   g.ld = ld;
-  return launch(h, h->softmax_grad, row_grid(h, p.rows), 1, 1, 256, g);
+  const int c = grad_cfg(p.cols, kGradNCfg);
+  if (c < 0) return launch(h, h->softmax_grad, row_grid(h, p.rows), 1, 1, 256, g);
+  const bool vec = p.cols % 4 == 0 && ld % 4 == 0 && aligned16(y) && aligned16(dy) && aligned16(dx);
+  const uint32_t rpb = row_rows_per_block(kGradCfgs[c]);
+  return launch(h, h->softmax_grad_reg[c][vec ? 1 : 0], (uint32_t)(((uint64_t)p.rows + rpb - 1) / rpb), 1, 1,
+                row_block(kGradCfgs[c]), g);
 }
 
 extern "C" BwppHipStatus bwpp_hip_dispatch_rmsnorm_grad(BwppHip *h, const float *x, const float *gamma,
@@ -1665,31 +1690,31 @@ extern "C" BwppHipStatus bwpp_hip_dispatch_rmsnorm_grad_acc(BwppHip *h, const fl
   g.cols = p.cols;
   g.ld = ld;
   g.eps = p.eps;
-  // With column partials, at most kMaxParts blocks (each loops over its
-  // rows), which bounds the partial arrays to kMaxParts rows.
-  constexpr uint32_t kMaxParts = 512;
-  // 16-byte rows of at most 2048 columns: one wave per row (no block
-  // barriers in the row loop), 4 rows per block per trip.
-  int wv = -1;
-  if (p.cols <= 2048 && p.cols % 4 == 0 && ld % 4 == 0 && aligned16(x) && aligned16(dy) && aligned16(dx) &&
-      (!gamma || aligned16(gamma)) && (!acc || aligned16(acc)))
-    wv = p.cols <= 256 ? 0 : p.cols <= 512 ? 1 : p.cols <= 1024 ? 2 : 3;
-  uint32_t grid;
-  if (wv >= 0) {
-    const uint32_t cap = parts ? kMaxParts : (h->cus > 0 ? 8u * (uint32_t)h->cus : 2048u);
-    grid = p.rows == 0 ? 1u : std::min<uint32_t>((p.rows + 3) / 4, cap);
-  } else {
-    grid = p.rows == 0 ? 1u : row_grid(h, p.rows);
-    if (parts && grid > kMaxParts) grid = kMaxParts;
-  }
+  // Rows of at most 8192 columns stay in registers.  With column partials,
+  // at most kMaxParts blocks (each loops over its rows), which bounds the
+  // partial arrays: 512 for one wave per row (4 rows per block), half that
+  // for longer rows, whose blocks hold a whole row and prefetch the next
+  // (4096 x 4096: 8 MB of partials beside 201 MB of rows, 31.4 us).
+  const int c = grad_cfg(p.cols, kGradNCfg - 1);
+  const uint32_t rpb = c >= 0 ? row_rows_per_block(kGradCfgs[c]) : 1u;
+  uint32_t grid = (uint32_t)std::max<uint64_t>(1, ((uint64_t)p.rows + rpb - 1) / rpb);
+  const uint32_t kMaxParts = c >= 0 && kGradCfgs[c].wpr > 1 ? 256u : 512u;
+  grid = std::min(grid, parts ? kMaxParts : h->cus > 0 ? 8u * (uint32_t)h->cus : 2048u);
   if (parts) {
     if ((s = ensure_ws(h, (size_t)2 * grid * p.cols * sizeof(float))) != BWPP_HIP_OK) return s;
     g.part_g = static_cast<float *>(h->ws);
     g.part_b = g.part_g + (size_t)grid * p.cols;
   }
   if (p.rows > 0 || parts) {
-    s = wv >= 0 ? launch(h, h->rmsnorm_grad_w[wv], grid, 1, 1, 256, g, parts ? 8u * p.cols * 4u : 0u)
-                : launch(h, h->rmsnorm_grad, grid, 1, 1, 256, g, parts ? 2u * p.cols * 4u : 0u);
+    if (c >= 0) {
+      // part_b's rows follow part_g's: 16-byte rows there too, as cols % 4 == 0.
+      const bool vec = p.cols % 4 == 0 && ld % 4 == 0 && aligned16(x) && aligned16(dy) && aligned16(dx) &&
+                       (!gamma || aligned16(gamma)) && (!acc || aligned16(acc));
+      s = launch(h, h->rmsnorm_grad_reg[c][vec ? 1 : 0], grid, 1, 1, row_block(kGradCfgs[c]), g,
+                 parts && rpb > 1 ? 2u * rpb * p.cols * 4u : 0u);
+    } else {
+      s = launch(h, h->rmsnorm_grad, grid, 1, 1, 256, g);
+    }
     if (s != BWPP_HIP_OK) return s;
   }
   if (!parts) return BWPP_HIP_OK;
@@ -1720,10 +1745,13 @@ extern "C" BwppHipStatus bwpp_hip_dispatch_reduce_sum(BwppHip *h, const float *x
     return launch(h, h->reduce_sum_rows, row_grid(h, p.rows), 1, 1, 256, g);
   }
   if (p.cols == 0) return BWPP_HIP_OK;
-  const uint32_t bands = p.rows == 0 ? 1u : (p.rows < 64u ? p.rows : 64u);
-  if ((s = ensure_ws(h, (size_t)bands * p.cols * sizeof(float))) != BWPP_HIP_OK) return s;
-  g.part_g = static_cast<float *>(h->ws);
-  if ((s = launch(h, h->reduce_sum_cols, (p.cols + 255) / 256, bands, 1, 256, g)) != BWPP_HIP_OK) return s;
+  const uint32_t bands = col_bands(h, p.rows, p.cols);
+  if (bands > 1) {
+    if ((s = ensure_ws(h, (size_t)bands * p.cols * sizeof(float))) != BWPP_HIP_OK) return s;
+    g.part_g = static_cast<float *>(h->ws);
+  }
+  s = launch(h, h->reduce_sum_cols, (uint32_t)(((uint64_t)p.cols + 63) / 64), bands, 1, 256, g);
+  if (s != BWPP_HIP_OK || bands == 1) return s;
   BwppGradArgs r = {};
   r.part_g = g.part_g;
   r.part_b = g.part_g;
