@@ -47,6 +47,36 @@ typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
 
 namespace {
 
+typedef unsigned short u16x2_t __attribute__((ext_vector_type(2)));
+
+// Eight fp32 probabilities (registers r0 .. r0 + 7 of an accumulator) as two
+// bf16 terms: the upper 16 bits, and the rounded rest.  The rest is kept
+// above zero wherever p is (by 2^-23 p), so that p * inf stays inf.
+__device__ __forceinline__ void split_bf16x8(const f32x16_t *s, int r0, bf16x8_t &hi, bf16x8_t &lo) {
+  uint32_t h[4], l[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float p0 = (*s)[r0 + 2 * i], p1 = (*s)[r0 + 2 * i + 1];
+    const uint32_t u0 = __float_as_uint(p0) & 0xffff0000u, u1 = __float_as_uint(p1) & 0xffff0000u;
+    h[i] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+    l[i] = pack_bf16x2(__builtin_fmaf(p0, 1.00000012f, -__uint_as_float(u0)),
+                       __builtin_fmaf(p1, 1.00000012f, -__uint_as_float(u1)));
+  }
+  hi = __builtin_bit_cast(bf16x8_t, make_uint4(h[0], h[1], h[2], h[3]));
+  lo = __builtin_bit_cast(bf16x8_t, make_uint4(l[0], l[1], l[2], l[3]));
+}
+
+// Running maximum of |v| as bit patterns, two bf16 lanes at a time (0x7f80
+// and above: infinity or NaN).
+__device__ __forceinline__ u16x2_t max_abs_bf16(u16x2_t m, v8s_t v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const u16x2_t w = {(unsigned short)(v[2 * i] & 0x7fff), (unsigned short)(v[2 * i + 1] & 0x7fff)};
+    m = __builtin_elementwise_max(m, w);
+  }
+  return m;
+}
+
 constexpr int kWaves = 4;               // generic path
 constexpr int kFW = 8;                  // flash path: waves per block
 constexpr int kQW = 32;                 // queries per wave
@@ -848,81 +878,374 @@ __device__ __forceinline__ void st_elem(T *p, float v) {
     *p = v;
 }
 
-template <class T, bool CAUSAL>
-__device__ __forceinline__ void attn_generic(const BwppAttnArgs &a) {
+// One query by one wave.  qs: [>= kdim] floats, ps: [64] floats of LDS of
+// the wave's own; DPL: ceil(vdim / 64) at most.
+template <class T, bool CAUSAL, int DPL>
+__device__ __forceinline__ void attn_generic_query(const BwppAttnArgs &a, uint32_t bh, uint32_t qi, float scale,
+                                                   float *qs, float *ps) {
   const uint32_t Kd = a.kdim, Dv = a.vdim;
-  __shared__ float qs[kWaves][kGenMaxDim];
-  __shared__ float ps[kWaves][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const uint32_t nbh = gridDim.x / a.q_tiles;
-  const uint32_t qt = a.q_tiles - 1 - blockIdx.x / nbh;
-  const uint32_t bh = blockIdx.x % nbh;
+  const int lane = threadIdx.x & 63;
   const uint32_t b = bh / a.heads, h = bh % a.heads;
   const T *Q = static_cast<const T *>(a.q) + b * a.q_bs + h * a.q_hs;
   const T *K = static_cast<const T *>(a.k) + b * a.k_bs + h * a.k_hs;
   const T *V = static_cast<const T *>(a.v) + b * a.v_bs + h * a.v_hs;
   T *O = static_cast<T *>(a.o) + b * a.o_bs + h * a.o_hs;
   const int64_t diag = (int64_t)a.N - (int64_t)a.M;
-  const float scale = a.scale_log2;  // the plain scale on this path
-  constexpr int DPL = kGenMaxDim / 64;
 
-  for (uint32_t qq = (uint32_t)wave; qq < kGenQ; qq += kWaves) {
-    const uint32_t qi = qt * kGenQ + qq;
-    if (qi >= a.M) break;  // wave-uniform
-    for (uint32_t k = (uint32_t)lane; k < Kd; k += 64) qs[wave][k] = ld_elem(Q + (size_t)qi * a.ldq + k);
+  for (uint32_t k = (uint32_t)lane; k < Kd; k += 64) qs[k] = ld_elem(Q + (size_t)qi * a.ldq + k);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  int64_t lim = CAUSAL ? (int64_t)qi + diag + 1 : (int64_t)a.N;
+  lim = lim < 0 ? 0 : (lim > (int64_t)a.N ? (int64_t)a.N : lim);
+  const uint32_t kend = (uint32_t)lim;
+  float m = -INFINITY, l = 0.0f;
+  float o[DPL];
+#pragma unroll
+  for (int j = 0; j < DPL; ++j) o[j] = 0.0f;
+  for (uint32_t n0 = 0; n0 < kend; n0 += 64) {
+    const uint32_t n = n0 + (uint32_t)lane;
+    float s = -INFINITY;
+    if (n < kend) {
+      const T *kr = K + (size_t)n * a.ldk;
+      float acc = 0.0f;
+      for (uint32_t k = 0; k < Kd; ++k) acc += qs[k] * ld_elem(kr + k);
+      s = acc * scale;
+    }
+    const float cm = wave_max(s);
+    const float mnew = fmaxf(m, cm);
+    const float muse = mnew == -INFINITY ? 0.0f : mnew;
+    const float alpha = expf(m - muse);
+    const float p = n < kend ? expf(s - muse) : 0.0f;
+    l = l * alpha + wave_sum(p);
+    m = mnew;
+    __builtin_amdgcn_wave_barrier();
+    ps[lane] = p;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    int64_t lim = CAUSAL ? (int64_t)qi + diag + 1 : (int64_t)a.N;
-    lim = lim < 0 ? 0 : (lim > (int64_t)a.N ? (int64_t)a.N : lim);
-    const uint32_t kend = (uint32_t)lim;
-    float m = -INFINITY, l = 0.0f;
-    float o[DPL];
+    const uint32_t cnt = min(64u, kend - n0);
 #pragma unroll
-    for (int j = 0; j < DPL; ++j) o[j] = 0.0f;
-    for (uint32_t n0 = 0; n0 < kend; n0 += 64) {
-      const uint32_t n = n0 + (uint32_t)lane;
-      float s = -INFINITY;
-      if (n < kend) {
-        const T *kr = K + (size_t)n * a.ldk;
-        float acc = 0.0f;
-        for (uint32_t k = 0; k < Kd; ++k) acc += qs[wave][k] * ld_elem(kr + k);
-        s = acc * scale;
+    for (int j = 0; j < DPL; ++j) o[j] *= alpha;
+    for (uint32_t t = 0; t < cnt; ++t) {
+      const float pn = ps[t];
+      const T *vr = V + (size_t)(n0 + t) * a.ldv;
+#pragma unroll
+      for (int j = 0; j < DPL; ++j) {
+        const uint32_t d = (uint32_t)lane + 64u * j;
+        if (d < Dv) o[j] += pn * ld_elem(vr + d);
       }
-      const float cm = wave_max(s);
-      const float mnew = fmaxf(m, cm);
-      const float muse = mnew == -INFINITY ? 0.0f : mnew;
-      const float alpha = expf(m - muse);
-      const float p = n < kend ? expf(s - muse) : 0.0f;
-      l = l * alpha + wave_sum(p);
-      m = mnew;
-      __builtin_amdgcn_wave_barrier();
-      ps[wave][lane] = p;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const uint32_t cnt = min(64u, kend - n0);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
-      for (int j = 0; j < DPL; ++j) o[j] *= alpha;
-      for (uint32_t t = 0; t < cnt; ++t) {
-        const float pn = ps[wave][t];
-        const T *vr = V + (size_t)(n0 + t) * a.ldv;
+  for (int j = 0; j < DPL; ++j) {
+    const uint32_t d = (uint32_t)lane + 64u * j;
+    if (d < Dv) st_elem(O + (size_t)qi * a.ldo + d, o[j] * inv);
+  }
+  if (a.lse && lane == 0) a.lse[(size_t)bh * a.M + qi] = l > 0.0f ? m + logf(l) : -INFINITY;
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <class T, bool CAUSAL>
+__device__ __forceinline__ void attn_generic(const BwppAttnArgs &a) {
+  __shared__ float qs[kWaves][kGenMaxDim];
+  __shared__ float ps[kWaves][64];
+  const int wave = threadIdx.x >> 6;
+  const uint32_t nbh = gridDim.x / a.q_tiles;
+  const uint32_t qt = a.q_tiles - 1 - blockIdx.x / nbh;
+  const uint32_t bh = blockIdx.x % nbh;
+  for (uint32_t qq = (uint32_t)wave; qq < kGenQ; qq += kWaves) {
+    const uint32_t qi = qt * kGenQ + qq;
+    if (qi >= a.M) break;  // wave-uniform
+    attn_generic_query<T, CAUSAL, kGenMaxDim / 64>(a, bh, qi, a.scale_log2 /* the plain scale on this path */, qs[wave],
+                                                  ps[wave]);
+  }
+}
+
+// --------------------------------------- bf16 forward, head dims 32, 64, 96
+// The flash scheme above (S^T = K Q^T on the matrix cores, softmax on the
+// accumulator registers, O^T += V^T P^T) for the smaller head dims, with the
+// probabilities at fp32 precision: P enters the second product as two bf16
+// terms, its upper 16 bits and the rounded rest (2^-16 of p together), so O
+// is as the fp32 arithmetic of the generic path gives it (error against 64
+// bits at B4 H16 S1000 d64: the rounding of the bf16 result, 1.6e-3, both
+// ways).  The second MFMA per V^T operand is cheap here: at d = 64 the
+// softmax (exp, max, sum, split: ~14 VALU slots per score) bounds the loop,
+// not the matrix pipe.
+//
+// A block of 4 waves owns 128 queries, each wave 32; keys stream in tiles of
+// 64 through a two-stage LDS ring filled by DMA.  Smaller tiles than d =
+// 128's: 16 KiB per stage and 126 registers leave room for four blocks per
+// CU, whose waves cover each other's barriers, and 128-query blocks fill the
+// chip at training's usual batch x heads (B4 H16 S1000: 512 blocks).
+// Measured there, causal: generic path 3784 us, this 32 us.
+//
+// Values that no query sees stay out: a masked key has p = 0, but 0 * v is
+// NaN for an infinite or NaN v.  Tiles with masked keys therefore look for
+// non-finite V elements, and a wave that finds one takes its queries through
+// the generic path's loop instead, which reads visible keys only.
+template <int D>
+struct AttnTile {
+  static constexpr int kSlots = D <= 64 ? 8 : 16;  // 16-byte chunks per LDS row (D / 8 of them in use)
+  static constexpr int kRowB = 16 * kSlots;
+  // Chunk c of K row r: the 16 rows of a quarter-wave's ds_read_b128 fall
+  // on 16 distinct 16-byte slots of the 64 banks.
+  static __device__ __forceinline__ uint32_t k_swz(uint32_t r) { return kSlots == 8 ? (r >> 1) & 7u : r & 15u; }
+  // Chunk c of V row r: the 4 rows x 4 chunks of a half-wave's transposing
+  // reads likewise; unchanged by steps of 8 rows.
+  static __device__ __forceinline__ uint32_t v_swz(uint32_t r) {
+    return kSlots == 8 ? 4u * ((r >> 1) & 1u) : 4u * (r & 3u);
+  }
+};
+
+template <int D, bool CAUSAL>
+__device__ __forceinline__ void attn_bf16_small(const BwppAttnArgs &a) {
+  using T = AttnTile<D>;
+  constexpr int NW = 4, kBKV = 64, KS = D / 16, DB = D / 32, KB = kBKV / 32;
+  constexpr int kTile = kBKV * T::kRowB, kStage = 2 * kTile;
+  constexpr int kBlkPW = kTile / 1024 / NW;  // 1 KiB DMA blocks per wave per K (or V) tile
+  constexpr int kOut = NW * kQW * T::kRowB;
+  static_assert(2 * kStage >= kOut && 2 * kStage >= NW * 4 * (D + 64), "epilogues reuse the ring");
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * kStage];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  // Contiguous runs of slices per XCD, as in attn_bf16_d128; the longest
+  // (last) query tile of a slice first.
+  const uint32_t G = gridDim.x, QT = a.q_tiles;
+  const uint32_t lb = G % 8u == 0 ? (blockIdx.x % 8u) * (G / 8u) + blockIdx.x / 8u : blockIdx.x;
+  const uint32_t bh = lb / QT, qt = QT - 1 - lb % QT;
+  const uint32_t b = bh / a.heads, h = bh % a.heads;
+  const uint16_t *Q = static_cast<const uint16_t *>(a.q) + b * a.q_bs + h * a.q_hs;
+  const uint16_t *K = static_cast<const uint16_t *>(a.k) + b * a.k_bs + h * a.k_hs;
+  const uint16_t *V = static_cast<const uint16_t *>(a.v) + b * a.v_bs + h * a.v_hs;
+  uint16_t *O = static_cast<uint16_t *>(a.o) + b * a.o_bs + h * a.o_hs;
+  const int64_t diag = (int64_t)a.N - (int64_t)a.M;  // key n visible to query m iff n <= m + diag
+
+  const uint32_t qb0 = qt * (NW * kQW), q0 = qb0 + (uint32_t)wave * kQW;
+  const uint32_t lq = (uint32_t)(lane & 31), lh = (uint32_t)(lane >> 5);
+  const uint32_t qi = q0 + lq;
+
+  uint32_t kend = a.N;
+  if (CAUSAL) {
+    const int64_t lim = (int64_t)min(qb0 + NW * kQW, a.M) + diag;
+    kend = lim <= 0 ? 0u : (uint32_t)min<int64_t>(lim, a.N);
+  }
+  const uint32_t nkt = (kend + kBKV - 1) / kBKV;
+
+  bf16x8_t qf[KS];  // query qi, d = 16 ks + 8 lh .. + 7
 #pragma unroll
-        for (int j = 0; j < DPL; ++j) {
-          const uint32_t d = (uint32_t)lane + 64u * j;
-          if (d < Dv) o[j] += pn * ld_elem(vr + d);
+  for (int ks = 0; ks < KS; ++ks) {
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (qi < a.M) v = *reinterpret_cast<const uint4 *>(Q + (size_t)qi * a.ldq + 16 * ks + 8 * lh);
+    qf[ks] = __builtin_bit_cast(bf16x8_t, v);
+  }
+  wait_vmcnt<0>();  // no load of the compiler's outstanding beside the DMA
+
+  // DMA: lane l of block i fills 16-byte slot l of it.  Rows past N re-read
+  // row N - 1 (masked below), slots past D / 8 a chunk of their row (unread).
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+  uint32_t dma_row[kBlkPW], dma_kcol[kBlkPW], dma_vcol[kBlkPW];
+#pragma unroll
+  for (int i = 0; i < kBlkPW; ++i) {
+    const uint32_t q = (uint32_t)(wave * kBlkPW + i) * 64u + (uint32_t)lane;
+    const uint32_t r = q / T::kSlots, pc = q % T::kSlots;
+    const uint32_t kc = pc ^ T::k_swz(r), vc = pc ^ T::v_swz(r);
+    dma_row[i] = r;
+    dma_kcol[i] = 8u * (kc < D / 8 ? kc : kc % (D / 8));
+    dma_vcol[i] = 8u * (vc < D / 8 ? vc : vc % (D / 8));
+  }
+  auto issue = [&](uint32_t t) {
+    const uint32_t st = lds0 + (t & 1u) * kStage + (uint32_t)(wave * kBlkPW) * 1024u;
+#pragma unroll
+    for (int i = 0; i < kBlkPW; ++i) {
+      uint32_t key = t * kBKV + dma_row[i];
+      key = key < a.N ? key : a.N - 1;
+      g2lds16_so(K, 2u * (key * a.ldk + dma_kcol[i]), st + (uint32_t)i * 1024u);
+      g2lds16_so(V, 2u * (key * a.ldv + dma_vcol[i]), st + kTile + (uint32_t)i * 1024u);
+    }
+  };
+
+  f32x16_t o[DB];
+#pragma unroll
+  for (int d = 0; d < DB; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+  float mrow = -INFINITY, lrow = 0.0f;
+  bool redo = false;  // wave-uniform
+  const float c = a.scale_log2;
+
+  const uint32_t grp = (uint32_t)((lane >> 4) & 3), L = (uint32_t)(lane & 15);
+  uint32_t koff[KS], voff[DB];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) koff[ks] = lq * T::kRowB + 16u * ((2u * ks + lh) ^ T::k_swz(lq));
+  {
+    const uint32_t kbase = 4u * (grp >> 1) + (L >> 2);
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+      const uint32_t col = 32u * d + 16u * (grp & 1u) + 4u * (L & 3u);
+      voff[d] = kTile + kbase * T::kRowB + 16u * ((col >> 3) ^ T::v_swz(kbase)) + (col & 7u) * 2u;
+    }
+  }
+
+  auto tile = [&](auto mask_tag, const unsigned char *Ks, uint32_t k0) {
+    constexpr bool MASK = decltype(mask_tag)::value;
+    int kbmax = KB - 1;  // last 32-key block that a query of this wave sees
+    if constexpr (MASK) {
+      int64_t kv = (int64_t)a.N - 1 - (int64_t)k0;
+      if (CAUSAL) kv = min(kv, (int64_t)(q0 + kQW - 1) + diag - (int64_t)k0);
+      kbmax = __builtin_amdgcn_readfirstlane(kv < 0 ? -1 : (int)min<int64_t>(kv / 32, KB - 1));
+    }
+    f32x16_t s[KB];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[kb][r] = 0.0f;
+      if (MASK && kb > kbmax) continue;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const bf16x8_t kf =
+            __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4 *>(Ks + koff[ks] + 32u * T::kRowB * kb));
+        s[kb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], s[kb], 0, 0, 0);
+      }
+    }
+    float mx = -INFINITY;
+    if constexpr (MASK) {
+      // Key of register r in block kb: k0 + 4 lh + 32 kb + 8 (r >> 2) + (r & 3).
+      int64_t lim64 = (int64_t)a.N - (int64_t)(k0 + 4u * lh);
+      if (CAUSAL) lim64 = min(lim64, (int64_t)qi + diag + 1 - (int64_t)(k0 + 4u * lh));
+      const int lim = (int)(lim64 < -1 ? -1 : (lim64 > kBKV ? kBKV : lim64));
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        if (kb > kbmax) continue;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float x = (32 * kb + 8 * (r >> 2) + (r & 3)) < lim ? s[kb][r] : -INFINITY;
+          s[kb][r] = x;
+          mx = fmaxf(mx, x);
         }
       }
-      __builtin_amdgcn_wave_barrier();
-    }
-    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    } else {
 #pragma unroll
-    for (int j = 0; j < DPL; ++j) {
-      const uint32_t d = (uint32_t)lane + 64u * j;
-      if (d < Dv) st_elem(O + (size_t)qi * a.ldo + d, o[j] * inv);
+      for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[kb][r]);
     }
-    if (a.lse && lane == 0) a.lse[(size_t)bh * a.M + qi] = l > 0.0f ? m + logf(l) : -INFINITY;
-    __builtin_amdgcn_wave_barrier();
+    {
+      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) * c;
+    }
+    float alpha = 1.0f;
+    if (mx > mrow + kLazy) {
+      alpha = __builtin_amdgcn_exp2f(mrow - mx);  // 0 when mrow is -inf
+      mrow = mx;
+    }
+    const float muse = mrow == -INFINITY ? 0.0f : mrow;
+    float sum = 0.0f;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      if (MASK && kb > kbmax) continue;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][r], c, -muse));
+        s[kb][r] = p;
+        sum += p;
+      }
+    }
+    {
+      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+      sum = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    lrow = lrow * alpha + sum;
+    if (__ballot(alpha != 1.0f)) {
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+    }
+    u16x2_t big = {0, 0};  // largest |V| bit patterns of a masked tile
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      if (MASK && kb > kbmax) continue;
+#pragma unroll
+      for (int kq = 0; kq < 2; ++kq) {
+        bf16x8_t ph, pl;
+        split_bf16x8(&s[kb], 8 * kq, ph, pl);
+        const uint32_t rstep = (32u * kb + 16u * kq) * T::kRowB;
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+          const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(Ks + voff[d] + rstep));
+          const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(Ks + voff[d] + rstep + 8u * T::kRowB));
+          const v8s_t vv = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+          if constexpr (MASK) big = max_abs_bf16(big, vv);
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vv), ph, o[d], 0, 0, 0);
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vv), pl, o[d], 0, 0, 0);
+        }
+      }
+    }
+    if constexpr (MASK) redo = redo || __ballot(big[0] >= 0x7f80u || big[1] >= 0x7f80u) != 0;
+  };
+
+  if (nkt > 0) issue(0);
+  // Tiles before t_mask need no mask for any query of the block.
+  uint32_t t_mask = a.N / kBKV;
+  if (CAUSAL) {
+    const int64_t first_hidden = (int64_t)qb0 + diag + 1;
+    t_mask = min(t_mask, first_hidden <= 0 ? 0u : (uint32_t)min<int64_t>(first_hidden / kBKV, (int64_t)nkt));
+  }
+  t_mask = min(t_mask, nkt);
+  auto step = [&](uint32_t t) {
+    wait_vmcnt<0>();
+    __syncthreads();
+    if (t + 1 < nkt) issue(t + 1);
+    return smem + __builtin_amdgcn_readfirstlane((t & 1u) * kStage);
+  };
+  for (uint32_t t = 0; t < t_mask; ++t) {
+    const unsigned char *Ks = step(t);
+    tile(std::integral_constant<bool, false>{}, Ks, t * kBKV);
+  }
+  for (uint32_t t = t_mask; t < nkt; ++t) {
+    const unsigned char *Ks = step(t);
+    const uint32_t k0 = t * kBKV;
+    if (CAUSAL && (int64_t)k0 > (int64_t)(q0 + kQW - 1) + diag) continue;  // no query of the wave sees it
+    tile(std::integral_constant<bool, true>{}, Ks, k0);
+  }
+  __syncthreads();
+
+  if (redo) {
+    float *qs = reinterpret_cast<float *>(smem) + wave * (D + 64);
+    for (uint32_t q = q0; q < min(q0 + kQW, a.M); ++q)
+      attn_generic_query<uint16_t, CAUSAL, (D + 63) / 64>(a, bh, q, a.scale, qs, qs + D);
+  }
+  __syncthreads();  // a wave's staging below may lie in another's qs
+  if (redo) return;
+  if (a.lse && lh == 0 && qi < a.M)
+    a.lse[(size_t)bh * a.M + qi] =
+        lrow > 0.0f ? __builtin_fmaf(mrow == -INFINITY ? 0.0f : mrow, 0.69314718055994531f, logf(lrow)) : -INFINITY;
+  uint16_t *os = reinterpret_cast<uint16_t *>(smem) + (size_t)wave * kQW * (T::kRowB / 2);
+  const float inv = lrow > 0.0f ? 1.0f / lrow : 0.0f;
+#pragma unroll
+  for (int d = 0; d < DB; ++d)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4) {
+      uint2 w;
+      w.x = pack_bf16x2(o[d][4 * q4 + 0] * inv, o[d][4 * q4 + 1] * inv);
+      w.y = pack_bf16x2(o[d][4 * q4 + 2] * inv, o[d][4 * q4 + 3] * inv);
+      *reinterpret_cast<uint2 *>(os + lq * (T::kRowB / 2) + 8u * ((4u * d + q4) ^ T::k_swz(lq)) + 4u * lh) = w;
+    }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  constexpr int kRowChunks = D / 8;
+#pragma unroll
+  for (int it = 0; it < kQW * kRowChunks / 64; ++it) {
+    const uint32_t q = (uint32_t)(lane + it * 64), ql = q / kRowChunks, cc = q % kRowChunks;
+    if (q0 + ql < a.M)
+      __builtin_nontemporal_store(
+          *reinterpret_cast<const u32x4_t *>(os + ql * (T::kRowB / 2) + 8u * (cc ^ T::k_swz(ql))),
+          reinterpret_cast<u32x4_t *>(O + (size_t)(q0 + ql) * a.ldo + 8u * cc));
   }
 }
 
@@ -1110,6 +1433,24 @@ BWPP_ATTN_BWD(bwpp_attn_bwd_f32, float, false)
 BWPP_ATTN_BWD(bwpp_attn_bwd_f32_causal, float, true)
 BWPP_ATTN_BWD(bwpp_attn_bwd_bf16, uint16_t, false)
 BWPP_ATTN_BWD(bwpp_attn_bwd_bf16_causal, uint16_t, true)
+
+// WPE: waves per SIMD the registers are cut to (the accumulators then stay
+// in VGPRs: with the compiler's own choice they moved to AGPRs and every
+// score was copied back for the softmax).
+#define BWPP_ATTN_SMALL(D, WPE)                                                                \
+  extern "C" __global__ __attribute__((amdgpu_flat_work_group_size(256, 256),                  \
+                                       amdgpu_waves_per_eu(WPE, WPE))) void                    \
+      bwpp_attn_bf16_d##D(const BwppAttnArgs a) {                                              \
+    attn_bf16_small<D, false>(a);                                                              \
+  }                                                                                            \
+  extern "C" __global__ __attribute__((amdgpu_flat_work_group_size(256, 256),                  \
+                                       amdgpu_waves_per_eu(WPE, WPE))) void                    \
+      bwpp_attn_bf16_d##D##_causal(const BwppAttnArgs a) {                                     \
+    attn_bf16_small<D, true>(a);                                                               \
+  }
+BWPP_ATTN_SMALL(32, 4)
+BWPP_ATTN_SMALL(64, 3)
+BWPP_ATTN_SMALL(96, 2)
 
 // Generic path entry points, one per storage type x mask.
 #define BWPP_ATTN_GENERIC(NAME, T, CAUSAL)                                                  \

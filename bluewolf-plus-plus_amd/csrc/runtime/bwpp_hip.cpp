@@ -92,6 +92,7 @@ struct BwppHip {
   hipFunction_t gemm_f32_reduce = nullptr;
   hipFunction_t attn_flash[2] = {};       // bf16, d = 128: [causal]
   hipFunction_t attn_flash_p[2] = {};     // bf16, d = 128, persistent (one block per CU): [causal]
+  hipFunction_t attn_bf16_small[3][2] = {};  // bf16, d = 32 / 64 / 96: [d / 32 - 1][causal]
   // BWPP_ATTN_FLASH_PERSIST: bit c set = persistent kernel when causal == c
   // (default unmasked only: causal C4 321.5 against 321.6 us, B2 H16 S4096
   // N 4096 +0.8 %, only B16 H16 S1024 -4.6 %).
@@ -333,6 +334,10 @@ BwppHipStatus resolve_all(BwppHip *h) {
       return s;
     if ((s = resolve(h, std::string("bwpp_attn_generic_bf16") + cs, &h->attn_generic[1][causal])) != BWPP_HIP_OK)
       return s;
+    for (int i = 0; i < 3; ++i)
+      if ((s = resolve(h, "bwpp_attn_bf16_d" + std::to_string(32 * (i + 1)) + cs, &h->attn_bf16_small[i][causal])) !=
+          BWPP_HIP_OK)
+        return s;
     for (int d128 = 0; d128 < 2; ++d128) {
       const std::string dn = std::string(d128 ? "128" : "64") + cs;
       if ((s = resolve(h, "bwpp_attn_f32_mfma_d" + dn, &h->attn_f32_fwd[d128][causal])) != BWPP_HIP_OK) return s;
@@ -1241,17 +1246,27 @@ BwppHipStatus attn_forward(BwppHip *h, const void *q, const void *k, const void 
   const float scale = p.scale != 0.0f ? p.scale : 1.0f;
   const int causal = p.causal ? 1 : 0;
   const bool bf16 = p.dtype == BWPP_HIP_BF16;
-  // The flash kernel takes the row maximum of the raw scores and scales it
-  // afterwards, which needs a positive scale (finite: NaN / inf go generic).
-  const bool flash = bf16 && p.K == 128 && p.D == 128 && p.N > 0 && scale > 0.0f && scale < INFINITY &&
-                     aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o) && g.ldq % 8 == 0 &&
-                     g.ldk % 8 == 0 && g.ldv % 8 == 0 && g.ldo % 8 == 0 && g.q_bs % 8 == 0 && g.q_hs % 8 == 0 &&
-                     g.k_bs % 8 == 0 && g.k_hs % 8 == 0 && g.v_bs % 8 == 0 && g.v_hs % 8 == 0 &&
-                     g.o_bs % 8 == 0 && g.o_hs % 8 == 0 &&
-                     // K / V byte offsets inside a slice are 32-bit in the kernel
-                     (uint64_t)(p.N - 1) * g.ldk + p.K < (1ull << 31) &&
-                     (uint64_t)(p.N - 1) * g.ldv + p.D < (1ull << 31);
-  if (flash) {
+  // The flash kernels take the row maximum of the raw scores and scale it
+  // afterwards, which needs a positive scale (finite: NaN / inf go generic);
+  // their operands come in 16-byte chunks and 32-wide blocks of the head dim.
+  const bool mfma = bf16 && p.K == p.D && p.K % 32 == 0 && p.K <= 128 && p.N > 0 && scale > 0.0f &&
+                    scale < INFINITY && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(o) &&
+                    g.ldq % 8 == 0 && g.ldk % 8 == 0 && g.ldv % 8 == 0 && g.ldo % 8 == 0 && g.q_bs % 8 == 0 &&
+                    g.q_hs % 8 == 0 && g.k_bs % 8 == 0 && g.k_hs % 8 == 0 && g.v_bs % 8 == 0 && g.v_hs % 8 == 0 &&
+                    g.o_bs % 8 == 0 && g.o_hs % 8 == 0 &&
+                    // K / V byte offsets inside a slice are 32-bit in the kernels
+                    (uint64_t)(p.N - 1) * g.ldk + p.K < (1ull << 31) &&
+                    (uint64_t)(p.N - 1) * g.ldv + p.D < (1ull << 31);
+  if (mfma && p.K < 128) {
+    g.scale = scale;
+    g.scale_log2 = scale * 1.4426950408889634f;
+    g.lse = lse;
+    g.q_tiles = (uint32_t)(((uint64_t)p.M + 127) / 128);
+    const uint64_t grid = slices * g.q_tiles;
+    if (grid > 0x7fffffffull) return fail(h, BWPP_HIP_ERR_UNSUPPORTED, "attention: grid too large");
+    return launch(h, h->attn_bf16_small[p.K / 32 - 1][causal], (uint32_t)grid, 1, 1, 256, g);
+  }
+  if (mfma) {
     g.scale_log2 = scale * 1.4426950408889634f;
     g.lse = lse;
     g.q_tiles = (p.M + 255) / 256;
