@@ -55,30 +55,6 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
-// (count, mean, M2) triples of Chan, Golub & LeVeque's pairwise variance
-// update: merging two partial row statistics costs one exchange step.
-__device__ __forceinline__ void chan_merge(float &n, float &mu, float &m2, float n2,
-                                           float mu2, float m22) {
-  const float nt = n + n2;
-  if (nt > 0.0f) {
-    const float d = mu2 - mu;
-    const float w = n2 / nt;
-    mu = mu + d * w;
-    m2 = m2 + m22 + d * d * n * w;
-  }
-  n = nt;
-}
-
-__device__ __forceinline__ void wave_chan(float &n, float &mu, float &m2) {
-  chan_merge(n, mu, m2, dpp_f32<kDppQuadXor1>(n), dpp_f32<kDppQuadXor1>(mu), dpp_f32<kDppQuadXor1>(m2));
-  chan_merge(n, mu, m2, dpp_f32<kDppQuadXor2>(n), dpp_f32<kDppQuadXor2>(mu), dpp_f32<kDppQuadXor2>(m2));
-  chan_merge(n, mu, m2, dpp_f32<kDppRowHalfMirror>(n), dpp_f32<kDppRowHalfMirror>(mu),
-             dpp_f32<kDppRowHalfMirror>(m2));
-  chan_merge(n, mu, m2, dpp_f32<kDppRowMirror>(n), dpp_f32<kDppRowMirror>(mu), dpp_f32<kDppRowMirror>(m2));
-  chan_merge(n, mu, m2, xor_f32(n, 16), xor_f32(mu, 16), xor_f32(m2, 16));
-  chan_merge(n, mu, m2, xor_f32(n, 32), xor_f32(mu, 32), xor_f32(m2, 32));
-}
-
 // (value, index) pairs: larger value wins, equal values keep the lower
 // index.  "No element" is (-INF, 0xFFFFFFFF), which loses to any real pair.
 __device__ __forceinline__ void argmax_merge(float &v, uint32_t &i, float v2,
@@ -113,8 +89,9 @@ __device__ __forceinline__ void wave_argmax(float &v, uint32_t &i) {
   i = w;
 }
 
-// 128-bit non-temporal global accesses for data streamed exactly once.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+// 128-bit global accesses at any 4-byte address (what the hardware asks of
+// a dwordx4), non-temporal for data streamed exactly once.
+typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ float4 load_nt4(const float *p) {
   const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p));
   return make_float4(t.x, t.y, t.z, t.w);
@@ -122,6 +99,10 @@ __device__ __forceinline__ float4 load_nt4(const float *p) {
 __device__ __forceinline__ void store_nt4(float *p, const float4 &o) {
   const f32x4 t = {o.x, o.y, o.z, o.w};
   __builtin_nontemporal_store(t, reinterpret_cast<f32x4 *>(p));
+}
+__device__ __forceinline__ float4 load4(const float *p) {
+  const f32x4 t = *reinterpret_cast<const f32x4 *>(p);
+  return make_float4(t.x, t.y, t.z, t.w);
 }
 
 // bf16 <-> fp32.  fp32 -> bf16 uses the gfx950 conversion instruction

@@ -18,8 +18,14 @@
 // grid); the next group's loads are issued before the current group's
 // reductions, and gamma/beta chunks are loaded once per block.
 //
+// Rows start at any 4-byte address (an odd row length): the 128-bit accesses
+// need no more, and a misaligned 1 KiB wave access touches nine 128-byte
+// lines instead of eight (2047 x 5003: softmax 30.6 -> 17.0 us, LayerNorm 40 ->
+// 17.1, RMSNorm 24.4 -> 15.7, reduce_max 11.0 -> 8.8 against the multi-pass
+// fallback, 4.8 TB/s; 1 to 3 columns take a thread per row).
+//
 // Fallback path ("gen"): one 256-thread block per row, scalar loads, several
-// passes; any cols, ld and alignment.
+// passes; rows longer than 32768.
 #include "common.h"
 #include "../kargs.h"
 
@@ -89,30 +95,9 @@ __device__ __forceinline__ void row_argmax(float &v, uint32_t &i, float *redf,
   }
 }
 
-// Row mean and M2 = sum (x - mean)^2 from per-thread partial statistics.
-template <int WPR>
-__device__ __forceinline__ void row_chan(float &n, float &mu, float &m2, float *red) {
-  wave_chan(n, mu, m2);
-  if constexpr (WPR > 1) {
-    const int w = threadIdx.x >> 6, w0 = (w / WPR) * WPR;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) {
-      red[3 * w] = n;
-      red[3 * w + 1] = mu;
-      red[3 * w + 2] = m2;
-    }
-    __syncthreads();
-    n = red[3 * w0];
-    mu = red[3 * w0 + 1];
-    m2 = red[3 * w0 + 2];
-#pragma unroll
-    for (int i = 1; i < WPR; ++i)
-      chan_merge(n, mu, m2, red[3 * (w0 + i)], red[3 * (w0 + i) + 1], red[3 * (w0 + i) + 2]);
-  }
-}
-
-// row_chan for equal per-thread counts n (full rows): the same statistics
-// with the equal-weight form of the merge; WPR waves' (mean, M2) combine as
+// Row mean and M2 = sum (x - mean)^2 from per-thread statistics over equal
+// counts n (full rows): the equal-weight form of Chan, Golub & LeVeque's
+// pairwise update, one exchange per step; WPR waves' (mean, M2) combine as
 // mean = average of the means, M2 = sum of M2 + n_wave * sum (mean_i - mean)^2.
 template <int WPR>
 __device__ __forceinline__ void row_chan_equal(float &n, float &mu, float &m2, float *red) {
@@ -185,10 +170,16 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
   const uint32_t sub = (uint32_t)(tid / GT);  // row slot in the block
   const uint32_t cols = a.cols;
   const uint32_t ngroups = (a.rows + G::kRows - 1) / G::kRows;
-  const float fill = kNorm ? 0.0f : -INFINITY;
 
   auto chunk_col = [&](int j) { return (uint32_t)(j * GT + g) * 4u; };
-  auto in_full = [&](uint32_t c) { return FULL || c + 4u <= cols; };
+  // A chunk that would pass the row's end starts at the row's last four
+  // columns instead (also one wholly past it), so that loads need neither
+  // tests nor branches (with them the compiler waited for one chunk before
+  // it issued the next).  Such a chunk repeats columns of other threads:
+  // harmless for maxima, left out of sums, and stored again with the same
+  // values.  Needs 4 columns.
+  auto chunk_at = [&](int j) { return FULL ? chunk_col(j) : min(chunk_col(j), cols - 4u); };
+  auto own = [&](int j, int e) { return FULL || chunk_at(j) + (uint32_t)e >= chunk_col(j); };
 
   // Loads the row of group `grp` (rows past the end re-read the last row;
   // their results are never stored), and for the max grad its dy with it.
@@ -203,35 +194,13 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
     const float *xr = a.x + (size_t)rr * a.ld;
     if constexpr (OP == OP_MAX_GRAD) dyv = a.dy[rr];
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-      const uint32_t c = chunk_col(j);
-      if (in_full(c)) {
-        v[j] = load_nt4(xr + c);
-      } else {
-        v[j] = make_float4(fill, fill, fill, fill);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (c + e < cols) set(v[j], e, xr[c + e]);
-      }
-    }
+    for (int j = 0; j < VPT; ++j) v[j] = load_nt4(xr + chunk_at(j));
   };
 
-  // gamma / beta chunk j (1 / 0 where absent or past the row end).
+  // gamma / beta chunk j (1 / 0 where absent).
   auto affine_chunk = [&](int j, float4 &gj, float4 &bj) {
-    const uint32_t c = chunk_col(j);
-    gj = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-    bj = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (in_full(c)) {
-      if (a.gamma) gj = *reinterpret_cast<const float4 *>(a.gamma + c);
-      if (a.beta) bj = *reinterpret_cast<const float4 *>(a.beta + c);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (c + e < cols) {
-          if (a.gamma) set(gj, e, a.gamma[c + e]);
-          if (a.beta) set(bj, e, a.beta[c + e]);
-        }
-    }
+    gj = a.gamma ? load4(a.gamma + chunk_at(j)) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+    bj = a.beta ? load4(a.beta + chunk_at(j)) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   };
   // Hoisted copies, reused for every row the block normalises.
   float4 gm[kHoist ? VPT : 1], bt[kHoist ? VPT : 1];
@@ -246,15 +215,7 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
     const bool valid = row < a.rows;
     float *yr = a.y ? a.y + (size_t)(valid ? row : 0) * a.ld : nullptr;
     auto store = [&](int j, const float4 &o) {
-      const uint32_t c = chunk_col(j);
-      if (!valid) return;
-      if (in_full(c)) {
-        store_nt4(yr + c, o);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (c + e < cols) yr[c + e] = get(o, e);
-      }
+      if (valid && (FULL || chunk_col(j) < cols)) store_nt4(yr + chunk_at(j), o);
     };
 
     if constexpr (OP == OP_SOFTMAX) {
@@ -270,13 +231,11 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
         v[j].y = __expf(v[j].y - m);
         v[j].z = __expf(v[j].z - m);
         v[j].w = __expf(v[j].w - m);
-        const uint32_t c = chunk_col(j);
-        if (in_full(c)) {
+        if constexpr (FULL) {
           s += (v[j].x + v[j].y) + (v[j].z + v[j].w);
         } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (c + e < cols) s += get(v[j], e);
+          for (int e = 0; e < 4; ++e) s += own(j, e) ? get(v[j], e) : 0.0f;
         }
       }
       s = row_sum<WPR>(s, redf);
@@ -285,53 +244,44 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
       for (int j = 0; j < VPT; ++j)
         store(j, make_float4(v[j].x * inv, v[j].y * inv, v[j].z * inv, v[j].w * inv));
     } else if constexpr (kNorm) {
+      // v past the row is not 0 (it repeats the row): sums take own columns.
+      auto mine = [&](int j, int e, float t) { return own(j, e) ? t : 0.0f; };
       float mean = 0.0f, ss = 0.0f;
       if constexpr (OP == OP_LAYERNORM) {
-        // Thread-local mean and M2 from registers (two passes, exact), then
-        // one merged reduction of (count, mean, M2) across the row.
-        float n = 0.0f, s = 0.0f;
+        float n = 4.0f * VPT, s = 0.0f;
 #pragma unroll
-        for (int j = 0; j < VPT; ++j) {
-          const uint32_t c = chunk_col(j);
-          if (in_full(c)) {
-            s += (v[j].x + v[j].y) + (v[j].z + v[j].w);
-            n += 4.0f;
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (c + e < cols) {
-                s += get(v[j], e);
-                n += 1.0f;
-              }
-          }
+        for (int j = 0; j < VPT; ++j)
+          s += (mine(j, 0, v[j].x) + mine(j, 1, v[j].y)) + (mine(j, 2, v[j].z) + mine(j, 3, v[j].w));
+        float mu, m2 = 0.0f;
+        if constexpr (FULL) {
+          // Thread-local mean and M2 from registers (two passes, exact),
+          // then one merged reduction of (count, mean, M2) across the row.
+          // Every thread holds 4 VPT values, so every merge step joins equal
+          // counts n and Chan's update needs no division:
+          // mu = (mu_a + mu_b) / 2, M2 = M2_a + M2_b + (mu_b - mu_a)^2 n / 2.
+          mu = s / n;
+        } else {
+          // Other rows: the row's mean first (a second reduction costs less
+          // than merging unequal counts, which divides at every step).
+          mu = row_sum<WPR>(s, redf) / (float)cols;
         }
-        float mu = n > 0.0f ? s / n : 0.0f;
-        float m2 = 0.0f;
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
-          const uint32_t c = chunk_col(j);
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            if (FULL || c + e < cols) {
-              const float d = get(v[j], e) - mu;
-              m2 += d * d;
-            }
+            const float d = mine(j, e, get(v[j], e) - mu);
+            m2 += d * d;
           }
         }
-        if constexpr (FULL) {
-          // Full rows: every thread holds 4 VPT values, so every merge step
-          // joins equal counts n and Chan's update needs no division:
-          // mu = (mu_a + mu_b) / 2, M2 = M2_a + M2_b + (mu_b - mu_a)^2 n / 2.
-          row_chan_equal<WPR>(n, mu, m2, redf);
-        } else {
-          row_chan<WPR>(n, mu, m2, redf);
-        }
+        if constexpr (FULL) row_chan_equal<WPR>(n, mu, m2, redf);
+        else m2 = row_sum<WPR>(m2, redf);
         mean = mu;
         ss = m2;
       } else {
 #pragma unroll
         for (int j = 0; j < VPT; ++j)
-          ss += (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w);
+          ss += (mine(j, 0, v[j].x * v[j].x) + mine(j, 1, v[j].y * v[j].y)) +
+                (mine(j, 2, v[j].z * v[j].z) + mine(j, 3, v[j].w * v[j].w));
         ss = row_sum<WPR>(ss, redf);
       }
       const float inv = 1.0f / sqrtf(ss / (float)cols + a.eps);
@@ -351,47 +301,30 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
         store(j, o);
       }
     } else if constexpr (OP == OP_MAX || OP == OP_MAX_GRAD) {
+      // Two passes over the registers: the lane's max (fmaxf skips NaN,
+      // -inf when the lane holds no number), then its first column
+      // holding that value and the element there (a backward scan, the
+      // last hit wins), which is the first strict-or-equal maximum of the
+      // fold in column order (the element, not fmaxf's result, carries the
+      // sign of a zero maximum).  Repeated chunks are scanned first and
+      // name columns of the row, so an earlier hit replaces theirs.
       float m = -INFINITY;
       uint32_t mi = kNoIndex;
-      if constexpr (FULL) {
-        // Two passes over the registers: the lane's max (fmaxf skips NaN,
-        // -inf when the lane holds no number), then its first column
-        // holding that value and the element there (a backward scan, the
-        // last hit wins), which is the first strict-or-equal maximum of the
-        // one-pass rule below (the element, not fmaxf's result, carries the
-        // sign of a zero maximum).
 #pragma unroll
-        for (int j = 0; j < VPT; ++j) m = fmaxf(fmaxf(m, fmaxf(v[j].x, v[j].y)), fmaxf(v[j].z, v[j].w));
-        float mv = m;
+      for (int j = 0; j < VPT; ++j) m = fmaxf(fmaxf(m, fmaxf(v[j].x, v[j].y)), fmaxf(v[j].z, v[j].w));
+      float mv = m;
 #pragma unroll
-        for (int j = VPT - 1; j >= 0; --j) {
-          const uint32_t c = chunk_col(j);
-          mi = v[j].w == m ? c + 3u : mi;
-          mv = v[j].w == m ? v[j].w : mv;
-          mi = v[j].z == m ? c + 2u : mi;
-          mv = v[j].z == m ? v[j].z : mv;
-          mi = v[j].y == m ? c + 1u : mi;
-          mv = v[j].y == m ? v[j].y : mv;
-          mi = v[j].x == m ? c : mi;
-          mv = v[j].x == m ? v[j].x : mv;
-        }
-        m = mv;
-      } else {
+      for (int j = VPT - 1; j >= 0; --j) {
+        const uint32_t c = chunk_at(j);
 #pragma unroll
-        for (int j = 0; j < VPT; ++j) {
-          const uint32_t c = chunk_col(j);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float t = get(v[j], e);
-            if (c + e < cols) {
-              if (t > m || (mi == kNoIndex && t == m)) {
-                m = t;
-                mi = c + e;
-              }
-            }
-          }
+        for (int e = 3; e >= 0; --e) {
+          const float t = get(v[j], e);
+          const bool hit = t == m;
+          mi = hit ? c + e : mi;
+          mv = hit ? t : mv;
         }
       }
+      m = mv;
       row_argmax<WPR>(m, mi, redf, redu);
       if constexpr (OP == OP_MAX) {
         if (g == 0 && valid) {
@@ -402,7 +335,7 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
         const float gv = valid ? dyv : 0.0f;
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
-          const uint32_t c = chunk_col(j);
+          const uint32_t c = chunk_at(j);
           float4 o;
           o.x = (c + 0 == mi) ? gv : 0.0f;
           o.y = (c + 1 == mi) ? gv : 0.0f;
@@ -456,6 +389,59 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
     process(vb, grp, db);
     if (!kPrefetch) load_row(next, va, da);
     grp = next;
+  }
+}
+
+// Rows of 1 to 3 columns: a thread per row.
+template <int OP>
+__device__ __forceinline__ void row_tiny(const BwppRowArgs &a) {
+  const uint64_t row = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+  if (row >= a.rows) return;
+  const uint32_t cols = a.cols;
+  float v[3], m = -INFINITY;
+  uint32_t mi = kNoIndex;
+#pragma unroll
+  for (uint32_t c = 0; c < 3; ++c) {
+    v[c] = c < cols ? a.x[row * a.ld + c] : 0.0f;
+    if (c < cols && (v[c] > m || (mi == kNoIndex && v[c] == m))) {
+      m = v[c];
+      mi = c;
+    }
+  }
+  auto put = [&](auto f) {
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c)
+      if (c < cols) a.y[row * a.ld + c] = f(c);
+  };
+  if constexpr (OP == OP_SOFTMAX) {
+    float s = 0.0f;
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c) {
+      v[c] = __expf(v[c] - m);
+      s += c < cols ? v[c] : 0.0f;
+    }
+    const float inv = s > 0.0f ? 1.0f / s : 0.0f;
+    put([&](uint32_t c) { return v[c] * inv; });
+  } else if constexpr (OP == OP_RMSNORM || OP == OP_LAYERNORM) {
+    const float mean = OP == OP_LAYERNORM ? (v[0] + v[1] + v[2]) / (float)cols : 0.0f;
+    float ss = 0.0f;
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c) {
+      const float d = c < cols ? v[c] - mean : 0.0f;
+      ss += d * d;
+    }
+    const float inv = 1.0f / sqrtf(ss / (float)cols + a.eps);
+    put([&](uint32_t c) {
+      return (v[c] - mean) * inv * (a.gamma ? a.gamma[c] : 1.0f) + (a.beta ? a.beta[c] : 0.0f);
+    });
+  } else if constexpr (OP == OP_MAX) {
+    if (a.maxv) a.maxv[row] = m;
+    if (a.argmax) a.argmax[row] = (mi == kNoIndex) ? -1 : (int32_t)mi;
+  } else if constexpr (OP == OP_MAX_GRAD) {
+    const float gv = a.dy[row];
+    put([&](uint32_t c) { return c == mi ? gv : 0.0f; });
+  } else {
+    put([&](uint32_t c) { return v[c] == m ? 1.0f : 0.0f; });
   }
 }
 
@@ -577,6 +563,9 @@ __device__ __forceinline__ void row_gen(const BwppRowArgs &a) {
   BWPP_ROW_REG(NAME, OP, 4, 8)                                                \
   BWPP_ROW_REG(NAME, OP, 8, 8)                                                \
   BWPP_ROW_REG(NAME, OP, 16, 8)                                               \
+  extern "C" __global__ __launch_bounds__(256) void bwpp_row_##NAME##_tiny(const BwppRowArgs a) { \
+    row_tiny<OP>(a);                                                          \
+  }                                                                           \
   extern "C" __global__ __launch_bounds__(256) void bwpp_row_##NAME##_gen(const BwppRowArgs a) { \
     row_gen<OP>(a);                                                           \
   }

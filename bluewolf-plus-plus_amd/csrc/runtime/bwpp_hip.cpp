@@ -76,6 +76,7 @@ struct BwppHip {
 
   hipFunction_t row_reg[ROW_NOPS][kRowNCfg][2] = {};
   hipFunction_t row_gen[ROW_NOPS] = {};
+  hipFunction_t row_tiny[ROW_NOPS] = {};  // 1 to 3 columns
   hipFunction_t row_maxgrad_idx = nullptr;
   hipFunction_t row_maxgrad_idx_v4 = nullptr;
   hipFunction_t row_maskgrad = nullptr;
@@ -248,6 +249,8 @@ BwppHipStatus resolve_all(BwppHip *h) {
       }
     }
     if ((s = resolve(h, std::string("bwpp_row_") + kRowOpNames[op] + "_gen", &h->row_gen[op])) != BWPP_HIP_OK)
+      return s;
+    if ((s = resolve(h, std::string("bwpp_row_") + kRowOpNames[op] + "_tiny", &h->row_tiny[op])) != BWPP_HIP_OK)
       return s;
   }
   struct {
@@ -428,7 +431,8 @@ BwppHipStatus launch(BwppHip *h, hipFunction_t f, uint32_t gx, uint32_t gy, uint
 inline uint32_t eff_ld(uint32_t ld, uint32_t cols) { return ld ? ld : cols; }
 
 // Picks the register-resident configuration for one operator on rows of
-// `cols` floats, or -1 for the multi-pass fallback.  Rows up to 1024 get one
+// `cols` floats (at least 4, at any alignment), or -1 for the multi-pass
+// fallback.  Rows up to 1024 get one
 // wave each (no cross-wave reduction, no barrier), and so do the norms' and
 // softmax's rows up to 1536; up to 2048 the norms and reduce_max take two
 // waves, and up to 3072 the norms take two waves of 8 chunks.  Longer rows
@@ -443,8 +447,7 @@ inline uint32_t eff_ld(uint32_t ld, uint32_t cols) { return ld ? ld : cols; }
 // at 4096 / 8192 / 16384 columns, LayerNorm 47.5 -> 46.3 / 51.3 -> 46.3 at
 // 8192 / 16384, the gradient 43.7 -> 43.0 / 45.0 -> 44.6 at 4096 / 8192
 // but 47.5 -> 49.2 at 16384, reduce_max 21.0 -> 24.1 at 4096).
-int pick_row_cfg(const BwppHip *h, RowOpId op, uint32_t cols, bool vec_ok) {
-  if (!vec_ok) return -1;
+int pick_row_cfg(const BwppHip *h, RowOpId op, uint32_t cols) {
   if (h->row_cfg_override >= 0 && h->row_cfg_override < kRowNCfg &&
       row_capacity(kRowCfgs[h->row_cfg_override]) >= cols)
     return h->row_cfg_override;
@@ -470,8 +473,9 @@ int pick_row_cfg(const BwppHip *h, RowOpId op, uint32_t cols, bool vec_ok) {
 // grid of 2 blocks per CU (measured best of 1 / 2 / 4 / one per row) so each
 // block reuses its gamma/beta registers over several rows; the others launch
 // one block per row group.
-BwppHipStatus row_dispatch(BwppHip *h, RowOpId op, const BwppRowArgs &a, bool vec_ok) {
-  const int c = pick_row_cfg(h, op, a.cols, vec_ok);
+BwppHipStatus row_dispatch(BwppHip *h, RowOpId op, const BwppRowArgs &a) {
+  if (a.cols < 4) return launch(h, h->row_tiny[op], (uint32_t)(((uint64_t)a.rows + 255) / 256), 1, 1, 256, a);
+  const int c = pick_row_cfg(h, op, a.cols);
   if (c < 0) return launch(h, h->row_gen[op], a.rows, 1, 1, 256, a);
   const RowCfg &cfg = kRowCfgs[c];
   const int full = (a.cols == row_capacity(cfg)) ? 1 : 0;
@@ -746,8 +750,7 @@ BwppHipStatus bwpp_hip_dispatch_softmax(BwppHip *h, const float *x, float *y, Bw
   a.rows = p.rows;
   a.cols = p.cols;
   a.ld = ld;
-  const bool vec = aligned16(x) && aligned16(y) && (ld % 4 == 0);
-  return row_dispatch(h, ROW_SOFTMAX, a, vec);
+  return row_dispatch(h, ROW_SOFTMAX, a);
 }
 
 static BwppHipStatus norm_dispatch(BwppHip *h, RowOpId op, const float *x, const float *gamma, const float *beta,
@@ -767,9 +770,7 @@ static BwppHipStatus norm_dispatch(BwppHip *h, RowOpId op, const float *x, const
   a.cols = p.cols;
   a.ld = ld;
   a.eps = p.eps;
-  const bool vec = aligned16(x) && aligned16(y) && (ld % 4 == 0) && (!gamma || aligned16(gamma)) &&
-                   (!beta || aligned16(beta));
-  return row_dispatch(h, op, a, vec);
+  return row_dispatch(h, op, a);
 }
 
 BwppHipStatus bwpp_hip_dispatch_rmsnorm(BwppHip *h, const float *x, const float *gamma, const float *beta,
@@ -805,7 +806,7 @@ BwppHipStatus bwpp_hip_dispatch_reduce_max(BwppHip *h, const float *x, float *ma
   }
   if (p.rows == 0) return BWPP_HIP_OK;
   if (p.cols == 0) return launch(h, h->row_gen[ROW_MAX], p.rows, 1, 1, 256, a);
-  return row_dispatch(h, ROW_MAX, a, aligned16(x) && (ld % 4 == 0));
+  return row_dispatch(h, ROW_MAX, a);
 }
 
 BwppHipStatus bwpp_hip_dispatch_reduce_max_mask(BwppHip *h, const float *x, float *mask, BwppReduceParams p) {
@@ -832,7 +833,7 @@ BwppHipStatus bwpp_hip_dispatch_reduce_max_mask(BwppHip *h, const float *x, floa
     return col_apply_launch(h, h->col_mask_apply, a,
                             aligned16(x) && aligned16(mask) && p.cols % 4 == 0 && ld % 4 == 0);
   }
-  return row_dispatch(h, ROW_MASK, a, aligned16(x) && aligned16(mask) && (ld % 4 == 0));
+  return row_dispatch(h, ROW_MASK, a);
 }
 
 BwppHipStatus bwpp_hip_dispatch_reduce_max_grad(BwppHip *h, const float *mask, const float *dy, float *dx,
@@ -886,7 +887,7 @@ BwppHipStatus bwpp_hip_dispatch_reduce_max_grad_argmax(BwppHip *h, const float *
     const bool vec = aligned16(dx) && (ld % 4 == 0);
     return launch(h, vec ? h->row_maxgrad_idx_v4 : h->row_maxgrad_idx, stream_grid(p.rows), 1, 1, 256, a);
   }
-  return row_dispatch(h, ROW_MAXGRAD, a, aligned16(x) && aligned16(dx) && (ld % 4 == 0));
+  return row_dispatch(h, ROW_MAXGRAD, a);
 }
 
 }  // extern "C"
