@@ -353,12 +353,17 @@ constexpr int kPipeBK = 32;
 __device__ __forceinline__ uint32_t kc_off(uint32_t row, uint32_t c) {
   return row * 64u + 16u * (c ^ ((row >> 2) & 3u));
 }
-// MN-contiguous tile W elements wide: 2 W-byte k-rows of W / 8 chunks (a
-// multiple of 16, so the XOR stays inside the row).
+// MN-contiguous tile W elements wide: 2 W-byte k-rows of W / 8 chunks, chunk
+// c of row k at c ^ mnc_swz(k): the 4 k-rows x 4 chunks of a half-wave's
+// transposing reads fall on 16 distinct 16-byte slots of the 64 banks.
+template <int W>
+__device__ __forceinline__ uint32_t mnc_swz(uint32_t k) {
+  static_assert(W % 128 == 0 || W == 64 || W == 32, "k-rows of 4, 8 or a multiple of 16 chunks");
+  return W == 32 ? 0u : W == 64 ? 4u * ((k >> 1) & 1u) : 4u * (k & 3u);
+}
 template <int W>
 __device__ __forceinline__ uint32_t mnc_off(uint32_t k, uint32_t c) {
-  static_assert(W % 128 == 0, "k-rows of a multiple of 16 chunks");
-  return k * (2u * W) + 16u * (c ^ (4u * (k & 3u)));
+  return k * (2u * W) + 16u * (c ^ mnc_swz<W>(k));
 }
 
 // 16 bytes per lane, global -> LDS (M0 holds the wave's LDS destination;
@@ -719,6 +724,326 @@ __device__ __forceinline__ void gemm_bf16_pipe(const BwppGemmArgs &a) {
       if (!kEdgeN || n0 + (uint32_t)c * 8u < a.N)
         *reinterpret_cast<uint4 *>(C + (size_t)(m0 + hv * kHR + row) * a.ldc + n0 + c * 8) =
             *reinterpret_cast<const uint4 *>(cs + row * kCld + c * 8);
+    }
+  }
+}
+
+// ------------------------------------------ bf16, pipelined, any M, N and K
+//
+// The same LDS-DMA ring with smaller tiles, for what the 256-wide tiles leave
+// idle CUs or padding: ragged M, N and K, few rows (decoding), and products
+// with fewer tiles than CUs, whose K is then cut into ksplit ranges (raw
+// partial tiles, added in order by bwpp_gemm_bf16_splitk_reduce).  Rows or
+// columns past M / N re-read the last ones and are not stored; the chunks
+// past K of the last stage are zeroed in LDS, in both operands, before it is
+// multiplied.
+//
+// BM x BN tiles on WM x WN waves; KPS K tiles of 32 per stage, STAGES stages.
+// Small blocks, several per CU: a block waits for its stage and reads its
+// operands while another multiplies, which is worth more here than the
+// 256-wide kernels' hand-ordered loop.  32 x 64 streams op(B) with 48 KiB in
+// flight per block (16 x 4096 x 11008: 18.2 us, 5.0 TB/s; 210 on the 256 x 256
+// edge tile); 64 x 128 and 128 x 128 are bound by LDS reads (a wave's 64 x 64
+// tile reads 8 KiB per 8 MFMAs: 1337 x 1024 x 3000 17.4 us, 94 before).
+//
+// REG: the operands go through registers instead (16-byte loads at any
+// 2-byte address, the same LDS layout), for rows that are not 16-byte
+// aligned or extents that are no multiple of 8: one stage ahead, so bound by
+// the load latency where few blocks share a CU (4095 x 8191 x 2048: 170 us,
+// 1085 on the edge tile's element-wise loads; 257 x 255 x 4097 split 8 ways
+// 13.2, 1385).
+template <bool MNC, int W>
+__device__ __forceinline__ uint32_t ring_off(uint32_t ld, uint32_t blk, int lane, uint32_t lim, uint32_t klim) {
+  // Byte offset of this lane's chunk of 1 KiB block `blk` (over the stage's
+  // 32-deep K tiles) from the tile's origin; lim rows / columns and klim k
+  // exist (multiples of 8 where chunks run along them).
+  constexpr uint32_t kBlocks = W / 16;
+  const uint32_t sub = blk / kBlocks, q = (blk % kBlocks) * 64u + (uint32_t)lane;
+  if constexpr (!MNC) {
+    const uint32_t row = q >> 2, c = (q & 3u) ^ ((row >> 2) & 3u);
+    return 2u * (min(row, lim - 1u) * ld + min(sub * 32u + 8u * c, klim - 8u));
+  } else {
+    constexpr uint32_t kChunks = W / 8;
+    const uint32_t k = q / kChunks, c = (q % kChunks) ^ mnc_swz<W>(k);
+    return 2u * (min(sub * 32u + k, klim - 1u) * ld + min(8u * c, lim - 8u));
+  }
+}
+
+typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4a2_t __attribute__((ext_vector_type(4), aligned(2)));
+// 16 bytes at any 2-byte address (unaligned accesses are on for HSA code).
+__device__ __forceinline__ u32x4_t load16_b16(const uint16_t *p) { return *reinterpret_cast<const u32x4a2_t *>(p); }
+// v's bf16 elements moved down by n (0 .. 7; 8 and more: all gone), zeros
+// behind them.  (No array: the compiler indexed it, in scratch.)
+__device__ __forceinline__ u32x4_t shift_down_b16(u32x4_t v, uint32_t n) {
+  const bool s4 = n & 4u, s2 = n & 2u, s1 = n & 1u;
+  const uint32_t a0 = s4 ? v[2] : v[0], a1 = s4 ? v[3] : v[1], a2 = s4 ? 0u : v[2], a3 = s4 ? 0u : v[3];
+  const uint32_t b0 = s2 ? a1 : a0, b1 = s2 ? a2 : a1, b2 = s2 ? a3 : a2, b3 = s2 ? 0u : a3;
+  const uint32_t c0 = s1 ? (b0 >> 16 | b1 << 16) : b0, c1 = s1 ? (b1 >> 16 | b2 << 16) : b1;
+  const uint32_t c2 = s1 ? (b2 >> 16 | b3 << 16) : b2, c3 = s1 ? b3 >> 16 : b3;
+  const uint32_t keep = n < 8u ? 0xffffffffu : 0u;
+  return u32x4_t{c0 & keep, c1 & keep, c2 & keep, c3 & keep};
+}
+// This lane's chunk of block `blk` of a stage (ring_off's chunk), for rows
+// at any address and extents of any size: a chunk that would pass its row's
+// end is read as the row's last 8 elements and moved down when it is stored
+// (ring_fix); rows past the last re-read that.  lim rows / columns, klim k.
+template <bool MNC, int W>
+struct RingChunk {
+  uint32_t row;  // row of the stored operand within the stage
+  int col;       // first element along it
+  __device__ __forceinline__ RingChunk(uint32_t blk, int lane) {
+    constexpr uint32_t kBlocks = W / 16, kChunks = W / 8;
+    const uint32_t sub = blk / kBlocks, q = (blk % kBlocks) * 64u + (uint32_t)lane;
+    if constexpr (!MNC) {
+      row = q >> 2;
+      col = (int)(sub * 32u + 8u * ((q & 3u) ^ ((row >> 2) & 3u)));
+    } else {
+      row = sub * 32u + q / kChunks;
+      col = (int)(8u * ((q % kChunks) ^ mnc_swz<W>(q / kChunks)));
+    }
+  }
+  __device__ __forceinline__ int at(uint32_t lim, uint32_t klim) const { return min(col, (int)(MNC ? lim : klim) - 8); }
+  __device__ __forceinline__ u32x4_t load(const uint16_t *g, uint32_t ld, uint32_t lim, uint32_t klim) const {
+    return load16_b16(g + ((int64_t)min(row, (MNC ? klim : lim) - 1u) * ld + at(lim, klim)));
+  }
+  __device__ __forceinline__ u32x4_t fix(u32x4_t v, uint32_t lim, uint32_t klim) const {
+    const u32x4_t r = shift_down_b16(v, (uint32_t)(col - at(lim, klim)));
+    const uint32_t keep = MNC && row >= klim ? 0u : 0xffffffffu;
+    return u32x4_t{r[0] & keep, r[1] & keep, r[2] & keep, r[3] & keep};
+  }
+};
+
+// Zeroes the chunks of a staged operand (KPS K tiles, kTileBytes apart)
+// whose k is krem or more.
+template <bool MNC, int W, int KPS, int NT>
+__device__ __forceinline__ void ring_zero(unsigned char *tile, uint32_t stride, uint32_t krem, int tid) {
+#pragma unroll
+  for (int sub = 0; sub < KPS; ++sub) {
+    for (uint32_t i = (uint32_t)tid; i < W * 4u; i += NT) {
+      const uint32_t row = i >> 2;
+      const uint32_t k = MNC ? i / (W / 8) : 8u * ((i & 3u) ^ ((row >> 2) & 3u));
+      if ((uint32_t)sub * 32u + k >= krem)
+        *reinterpret_cast<uint4 *>(tile + sub * stride + 16u * i) = make_uint4(0, 0, 0, 0);
+    }
+  }
+}
+
+template <bool TA, bool TB, int BM, int BN, int WM, int WN, int KPS, int STAGES, bool REG>
+__device__ __forceinline__ void gemm_bf16_ring(const BwppGemmArgs &a) {
+  constexpr int NW = WM * WN, NT = 64 * NW, BK = 32 * KPS;
+  constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32;
+  constexpr int kTileA = BM * 64, kTileB = BN * 64, kSub = kTileA + kTileB, kStage = KPS * kSub;
+  constexpr int LPA = KPS * (BM / 16) / NW, LPB = KPS * (BN / 16) / NW, kDma = LPA + LPB;
+  static_assert(LPA * NW == KPS * (BM / 16) && LPB * NW == KPS * (BN / 16), "DMA blocks split evenly");
+  constexpr int kCld = BN + 8, kRing = STAGES * kStage, kOut = BM * kCld * 2;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kRing > kOut ? kRing : kOut];
+  __shared__ float bias_s[BN];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const uint32_t tiles = a.tiles_m * a.tiles_n;
+  const uint32_t split = a.ksplit > 1 ? blockIdx.x / tiles : 0u;
+  uint32_t tm, tn;
+  tile_coords(a, tm, tn, blockIdx.x - split * tiles);
+  const uint32_t m0 = tm * BM, n0 = tn * BN;
+  const uint32_t kbeg = a.ksplit > 1 ? split * a.kchunk : 0u;
+  const uint32_t klen = a.ksplit > 1 ? min(a.K - kbeg, a.kchunk) : a.K;
+  const uint32_t ns = (klen + BK - 1) / BK, krem = klen - (ns - 1) * BK;  // k of the last stage
+  const uint16_t *A = static_cast<const uint16_t *>(a.a) +
+                      (TA ? (size_t)kbeg * a.lda + m0 : (size_t)m0 * a.lda + kbeg);
+  const uint16_t *B = static_cast<const uint16_t *>(a.b) +
+                      (TB ? (size_t)n0 * a.ldb + kbeg : (size_t)kbeg * a.ldb + n0);
+  const size_t stepA = TA ? (size_t)BK * a.lda : (size_t)BK, stepB = TB ? (size_t)BK : (size_t)BK * a.ldb;
+
+  const uint16_t *bias = static_cast<const uint16_t *>(a.bias);
+  const bool add = (a.epilogue & kEpiAdd) && bias && a.ksplit <= 1;
+  const bool act = (a.epilogue & kEpiSilu) != 0;
+  if (tid < BN) bias_s[tid] = add ? bf16_bits_to_f32(bias[min(n0 + (uint32_t)tid, a.N - 1u)]) : 0.0f;
+  wait_vmcnt<0>();  // no load of the compiler's outstanding beside the DMA
+
+  f32x16_t acc[FN][FM];
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  auto multiply = [&](const unsigned char *st) {
+#pragma unroll
+    for (int ks = 0; ks < 2 * KPS; ++ks) {
+      const unsigned char *sub = st + (ks / 2) * kSub;
+      bf16x8_t fa[FM], fb[FN];
+#pragma unroll
+      for (int j = 0; j < FM; ++j) fa[j] = read_operand<TA, BM>(sub, (uint32_t)(wm * TM + j * 32), ks % 2, lane);
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+        fb[i] = read_operand<!TB, BN>(sub + kTileA, (uint32_t)(wn * TN + i * 32), ks % 2, lane);
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int j = 0; j < FM; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[i], fa[j], acc[i][j], 0, 0, 0);
+    }
+  };
+
+  if constexpr (!REG) {
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+    uint32_t offA[LPA], offB[LPB];
+    uint32_t dstA[LPA], dstB[LPB];  // wave-uniform
+#pragma unroll
+    for (int i = 0; i < LPA; ++i) {
+      const uint32_t blk = (uint32_t)(wave * LPA + i);
+      offA[i] = ring_off<TA, BM>(a.lda, blk, lane, a.M - m0, 0xffffffffu);
+      dstA[i] = lds0 + blk / (BM / 16) * kSub + blk % (BM / 16) * 1024u;
+    }
+#pragma unroll
+    for (int i = 0; i < LPB; ++i) {
+      const uint32_t blk = (uint32_t)(wave * LPB + i);
+      offB[i] = ring_off<!TB, BN>(a.ldb, blk, lane, a.N - n0, 0xffffffffu);
+      dstB[i] = lds0 + blk / (BN / 16) * kSub + kTileA + blk % (BN / 16) * 1024u;
+    }
+    auto issue = [&](uint32_t t) {
+      const uint32_t st = (t % STAGES) * kStage;
+      const uint16_t *At = A + t * stepA, *Bt = B + t * stepB;
+      if (t + 1 < ns || krem == BK) {
+#pragma unroll
+        for (int i = 0; i < LPA; ++i) g2lds16_so(At, offA[i], dstA[i] + st);
+#pragma unroll
+        for (int i = 0; i < LPB; ++i) g2lds16_so(Bt, offB[i], dstB[i] + st);
+      } else {  // the last stage, short of k
+#pragma unroll
+        for (int i = 0; i < LPA; ++i)
+          g2lds16_so(At, ring_off<TA, BM>(a.lda, (uint32_t)(wave * LPA + i), lane, a.M - m0, krem), dstA[i] + st);
+#pragma unroll
+        for (int i = 0; i < LPB; ++i)
+          g2lds16_so(Bt, ring_off<!TB, BN>(a.ldb, (uint32_t)(wave * LPB + i), lane, a.N - n0, krem), dstB[i] + st);
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < STAGES - 1; ++t)
+      if ((uint32_t)t < ns) issue((uint32_t)t);
+    for (uint32_t t = 0; t < ns; ++t) {
+      // Stages t + 1 .. t + STAGES - 2 may still be in flight.
+      const uint32_t younger = min(ns - 1 - t, (uint32_t)(STAGES - 2));
+      if (STAGES >= 4 && younger >= 2) wait_vmcnt<2 * kDma>();
+      else if (STAGES >= 3 && younger >= 1) wait_vmcnt<kDma>();
+      else wait_vmcnt<0>();
+      __syncthreads();  // stage t is in LDS, and nobody reads stage t - 1 any more
+      if (t + STAGES - 1 < ns) issue(t + STAGES - 1);
+      unsigned char *st = smem + __builtin_amdgcn_readfirstlane((t % STAGES) * kStage);
+      if (t + 1 == ns && krem < BK) {
+        ring_zero<TA, BM, KPS, NT>(st, kSub, krem, tid);
+        ring_zero<!TB, BN, KPS, NT>(st + kTileA, kSub, krem, tid);
+        __syncthreads();
+      }
+      multiply(st);
+    }
+  } else {
+    // Through registers: stage t + 1 is loaded while stage t is multiplied,
+    // then written to the other LDS buffer.
+    static_assert(STAGES == 2, "two LDS buffers");
+    u32x4_t ra[LPA], rb[LPB];
+    const bool edge = (TA && a.M - m0 < BM) || (!TB && a.N - n0 < BN);  // block-uniform: chunks pass M or N
+    auto klim = [&](uint32_t t) { return t + 1 == ns ? krem : (uint32_t)BK; };
+    // The loads take no branch (their values would be merged, and waited
+    // for, where the paths meet).
+    auto load = [&](uint32_t t) {
+#pragma unroll
+      for (int i = 0; i < LPA; ++i)
+        ra[i] = RingChunk<TA, BM>((uint32_t)(wave * LPA + i), lane).load(A + t * stepA, a.lda, a.M - m0, klim(t));
+#pragma unroll
+      for (int i = 0; i < LPB; ++i)
+        rb[i] = RingChunk<!TB, BN>((uint32_t)(wave * LPB + i), lane).load(B + t * stepB, a.ldb, a.N - n0, klim(t));
+    };
+    auto store = [&](uint32_t t) {
+      if (edge || klim(t) < BK) {
+#pragma unroll
+        for (int i = 0; i < LPA; ++i)
+          ra[i] = RingChunk<TA, BM>((uint32_t)(wave * LPA + i), lane).fix(ra[i], a.M - m0, klim(t));
+#pragma unroll
+        for (int i = 0; i < LPB; ++i)
+          rb[i] = RingChunk<!TB, BN>((uint32_t)(wave * LPB + i), lane).fix(rb[i], a.N - n0, klim(t));
+      }
+      unsigned char *st = smem + (t & 1u) * kStage + 16 * lane;
+#pragma unroll
+      for (int i = 0; i < LPA; ++i) {
+        const int blk = wave * LPA + i;
+        *reinterpret_cast<u32x4_t *>(st + blk / (BM / 16) * kSub + blk % (BM / 16) * 1024) = ra[i];
+      }
+#pragma unroll
+      for (int i = 0; i < LPB; ++i) {
+        const int blk = wave * LPB + i;
+        *reinterpret_cast<u32x4_t *>(st + blk / (BN / 16) * kSub + kTileA + blk % (BN / 16) * 1024) = rb[i];
+      }
+    };
+    load(0);
+    store(0);
+    __syncthreads();
+    for (uint32_t t = 0; t < ns; ++t) {
+      if (t + 1 < ns) load(t + 1);
+      multiply(smem + (t & 1u) * kStage);
+      if (t + 1 < ns) store(t + 1);
+      __syncthreads();
+    }
+  }
+
+  const int lrow = lane & 31, lhalf = lane >> 5;
+  if (a.ksplit > 1) {
+    // Raw sums, rows of N rounded up to 4 floats.
+    const uint32_t np = (a.N + 3u) & ~3u;
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      const uint32_t m = m0 + (uint32_t)(wm * TM + j * 32 + lrow);
+      float *row = a.part + ((size_t)split * a.M + m) * np;
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t n = n0 + (uint32_t)(wn * TN + i * 32 + q * 8 + lhalf * 4);
+          if (m < a.M && n < np)
+            *reinterpret_cast<float4 *>(row + n) = make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                                                               acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
+        }
+    }
+    return;
+  }
+  __syncthreads();
+  uint16_t *cs = reinterpret_cast<uint16_t *>(smem);  // [BM][BN + 8]
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int nl = wn * TN + i * 32 + q * 8 + lhalf * 4;
+      const float4 bv = *reinterpret_cast<const float4 *>(bias_s + nl);
+#pragma unroll
+      for (int j = 0; j < FM; ++j) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float t = acc[i][j][4 * q + e] + (e == 0 ? bv.x : e == 1 ? bv.y : e == 2 ? bv.z : bv.w);
+          v[e] = act ? silu(t) : t;
+        }
+        uint2 o;
+        o.x = pack_bf16x2(v[0], v[1]);
+        o.y = pack_bf16x2(v[2], v[3]);
+        *reinterpret_cast<uint2 *>(cs + (wm * TM + j * 32 + lrow) * kCld + nl) = o;
+      }
+    }
+  __syncthreads();
+  uint16_t *C = static_cast<uint16_t *>(a.c);
+#pragma unroll 2
+  for (int it = 0; it < BM * (BN / 8) / NT; ++it) {
+    const int q = tid + it * NT, row = q / (BN / 8), c = q % (BN / 8);
+    const uint32_t m = m0 + (uint32_t)row, n = n0 + 8u * (uint32_t)c;
+    if (m >= a.M || n >= a.N) continue;
+    const uint16_t *h = cs + row * kCld + c * 8;
+    if (n + 8 <= a.N) {
+      *reinterpret_cast<u32x4a2_t *>(C + (size_t)m * a.ldc + n) = *reinterpret_cast<const u32x4_t *>(h);
+    } else {
+      for (uint32_t e = 0; e < 8 && n + e < a.N; ++e) C[(size_t)m * a.ldc + n + e] = h[e];
     }
   }
 }
@@ -1291,6 +1616,60 @@ extern "C" __global__ __launch_bounds__(256) void bwpp_gemm_f32_splitk_reduce(co
 
 // Entry points: bwpp_gemm_<bf16|f32>_t<TA><TB>_<f|e|s>  (f: no edges,
 // aligned; s: f with split-K partials)
+// C = epilogue(sum of the ksplit partial planes, in order), bf16: a thread
+// per 4 columns; the planes' loads are independent of one another.
+extern "C" __global__ __launch_bounds__(256) void bwpp_gemm_bf16_splitk_reduce(const BwppGemmArgs a) {
+  const uint32_t n4 = (a.N + 3u) / 4u;
+  const uint64_t total = (uint64_t)a.M * n4, plane = (uint64_t)a.M * n4 * 4u;
+  const uint16_t *bias = static_cast<const uint16_t *>(a.bias);
+  const bool add = (a.epilogue & kEpiAdd) && bias, act = (a.epilogue & kEpiSilu) != 0;
+  uint16_t *C = static_cast<uint16_t *>(a.c);
+  for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < total; i += (uint64_t)gridDim.x * 256u) {
+    const uint32_t m = (uint32_t)(i / n4), n = 4u * (uint32_t)(i % n4);
+    const float *p = a.part + 4u * i;
+    float4 t = *reinterpret_cast<const float4 *>(p);
+#pragma unroll 4
+    for (uint32_t k = 1; k < a.ksplit; ++k) {
+      const float4 u = *reinterpret_cast<const float4 *>(p + k * plane);
+      t.x += u.x, t.y += u.y, t.z += u.z, t.w += u.w;
+    }
+    float v[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e) {
+      if (add) v[e] += bf16_bits_to_f32(bias[min(n + e, a.N - 1u)]);
+      if (act) v[e] = silu(v[e]);
+    }
+    uint16_t *o = C + (size_t)m * a.ldc + n;
+    if (n + 4 <= a.N) {
+      typedef uint32_t u32x2a2_t __attribute__((ext_vector_type(2), aligned(2)));
+      *reinterpret_cast<u32x2a2_t *>(o) = u32x2a2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+    } else {
+      for (uint32_t e = 0; e < 4 && n + e < a.N; ++e) o[e] = f32_to_bf16_bits(v[e]);
+    }
+  }
+}
+
+// bwpp_gemm_bf16r<BM>x<BN>_t<TA><TB> (LDS-DMA) and .._u (through registers).
+#define BWPP_GEMM_BF16_RING(TA, TB, BM, BN, WM, WN, KPS, STAGES, WPE, KPSU, WPEU)                 \
+  extern "C" __global__ __launch_bounds__(64 * WM * WN, WPE) void                                 \
+      bwpp_gemm_bf16r##BM##x##BN##_t##TA##TB(const BwppGemmArgs a) {                              \
+    gemm_bf16_ring<TA != 0, TB != 0, BM, BN, WM, WN, KPS, STAGES, false>(a);                       \
+  }                                                                                               \
+  extern "C" __global__ __launch_bounds__(64 * WM * WN, WPEU) void                                \
+      bwpp_gemm_bf16r##BM##x##BN##_t##TA##TB##_u(const BwppGemmArgs a) {                          \
+    gemm_bf16_ring<TA != 0, TB != 0, BM, BN, WM, WN, KPSU, 2, true>(a);                            \
+  }
+#define BWPP_GEMM_BF16_RINGS(TA, TB)                        \
+  BWPP_GEMM_BF16_RING(TA, TB, 32, 64, 1, 2, 4, 4, 1, 4, 1)  \
+  BWPP_GEMM_BF16_RING(TA, TB, 64, 64, 2, 2, 2, 4, 2, 4, 2)  \
+  BWPP_GEMM_BF16_RING(TA, TB, 64, 128, 1, 4, 1, 4, 3, 2, 2) \
+  BWPP_GEMM_BF16_RING(TA, TB, 128, 128, 2, 2, 1, 3, 2, 2, 2) \
+  BWPP_GEMM_BF16_RING(TA, TB, 128, 256, 2, 4, 1, 3, 2, 1, 2)
+BWPP_GEMM_BF16_RINGS(0, 0)
+BWPP_GEMM_BF16_RINGS(0, 1)
+BWPP_GEMM_BF16_RINGS(1, 0)
+BWPP_GEMM_BF16_RINGS(1, 1)
+
 #define BWPP_GEMM_BF16(TA, TB, EDGE, SUF)                                                  \
   extern "C" __global__ __attribute__((amdgpu_flat_work_group_size(256, 256),            \
                                        amdgpu_waves_per_eu(1, 1))) void                  \

@@ -53,6 +53,12 @@ inline uint32_t row_rows_per_block(const RowCfg &c) { return row_block(c) / (64u
 // one exists for softmax_grad only.
 constexpr int kGradNCfg = 7;
 const RowCfg kGradCfgs[kGradNCfg] = {{1, 1}, {2, 1}, {4, 1}, {2, 4}, {2, 8}, {4, 8}, {8, 8}};
+// Tiles of the bf16 ring kernels for any M, N and K (gemm.hip).
+struct RingCfg {
+  uint32_t bm, bn, threads;
+};
+constexpr int kRingNCfg = 5;
+const RingCfg kRingCfgs[kRingNCfg] = {{32, 64, 128}, {64, 64, 256}, {64, 128, 256}, {128, 128, 256}, {128, 256, 512}};
 int find_cfg(int vpt, int wpr) {
   for (int i = 0; i < kRowNCfg; ++i)
     if (kRowCfgs[i].vpt == vpt && kRowCfgs[i].wpr == wpr) return i;
@@ -87,6 +93,13 @@ struct BwppHip {
   hipFunction_t col_mask = nullptr;                                  // no workspace
   // bwpp_gemm_<bf16|f32>_t<TA><TB>_<e|f>: [dtype][ta][tb][full]
   hipFunction_t gemm[2][2][2][2] = {};
+  hipFunction_t gemm_bf16_ring[kRingNCfg][2][2][2] = {};  // any M, N, K: [kRingCfgs][ta][tb][unaligned]
+  hipFunction_t gemm_bf16_reduce = nullptr;
+  // BWPP_GEMM_RING: 0 = those kernels off; c,S = tile kRingCfgs[c - 1] with S
+  // K ranges (through registers with a trailing u) wherever they can run.
+  int gemm_ring = -1;
+  uint32_t gemm_ring_split = 1;
+  bool gemm_ring_u = false;
   hipFunction_t gemm_bf16_w8[2][2] = {};  // 8-wave full-tile bf16: [ta][tb]
   hipFunction_t gemm_f32_split[2][2] = {};  // fp32 full tiles, split-K partials: [ta][tb]
   hipFunction_t gemm_f32p[2][2][2][2] = {};  // fp32 full tiles, DMA ring: [4-stage][ta][tb][split]
@@ -266,6 +279,7 @@ BwppHipStatus resolve_all(BwppHip *h) {
       {"bwpp_col_maxgrad_apply_v4", &h->col_maxgrad_apply[1]},
       {"bwpp_col_maxgrad", &h->col_maxgrad},         {"bwpp_col_mask", &h->col_mask},
       {"bwpp_silu_grad", &h->silu_grad},             {"bwpp_softmax_grad", &h->softmax_grad},
+      {"bwpp_gemm_bf16_splitk_reduce", &h->gemm_bf16_reduce},
       {"bwpp_rmsnorm_grad", &h->rmsnorm_grad},       {"bwpp_col_partials_sum", &h->col_partials_sum},
       {"bwpp_reduce_sum_rows", &h->reduce_sum_rows}, {"bwpp_reduce_sum_cols", &h->reduce_sum_cols},
       {"bwpp_mean_square_part", &h->mean_square_part}, {"bwpp_mean_square_final", &h->mean_square_final},
@@ -312,6 +326,12 @@ BwppHipStatus resolve_all(BwppHip *h) {
         }
   for (int ta = 0; ta < 2; ++ta)
     for (int tb = 0; tb < 2; ++tb) {
+      for (int c = 0; c < kRingNCfg; ++c) {
+        const std::string nr = "bwpp_gemm_bf16r" + std::to_string(kRingCfgs[c].bm) + "x" +
+                               std::to_string(kRingCfgs[c].bn) + "_t" + std::to_string(ta) + std::to_string(tb);
+        if ((s = resolve(h, nr, &h->gemm_bf16_ring[c][ta][tb][0])) != BWPP_HIP_OK) return s;
+        if ((s = resolve(h, nr + "_u", &h->gemm_bf16_ring[c][ta][tb][1])) != BWPP_HIP_OK) return s;
+      }
       const std::string n = "bwpp_gemm_bf16w8_t" + std::to_string(ta) + std::to_string(tb) + "_f";
       if ((s = resolve(h, n, &h->gemm_bf16_w8[ta][tb])) != BWPP_HIP_OK) return s;
       if (ta == 0) {
@@ -574,6 +594,15 @@ BwppHipStatus bwpp_hip_create(BwppHip **out, int device, const char *code_object
   if (const char *bn = getenv("BWPP_GEMM_BN")) {
     const uint32_t v = (uint32_t)strtoul(bn, nullptr, 10);
     h->gemm_bn = v == 256 || v == 384 ? v : 0u;
+  }
+  if (const char *rg = getenv("BWPP_GEMM_RING")) {
+    int c = 0;
+    unsigned sp = 1;
+    if (sscanf(rg, "%d,%u", &c, &sp) >= 1 && c >= 0 && c <= kRingNCfg) {
+      h->gemm_ring = c;
+      h->gemm_ring_split = sp ? sp : 1;
+      h->gemm_ring_u = strchr(rg, 'u') != nullptr;
+    }
   }
   if (const char *sk = getenv("BWPP_GEMM_SPLITK")) h->gemm_splitk = atoi(sk) != 0 ? 1u : 0u;
   if (const char *zz = getenv("BWPP_ATTN_ZIGZAG")) h->attn_zigzag = atoi(zz) != 0 ? 1u : 0u;
@@ -939,6 +968,79 @@ BwppHipStatus ensure_ws(BwppHip *h, size_t bytes);
 
 namespace {
 
+// bf16 ring kernels (gemm.hip, gemm_bf16_ring) for a product whose operands
+// are set in g: picks the tile and the number of K ranges S with the least
+// modelled time and launches them unless full_us, the modelled time of a
+// full-tile kernel that could run, is less (done stays false).  Per K element,
+// n blocks on a CU take lat + (n - 1) inc us; every launch costs 4 us with
+// its prologue and epilogue, a split 3.5 us and its partial planes' traffic at
+// 7 TB/s (they stay in the Infinity Cache), and no product runs faster than
+// its operands arrive (5.6 TB/s).  The full tiles: 0.0272 us per K and round
+// of 256 x 256 tiles (4096^3: 115 us), 0.041 of 256 x 384.  Fitted on MI355X
+// to 26 products from 9 x 9 x 200 to 4095 x 8191 x 2048, all transposes,
+// S = 1 .. 8; the choice is within 15 % of the best of all tiles and splits
+// on each (16 x 11008 x 4096: 210 us on the 256 x 256 edge tile, 18.2 so;
+// 1337 x 3000 x 1024 94 -> 17.5; 512 x 1024 x 1024 25.5 -> 6.5; 4000^3, B
+// transposed, 189 -> 134; 4095 x 8191 x 2048, odd rows, 1085 -> 170).
+BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool ta, bool tb, double full_us, bool &done) {
+  struct Cost {
+    double lat, inc;
+  };
+  // [through registers][kRingCfgs]
+  static const Cost kCost[2][kRingNCfg] = {
+      {{0.0039, 0.0045}, {0.0046, 0.0037}, {0.0085, 0.0055}, {0.0114, 0.0085}, {0.0158, 0.0158}},
+      {{0.0085, 0.0031}, {0.0088, 0.0042}, {0.0146, 0.0060}, {0.0185, 0.0105}, {0.0275, 0.0180}}};
+  constexpr uint32_t kQuantum = 128;  // K ranges in multiples of the deepest stage
+  const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
+  if (std::max({g.M, g.N, g.K}) > 0x7fffffffu || (ta && g.M < 8) || (!tb && g.N < 8)) return BWPP_HIP_OK;
+  // The DMA reads whole 16-byte chunks; anything else goes through registers.
+  const bool dma = aligned16(g.a) && aligned16(g.b) && g.lda % 8 == 0 && g.ldb % 8 == 0 &&
+                   (ta ? g.M : g.K) % 8 == 0 && (tb ? g.K : g.N) % 8 == 0 &&
+                   128ull * 2ull * std::max(g.lda, g.ldb) < (1ull << 31) && !(h->gemm_ring > 0 && h->gemm_ring_u);
+  const uint64_t np = ((uint64_t)g.N + 3) / 4 * 4, plane = (uint64_t)g.M * np * 4;
+  const double mem = 4.0 + ((double)g.M * g.K + (double)g.K * g.N + (double)g.M * g.N) * 2.0 / 5.6e6;
+  int best = -1;
+  uint32_t bestS = 1;
+  double best_us = h->gemm_ring > 0 ? 1e301 : full_us;
+  for (int c = 0; c < kRingNCfg; ++c) {
+    if (h->gemm_ring > 0 && c != h->gemm_ring - 1) continue;
+    const RingCfg &r = kRingCfgs[c];
+    const uint64_t tiles = (((uint64_t)g.M + r.bm - 1) / r.bm) * (((uint64_t)g.N + r.bn - 1) / r.bn);
+    for (uint32_t want = 1; want <= 16; ++want) {
+      if (h->gemm_ring > 0 && want != h->gemm_ring_split) continue;
+      const uint32_t kchunk = (uint32_t)((((uint64_t)g.K + want - 1) / want + kQuantum - 1) / kQuantum * kQuantum);
+      const uint32_t S = (g.K + kchunk - 1) / kchunk;
+      if (S != want && h->gemm_ring <= 0) continue;
+      if (tiles * S > 0x7fffffffull || (S > 1 && (!h->gemm_splitk || plane * S > kSplitBytes))) continue;
+      const double n = (double)((tiles * S + cus - 1) / cus);
+      const Cost &k = kCost[dma ? 0 : 1][c];
+      double us = std::max(4.0 + (double)std::min(kchunk, g.K) * (k.lat + (n - 1.0) * k.inc), mem);
+      if (S > 1) us += 3.5 + 2.0 * (double)plane * S / 7e6;
+      if (us < best_us) {
+        best = c;
+        bestS = S;
+        best_us = us;
+      }
+    }
+  }
+  if (best < 0) return BWPP_HIP_OK;
+  void *part = bestS > 1 ? split_scratch(h, (size_t)(plane * bestS)) : nullptr;
+  if (!part) bestS = 1;  // this tile without a split
+  const RingCfg &r = kRingCfgs[best];
+  g.tiles_m = (g.M + r.bm - 1) / r.bm;
+  g.tiles_n = (g.N + r.bn - 1) / r.bn;
+  const uint64_t tiles = (uint64_t)g.tiles_m * g.tiles_n;
+  if (tiles > 0x7fffffffull) return BWPP_HIP_OK;
+  g.ksplit = bestS;
+  g.kchunk = bestS > 1 ? (uint32_t)((((uint64_t)g.K + bestS - 1) / bestS + kQuantum - 1) / kQuantum * kQuantum) : g.K;
+  g.part = static_cast<float *>(part);
+  done = true;
+  BwppHipStatus s = launch(h, h->gemm_bf16_ring[best][ta][tb][dma ? 0 : 1], (uint32_t)(tiles * bestS), 1, 1, r.threads, g);
+  if (s != BWPP_HIP_OK || bestS == 1) return s;
+  const uint64_t vecs = (uint64_t)g.M * (np / 4);
+  return launch(h, h->gemm_bf16_reduce, (uint32_t)std::min<uint64_t>((vecs + 255) / 256, 8 * cus), 1, 1, 256, g);
+}
+
 BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, const void *bias, BwppMatmulParams p,
                           const float *aux, float *c2, BwppHipFusionParams fz) {
   BwppHipStatus s = enter(h);
@@ -1028,6 +1130,17 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
   // BWPP_GEMM_BN=384 asks.
   const bool wide_ok = bf16 && !ta && vec && (!use_bias || aligned16(bias)) && p.M % BM == 0 && p.K % BK == 0 &&
                        p.N % 8 == 0 && h->gemm_waves == 8 && 384ull * 2ull * std::max(lda, ldb) < (1ull << 31);
+  // bf16 ring kernels for any M, N and K, where the model below finds them
+  // faster than the full tiles (whose knobs, when set, ask for those).
+  if (bf16 && p.K >= 128 && h->gemm_ring != 0 && (h->gemm_ring > 0 || (h->gemm_bn == 0 && h->gemm_waves == 8))) {
+    double full_us = 1e300;
+    const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
+    if (full) full_us = 4.0 + 0.0272 * p.K * (double)((tiles + cus - 1) / cus);
+    else if (wide_ok) full_us = 4.0 + 0.041 * p.K * (double)(((uint64_t)g.tiles_m * ((p.N + 383) / 384) + cus - 1) / cus);
+    bool done = false;
+    s = ring_dispatch(h, g, ta, tb, full_us, done);
+    if (s != BWPP_HIP_OK || done) return s;
+  }
   if (wide_ok && (h->gemm_bn == 384 || (h->gemm_bn == 0 && p.N % BN != 0))) {
     g.tiles_n = (p.N + 383) / 384;
     const uint64_t wt = (uint64_t)g.tiles_m * g.tiles_n;
