@@ -100,6 +100,10 @@ __device__ __forceinline__ void store_nt4(float *p, const float4 &o) {
   const f32x4 t = {o.x, o.y, o.z, o.w};
   __builtin_nontemporal_store(t, reinterpret_cast<f32x4 *>(p));
 }
+__device__ __forceinline__ void store4(float *p, const float4 &o) {
+  const f32x4 t = {o.x, o.y, o.z, o.w};
+  *reinterpret_cast<f32x4 *>(p) = t;
+}
 __device__ __forceinline__ float4 load4(const float *p) {
   const f32x4 t = *reinterpret_cast<const f32x4 *>(p);
   return make_float4(t.x, t.y, t.z, t.w);

@@ -1305,6 +1305,281 @@ __device__ __forceinline__ void gemm_f32(const BwppGemmArgs &a) {
   }
 }
 
+// ------------------------------------------------------- fp32, any M, N and K
+//
+// Register-staged tiles for what the 128 x 128 full-tile kernels cannot take
+// or leave idle CUs on: ragged sizes, rows at any 4-byte address (the
+// 16-byte loads need no more), few rows, and small products.  An operand
+// chunk that would pass its row's end is read as the row's last four floats
+// and moved down when it is stored to LDS; rows past M / N re-read the last
+// one (not stored), k past K is zero.  LDS holds both operands K-contiguous
+// as in the kernel above, KPS 32-deep tiles per stage, two stages; the next
+// stage's loads issue before the current one's MFMAs.
+//
+// KW > 1: the waves of a block split each stage's k instead of its tile (one
+// 32 x 32 tile per block, its KW partial sums added in LDS), so that a small
+// product or a few rows still spread over the chip in one launch: 256^3 runs
+// 64 blocks (4.8 us; 10.5 as split-K 128 x 128 tiles and a reduce).  The
+// large tile is bound by the fp32 matrix pipe, one or two blocks per CU
+// hiding the stage's loads (777 x 2043 x 1021, odd rows: 52 us, 122 with
+// guarded element loads).
+template <int R, int NT, bool KC, int KPS>
+struct StageF32 {
+  static constexpr int kVecs = R * 8 * KPS / NT;
+  static_assert(kVecs * NT == R * 8 * KPS && (KC || kVecs % 4 == 0), "tile shape");
+  float4 v[kVecs];
+
+  // Chunk i: its row of the stored operand and first element along it.
+  __device__ __forceinline__ static void place(int i, int tid, uint32_t &row, int &col) {
+    if constexpr (KC) {  // rows of 8 KPS chunks
+      constexpr int kPer = 8 * KPS;
+      const int q = tid + NT * i;
+      row = (uint32_t)(q / kPer);
+      col = 4 * (q % kPer);
+    } else {  // 4 x 4 blocks: four k rows of one mn chunk
+      constexpr int kPer = R / 4;
+      const int q = tid + NT * (i / 4);
+      row = 4u * (uint32_t)(q / kPer) + (uint32_t)(i % 4);
+      col = 4 * (q % kPer);
+    }
+  }
+  // lim rows (KC) or columns, klim k exist.
+  __device__ __forceinline__ void load(const float *g, uint32_t ld, uint32_t lim, uint32_t klim, int tid) {
+    const uint32_t rows = KC ? lim : klim;
+    const int end = (int)(KC ? klim : lim);
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+      uint32_t row;
+      int col;
+      place(i, tid, row, col);
+      v[i] = load4(g + ((int64_t)min(row, rows - 1u) * ld + min(col, end - 4)));
+    }
+  }
+  __device__ __forceinline__ void fix(uint32_t lim, uint32_t klim, int tid) {
+    const int end = (int)(KC ? klim : lim);
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+      uint32_t row;
+      int col;
+      place(i, tid, row, col);
+      const int n = col - min(col, end - 4);  // moved down by n: 0 .. 3, else all past the end
+      float4 x = v[i];
+      const float a0 = n & 2 ? x.z : x.x, a1 = n & 2 ? x.w : x.y, a2 = n & 2 ? 0.0f : x.z, a3 = n & 2 ? 0.0f : x.w;
+      const bool keep = n < 4 && (KC || row < klim);
+      v[i].x = keep ? (n & 1 ? a1 : a0) : 0.0f;
+      v[i].y = keep ? (n & 1 ? a2 : a1) : 0.0f;
+      v[i].z = keep ? (n & 1 ? a3 : a2) : 0.0f;
+      v[i].w = keep ? (n & 1 ? 0.0f : a3) : 0.0f;
+    }
+  }
+  __device__ __forceinline__ void store(float *s, int tid) const {
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+      uint32_t row;
+      int col;
+      place(i, tid, row, col);
+      if constexpr (KC) {
+        *reinterpret_cast<float4 *>(s + (col / 32) * (R * 32) + f32_off(row, (uint32_t)(col % 32) / 4u)) = v[i];
+      } else if (i % 4 == 0) {
+        const float4 &x0 = v[i], &x1 = v[i + 1], &x2 = v[i + 2], &x3 = v[i + 3];
+        float *t = s + (row / 32) * (R * 32);
+        const uint32_t q = (row % 32) / 4u, mn = (uint32_t)col;
+        *reinterpret_cast<float4 *>(t + f32_off(mn + 0, q)) = make_float4(x0.x, x1.x, x2.x, x3.x);
+        *reinterpret_cast<float4 *>(t + f32_off(mn + 1, q)) = make_float4(x0.y, x1.y, x2.y, x3.y);
+        *reinterpret_cast<float4 *>(t + f32_off(mn + 2, q)) = make_float4(x0.z, x1.z, x2.z, x3.z);
+        *reinterpret_cast<float4 *>(t + f32_off(mn + 3, q)) = make_float4(x0.w, x1.w, x2.w, x3.w);
+      }
+    }
+  }
+};
+
+// The fused tail and store of y = C[m][n .. n + 3] (n + 4 <= N, or the
+// elements before N), at any alignment.
+__device__ __forceinline__ void store_c4(const BwppGemmArgs &a, uint32_t m, uint32_t n, float4 y) {
+  float *c = static_cast<float *>(a.c) + (size_t)m * a.ldc + n;
+  const float *aux = a.aux + (size_t)m * a.ldaux + n;
+  float *c2 = a.c2 + (size_t)m * a.ldc2 + n;
+  if (n + 4 <= a.N) {
+    if (fuse_reads_aux(a.fuse)) y = fuse4(a.fuse, y, load4(aux));
+    store4(c, y);
+    if (a.fuse == kFuseDualSilu) store4(c2, make_float4(silu(y.x), silu(y.y), silu(y.z), silu(y.w)));
+  } else {
+    const float v[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e)
+      if (n + e < a.N) {
+        const float t = fuse_reads_aux(a.fuse) ? fuse1(a.fuse, v[e], aux[e]) : v[e];
+        c[e] = t;
+        if (a.fuse == kFuseDualSilu) c2[e] = silu(t);
+      }
+  }
+}
+// bias[n .. n + 3], 0 past N.
+__device__ __forceinline__ float4 bias4(const float *bias, uint32_t n, uint32_t N) {
+  if (n + 4 <= N) return load4(bias + n);
+  float4 b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  if (n < N) b.x = bias[n];
+  if (n + 1 < N) b.y = bias[n + 1];
+  if (n + 2 < N) b.z = bias[n + 2];
+  return b;
+}
+
+template <bool TA, bool TB, int BM, int BN, int WM, int WN, int KW, int KPS>
+__device__ __forceinline__ void gemm_f32_any(const BwppGemmArgs &a) {
+  constexpr int NT = 64 * WM * WN * KW, BK = 32 * KPS;
+  constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32;
+  static_assert(KPS % KW == 0, "each wave takes whole 32-deep tiles");
+  using SA = StageF32<BM, NT, !TA, KPS>;
+  using SB = StageF32<BN, NT, TB, KPS>;
+  constexpr int kTileA = BM * BK, kBuf = kTileA + BN * BK, kCld = BN + 4;
+  constexpr int kOut = KW * BM * kCld;
+  __shared__ __attribute__((aligned(16))) float smemf[2 * kBuf > kOut ? 2 * kBuf : kOut];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kw = wave / (WM * WN), wm = wave % (WM * WN) / WN, wn = wave % WN;
+  const uint32_t tiles = a.tiles_m * a.tiles_n;
+  const uint32_t split = a.ksplit > 1 ? blockIdx.x / tiles : 0u;
+  uint32_t tm, tn;
+  tile_coords(a, tm, tn, blockIdx.x - split * tiles);
+  const uint32_t m0 = tm * BM, n0 = tn * BN;
+  const uint32_t kbeg = a.ksplit > 1 ? split * a.kchunk : 0u;
+  const uint32_t klen = a.ksplit > 1 ? min(a.K - kbeg, a.kchunk) : a.K;
+  const uint32_t ns = (klen + BK - 1) / BK, krem = klen - (ns - 1) * BK;  // k of the last stage
+  const float *A = static_cast<const float *>(a.a) + (TA ? (size_t)kbeg * a.lda + m0 : (size_t)m0 * a.lda + kbeg);
+  const float *B = static_cast<const float *>(a.b) + (TB ? (size_t)n0 * a.ldb + kbeg : (size_t)kbeg * a.ldb + n0);
+  const size_t stepA = TA ? (size_t)BK * a.lda : (size_t)BK, stepB = TB ? (size_t)BK : (size_t)BK * a.ldb;
+  const bool edge = (TA && a.M - m0 < BM) || (!TB && a.N - n0 < BN);  // block-uniform: chunks pass M or N
+
+  // Sums of at most kFlush stages in the MFMA accumulators, then added to
+  // sum: chains of 32 (KW = 4), 64 or 128 products instead of K, as a split
+  // of K would give them (256^3 against 64 bits: 1.6e-7 with one chain per
+  // wave, 1.2e-7 so; 1.3e-7 split 8 ways; 777 x 2043 x 1021 5.7e-7 before,
+  // 1.6e-7).
+  constexpr uint32_t kFlush = KPS >= 2 ? 1 : 4;
+  f32x16_t acc[FN][FM], sum[FN][FM];
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = sum[i][j][r] = 0.0f;
+
+  SA sa;
+  SB sb;
+  auto klim = [&](uint32_t t) { return t + 1 == ns ? krem : (uint32_t)BK; };
+  auto load = [&](uint32_t t) {
+    sa.load(A + t * stepA, a.lda, a.M - m0, klim(t), tid);
+    sb.load(B + t * stepB, a.ldb, a.N - n0, klim(t), tid);
+  };
+  auto store = [&](uint32_t t) {
+    if (edge || klim(t) < BK) {
+      sa.fix(a.M - m0, klim(t), tid);
+      sb.fix(a.N - n0, klim(t), tid);
+    }
+    float *st = smemf + (t & 1u) * kBuf;
+    sa.store(st, tid);
+    sb.store(st + kTileA, tid);
+  };
+  const uint32_t lrow = (uint32_t)(lane & 31), lhi = (uint32_t)(lane >> 5);
+  // 8-k chunk j (0 .. kChunks - 1) of this wave's share of a stage.
+  constexpr int kChunks = 4 * KPS / KW;
+  float4 ac[2][FM], bc[2][FN];
+  auto read = [&](const float *st, int j) {
+    const int sub = kw * (KPS / KW) + j / 4;
+    const uint32_t q = 2u * (uint32_t)(j % 4) + lhi;
+    const float *As = st + sub * (BM * 32), *Bs = st + kTileA + sub * (BN * 32);
+#pragma unroll
+    for (int f = 0; f < FM; ++f)
+      ac[j & 1][f] = *reinterpret_cast<const float4 *>(As + f32_off((uint32_t)(wm * TM + f * 32) + lrow, q));
+#pragma unroll
+    for (int f = 0; f < FN; ++f)
+      bc[j & 1][f] = *reinterpret_cast<const float4 *>(Bs + f32_off((uint32_t)(wn * TN + f * 32) + lrow, q));
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  for (uint32_t t = 0; t < ns; ++t) {
+    const float *st = smemf + (t & 1u) * kBuf;
+    read(st, 0);
+    if (t + 1 < ns) load(t + 1);
+    __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the MFMAs
+#pragma unroll
+    for (int j = 0; j < kChunks; ++j) {
+      if (j + 1 < kChunks) read(st, j + 1);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < FN; ++i)
+#pragma unroll
+          for (int jj = 0; jj < FM; ++jj) {
+            const float4 &xb = bc[j & 1][i], &ya = ac[j & 1][jj];
+            const float x = e == 0 ? xb.x : e == 1 ? xb.y : e == 2 ? xb.z : xb.w;
+            const float y = e == 0 ? ya.x : e == 1 ? ya.y : e == 2 ? ya.z : ya.w;
+            acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x2f32(x, y, acc[i][jj], 0, 0, 0);
+          }
+      // The next stage into the other buffer (nobody reads it during this
+      // one) ahead of the last chunks, which cover the LDS writes.
+      if (j == (kChunks + 1) / 2 - 1) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + 1 < ns) store(t + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (t % kFlush == kFlush - 1 || t + 1 == ns) {
+#pragma unroll
+      for (int i = 0; i < FN; ++i)
+#pragma unroll
+        for (int jj = 0; jj < FM; ++jj)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            sum[i][jj][r] += acc[i][jj][r];
+            acc[i][jj][r] = 0.0f;
+          }
+    }
+    __syncthreads();
+  }
+
+  // C through LDS: raw sums (KW planes), then bias, SiLU and the fused tail
+  // on 16-byte runs; a split's raw sums go to its partial plane.
+  float *mine = smemf + kw * (BM * kCld);
+#pragma unroll
+  for (int i = 0; i < FN; ++i)
+#pragma unroll
+    for (int j = 0; j < FM; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<float4 *>(mine + (wm * TM + j * 32 + (int)lrow) * kCld + wn * TN + i * 32 + q * 8 +
+                                    (int)lhi * 4) =
+            make_float4(sum[i][j][4 * q], sum[i][j][4 * q + 1], sum[i][j][4 * q + 2], sum[i][j][4 * q + 3]);
+  __syncthreads();
+  const float *bias = static_cast<const float *>(a.bias);
+  const bool add = (a.epilogue & kEpiAdd) && bias, act = (a.epilogue & kEpiSilu) != 0;
+  const uint32_t np = (a.N + 3u) & ~3u;
+#pragma unroll 2
+  for (int it = 0; it < BM * (BN / 4) / NT; ++it) {
+    const int q = tid + it * NT, row = q / (BN / 4), c = q % (BN / 4);
+    const uint32_t m = m0 + (uint32_t)row, n = n0 + 4u * (uint32_t)c;
+    if (m >= a.M || n >= a.N) continue;
+    float4 v = *reinterpret_cast<const float4 *>(smemf + row * kCld + c * 4);
+#pragma unroll
+    for (int w = 1; w < KW; ++w) {
+      const float4 u = *reinterpret_cast<const float4 *>(smemf + w * (BM * kCld) + row * kCld + c * 4);
+      v.x += u.x, v.y += u.y, v.z += u.z, v.w += u.w;
+    }
+    if (a.ksplit > 1) {
+      *reinterpret_cast<float4 *>(a.part + ((size_t)split * a.M + m) * np + n) = v;
+      continue;
+    }
+    if (add) {
+      const float4 b = bias4(bias, n, a.N);
+      v.x += b.x, v.y += b.y, v.z += b.z, v.w += b.w;
+    }
+    if (act) v = make_float4(silu(v.x), silu(v.y), silu(v.z), silu(v.w));
+    store_c4(a, m, n, v);
+  }
+}
+
 // ------------------------------------------------------- fp32, DMA ring
 //
 // Full tiles (M, N multiples of 128, K of 32, 16-byte rows): 128 x 128
@@ -1575,19 +1850,18 @@ __device__ __forceinline__ void gemm_f32_pipe(const BwppGemmArgs &a) {
 
 // Split-K reduction: C[m][n..n+3] = epilogue(sum_s part[s][m][n..n+3]) in
 // split order, then bias and SiLU as the single-pass epilogue, then the
-// fused tail.  Needs N a multiple of 4 and 16-byte aligned C (and aux, c2)
-// rows (the full-tile conditions).
+// fused tail.  Partial rows are N rounded up to 4 floats.
 extern "C" __global__ __launch_bounds__(256) void bwpp_gemm_f32_splitk_reduce(const BwppGemmArgs a) {
-  const uint32_t nv = a.N / 4;
-  const size_t total = (size_t)a.M * nv, plane = (size_t)a.M * a.N;
+  const uint32_t nv = (a.N + 3u) / 4u;
+  const size_t total = (size_t)a.M * nv, plane = total * 4;
   const float *bias = static_cast<const float *>(a.bias);
   const bool add = (a.epilogue & kEpiAdd) && bias;
   const bool act = (a.epilogue & kEpiSilu) != 0;
-  float *C = static_cast<float *>(a.c);
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
     const uint32_t m = (uint32_t)(i / nv), n = (uint32_t)(i % nv) * 4;
-    const float *p = a.part + (size_t)m * a.N + n;
+    const float *p = a.part + i * 4;
     float4 t = *reinterpret_cast<const float4 *>(p);
+#pragma unroll 4
     for (uint32_t s = 1; s < a.ksplit; ++s) {
       const float4 u = *reinterpret_cast<const float4 *>(p + s * plane);
       t.x += u.x;
@@ -1596,10 +1870,11 @@ extern "C" __global__ __launch_bounds__(256) void bwpp_gemm_f32_splitk_reduce(co
       t.w += u.w;
     }
     if (add) {
-      t.x += bias[n];
-      t.y += bias[n + 1];
-      t.z += bias[n + 2];
-      t.w += bias[n + 3];
+      const float4 b = bias4(bias, n, a.N);
+      t.x += b.x;
+      t.y += b.y;
+      t.z += b.z;
+      t.w += b.w;
     }
     if (act) {
       t.x = silu(t.x);
@@ -1607,10 +1882,7 @@ extern "C" __global__ __launch_bounds__(256) void bwpp_gemm_f32_splitk_reduce(co
       t.z = silu(t.z);
       t.w = silu(t.w);
     }
-    if (fuse_reads_aux(a.fuse)) t = fuse4(a.fuse, t, *reinterpret_cast<const float4 *>(a.aux + (size_t)m * a.ldaux + n));
-    *reinterpret_cast<float4 *>(C + (size_t)m * a.ldc + n) = t;
-    if (a.fuse == kFuseDualSilu)
-      *reinterpret_cast<float4 *>(a.c2 + (size_t)m * a.ldc2 + n) = make_float4(silu(t.x), silu(t.y), silu(t.z), silu(t.w));
+    store_c4(a, m, n, t);
   }
 }
 
@@ -1669,6 +1941,21 @@ BWPP_GEMM_BF16_RINGS(0, 0)
 BWPP_GEMM_BF16_RINGS(0, 1)
 BWPP_GEMM_BF16_RINGS(1, 0)
 BWPP_GEMM_BF16_RINGS(1, 1)
+
+// bwpp_gemm_f32r<BM>x<BN>_t<TA><TB>.
+#define BWPP_GEMM_F32_ANY(TA, TB, BM, BN, WM, WN, KW, KPS)                                       \
+  extern "C" __global__ __launch_bounds__(64 * WM * WN * KW, 2) void                             \
+      bwpp_gemm_f32r##BM##x##BN##_t##TA##TB(const BwppGemmArgs a) {                              \
+    gemm_f32_any<TA != 0, TB != 0, BM, BN, WM, WN, KW, KPS>(a);                                   \
+  }
+#define BWPP_GEMM_F32_ANYS(TA, TB)                  \
+  BWPP_GEMM_F32_ANY(TA, TB, 32, 32, 1, 1, 4, 4)     \
+  BWPP_GEMM_F32_ANY(TA, TB, 64, 64, 2, 2, 1, 2)     \
+  BWPP_GEMM_F32_ANY(TA, TB, 128, 128, 2, 2, 1, 1)
+BWPP_GEMM_F32_ANYS(0, 0)
+BWPP_GEMM_F32_ANYS(0, 1)
+BWPP_GEMM_F32_ANYS(1, 0)
+BWPP_GEMM_F32_ANYS(1, 1)
 
 #define BWPP_GEMM_BF16(TA, TB, EDGE, SUF)                                                  \
   extern "C" __global__ __attribute__((amdgpu_flat_work_group_size(256, 256),            \

@@ -59,6 +59,9 @@ struct RingCfg {
 };
 constexpr int kRingNCfg = 5;
 const RingCfg kRingCfgs[kRingNCfg] = {{32, 64, 128}, {64, 64, 256}, {64, 128, 256}, {128, 128, 256}, {128, 256, 512}};
+// Tiles of the fp32 kernels for any M, N and K (256 threads each).
+constexpr int kAnyNCfg = 3;
+const RingCfg kAnyCfgs[kAnyNCfg] = {{32, 32, 256}, {64, 64, 256}, {128, 128, 256}};
 int find_cfg(int vpt, int wpr) {
   for (int i = 0; i < kRowNCfg; ++i)
     if (kRowCfgs[i].vpt == vpt && kRowCfgs[i].wpr == wpr) return i;
@@ -95,8 +98,10 @@ struct BwppHip {
   hipFunction_t gemm[2][2][2][2] = {};
   hipFunction_t gemm_bf16_ring[kRingNCfg][2][2][2] = {};  // any M, N, K: [kRingCfgs][ta][tb][unaligned]
   hipFunction_t gemm_bf16_reduce = nullptr;
-  // BWPP_GEMM_RING: 0 = those kernels off; c,S = tile kRingCfgs[c - 1] with S
-  // K ranges (through registers with a trailing u) wherever they can run.
+  hipFunction_t gemm_f32_any[kAnyNCfg][2][2] = {};  // fp32, any M, N, K: [kAnyCfgs][ta][tb]
+  // BWPP_GEMM_RING: 0 = the kernels for any M, N, K off; c,S = their tile c
+  // (kRingCfgs / kAnyCfgs from 1) with S K ranges (bf16 through registers with
+  // a trailing u) wherever they can run.
   int gemm_ring = -1;
   uint32_t gemm_ring_split = 1;
   bool gemm_ring_u = false;
@@ -331,6 +336,11 @@ BwppHipStatus resolve_all(BwppHip *h) {
                                std::to_string(kRingCfgs[c].bn) + "_t" + std::to_string(ta) + std::to_string(tb);
         if ((s = resolve(h, nr, &h->gemm_bf16_ring[c][ta][tb][0])) != BWPP_HIP_OK) return s;
         if ((s = resolve(h, nr + "_u", &h->gemm_bf16_ring[c][ta][tb][1])) != BWPP_HIP_OK) return s;
+      }
+      for (int c = 0; c < kAnyNCfg; ++c) {
+        const std::string na = "bwpp_gemm_f32r" + std::to_string(kAnyCfgs[c].bm) + "x" +
+                               std::to_string(kAnyCfgs[c].bn) + "_t" + std::to_string(ta) + std::to_string(tb);
+        if ((s = resolve(h, na, &h->gemm_f32_any[c][ta][tb])) != BWPP_HIP_OK) return s;
       }
       const std::string n = "bwpp_gemm_bf16w8_t" + std::to_string(ta) + std::to_string(tb) + "_f";
       if ((s = resolve(h, n, &h->gemm_bf16_w8[ta][tb])) != BWPP_HIP_OK) return s;
@@ -968,53 +978,61 @@ BwppHipStatus ensure_ws(BwppHip *h, size_t bytes);
 
 namespace {
 
-// bf16 ring kernels (gemm.hip, gemm_bf16_ring) for a product whose operands
-// are set in g: picks the tile and the number of K ranges S with the least
-// modelled time and launches them unless full_us, the modelled time of a
-// full-tile kernel that could run, is less (done stays false).  Per K element,
-// n blocks on a CU take lat + (n - 1) inc us; every launch costs 4 us with
-// its prologue and epilogue, a split 3.5 us and its partial planes' traffic at
-// 7 TB/s (they stay in the Infinity Cache), and no product runs faster than
-// its operands arrive (5.6 TB/s).  The full tiles: 0.0272 us per K and round
-// of 256 x 256 tiles (4096^3: 115 us), 0.041 of 256 x 384.  Fitted on MI355X
-// to 26 products from 9 x 9 x 200 to 4095 x 8191 x 2048, all transposes,
-// S = 1 .. 8; the choice is within 15 % of the best of all tiles and splits
-// on each (16 x 11008 x 4096: 210 us on the 256 x 256 edge tile, 18.2 so;
-// 1337 x 3000 x 1024 94 -> 17.5; 512 x 1024 x 1024 25.5 -> 6.5; 4000^3, B
-// transposed, 189 -> 134; 4095 x 8191 x 2048, odd rows, 1085 -> 170).
-BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool ta, bool tb, double full_us, bool &done) {
+// Kernels for any M, N and K (gemm.hip: gemm_bf16_ring, gemm_f32_any) for a
+// product whose operands are set in g: picks the tile and the number of K
+// ranges S with the least modelled time and launches them unless full_us, the
+// modelled time of a full-tile kernel that could run, is less (done stays
+// false, as where the operands are too small for their 16-byte chunks).
+// Per K element, n blocks on a CU take lat + (n - 1) inc us; every launch
+// costs 4 us with its prologue and epilogue, a split 3.5 us and its partial
+// planes' traffic at 7 TB/s (they stay in the Infinity Cache), and no product
+// runs faster than its operands arrive (5.6 TB/s).  Fitted on MI355X to 26
+// bf16 products from 9 x 9 x 200 to 4095 x 8191 x 2048 and 16 fp32 ones from 5
+// x 7 x 9 to 2048^3, all transposes, S = 1 .. 8; the choice is within 15 % of
+// the best of all tiles and splits on each.  M x N x K: bf16 16 x 11008 x 4096
+// 210 us on the 256 x 256 edge tile, 18.2 so; 1337 x 3000 x 1024 94 -> 17.5;
+// 512 x 1024 x 1024 25.5 (full tiles) -> 6.5; 4000^3, B transposed, 189 ->
+// 134; 4095 x 8191 x 2048, odd rows, 1085 -> 170.  fp32 256^3 10.0 (split full
+// tiles) -> 4.9; 777 x 2043 x 1021 122 -> 52; 32 x 384 x 5823 528 -> 14.
+BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool bf16, bool ta, bool tb, double full_us, bool &done) {
   struct Cost {
     double lat, inc;
   };
-  // [through registers][kRingCfgs]
-  static const Cost kCost[2][kRingNCfg] = {
+  static const Cost kBf16[2][kRingNCfg] = {  // [through registers]
       {{0.0039, 0.0045}, {0.0046, 0.0037}, {0.0085, 0.0055}, {0.0114, 0.0085}, {0.0158, 0.0158}},
       {{0.0085, 0.0031}, {0.0088, 0.0042}, {0.0146, 0.0060}, {0.0185, 0.0105}, {0.0275, 0.0180}}};
+  static const Cost kF32[kAnyNCfg] = {{0.0082, 0.0066}, {0.0225, 0.0210}, {0.0780, 0.0580}};
   constexpr uint32_t kQuantum = 128;  // K ranges in multiples of the deepest stage
   const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
-  if (std::max({g.M, g.N, g.K}) > 0x7fffffffu || (ta && g.M < 8) || (!tb && g.N < 8)) return BWPP_HIP_OK;
-  // The DMA reads whole 16-byte chunks; anything else goes through registers.
+  const uint32_t chunk = bf16 ? 8u : 4u, es = bf16 ? 2u : 4u;
+  if (std::max({g.M, g.N, g.K}) > 0x7fffffffu || (ta && g.M < chunk) || (!tb && g.N < chunk) ||
+      ((!ta || tb) && g.K < chunk) || g.K == 0)
+    return BWPP_HIP_OK;
+  const bool forced = h->gemm_ring > 0;
+  // The bf16 DMA reads whole 16-byte chunks; anything else goes through registers.
   const bool dma = aligned16(g.a) && aligned16(g.b) && g.lda % 8 == 0 && g.ldb % 8 == 0 &&
                    (ta ? g.M : g.K) % 8 == 0 && (tb ? g.K : g.N) % 8 == 0 &&
-                   128ull * 2ull * std::max(g.lda, g.ldb) < (1ull << 31) && !(h->gemm_ring > 0 && h->gemm_ring_u);
+                   128ull * 2ull * std::max(g.lda, g.ldb) < (1ull << 31) && !(forced && h->gemm_ring_u);
+  const RingCfg *cfgs = bf16 ? kRingCfgs : kAnyCfgs;
+  const Cost *costs = bf16 ? kBf16[dma ? 0 : 1] : kF32;
+  const int ncfg = bf16 ? kRingNCfg : kAnyNCfg;
   const uint64_t np = ((uint64_t)g.N + 3) / 4 * 4, plane = (uint64_t)g.M * np * 4;
-  const double mem = 4.0 + ((double)g.M * g.K + (double)g.K * g.N + (double)g.M * g.N) * 2.0 / 5.6e6;
+  const double mem = 4.0 + ((double)g.M * g.K + (double)g.K * g.N + (double)g.M * g.N) * es / 5.6e6;
   int best = -1;
   uint32_t bestS = 1;
-  double best_us = h->gemm_ring > 0 ? 1e301 : full_us;
-  for (int c = 0; c < kRingNCfg; ++c) {
-    if (h->gemm_ring > 0 && c != h->gemm_ring - 1) continue;
-    const RingCfg &r = kRingCfgs[c];
+  double best_us = forced ? 1e301 : full_us;
+  for (int c = 0; c < ncfg; ++c) {
+    if (forced && c != h->gemm_ring - 1) continue;
+    const RingCfg &r = cfgs[c];
     const uint64_t tiles = (((uint64_t)g.M + r.bm - 1) / r.bm) * (((uint64_t)g.N + r.bn - 1) / r.bn);
     for (uint32_t want = 1; want <= 16; ++want) {
-      if (h->gemm_ring > 0 && want != h->gemm_ring_split) continue;
+      if (forced && want != h->gemm_ring_split) continue;
       const uint32_t kchunk = (uint32_t)((((uint64_t)g.K + want - 1) / want + kQuantum - 1) / kQuantum * kQuantum);
       const uint32_t S = (g.K + kchunk - 1) / kchunk;
-      if (S != want && h->gemm_ring <= 0) continue;
+      if (S != want && !forced) continue;
       if (tiles * S > 0x7fffffffull || (S > 1 && (!h->gemm_splitk || plane * S > kSplitBytes))) continue;
       const double n = (double)((tiles * S + cus - 1) / cus);
-      const Cost &k = kCost[dma ? 0 : 1][c];
-      double us = std::max(4.0 + (double)std::min(kchunk, g.K) * (k.lat + (n - 1.0) * k.inc), mem);
+      double us = std::max(4.0 + (double)std::min(kchunk, g.K) * (costs[c].lat + (n - 1.0) * costs[c].inc), mem);
       if (S > 1) us += 3.5 + 2.0 * (double)plane * S / 7e6;
       if (us < best_us) {
         best = c;
@@ -1026,7 +1044,7 @@ BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool ta, bool tb, double
   if (best < 0) return BWPP_HIP_OK;
   void *part = bestS > 1 ? split_scratch(h, (size_t)(plane * bestS)) : nullptr;
   if (!part) bestS = 1;  // this tile without a split
-  const RingCfg &r = kRingCfgs[best];
+  const RingCfg &r = cfgs[best];
   g.tiles_m = (g.M + r.bm - 1) / r.bm;
   g.tiles_n = (g.N + r.bn - 1) / r.bn;
   const uint64_t tiles = (uint64_t)g.tiles_m * g.tiles_n;
@@ -1035,10 +1053,12 @@ BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool ta, bool tb, double
   g.kchunk = bestS > 1 ? (uint32_t)((((uint64_t)g.K + bestS - 1) / bestS + kQuantum - 1) / kQuantum * kQuantum) : g.K;
   g.part = static_cast<float *>(part);
   done = true;
-  BwppHipStatus s = launch(h, h->gemm_bf16_ring[best][ta][tb][dma ? 0 : 1], (uint32_t)(tiles * bestS), 1, 1, r.threads, g);
+  BwppHipStatus s = launch(h, bf16 ? h->gemm_bf16_ring[best][ta][tb][dma ? 0 : 1] : h->gemm_f32_any[best][ta][tb],
+                           (uint32_t)(tiles * bestS), 1, 1, r.threads, g);
   if (s != BWPP_HIP_OK || bestS == 1) return s;
   const uint64_t vecs = (uint64_t)g.M * (np / 4);
-  return launch(h, h->gemm_bf16_reduce, (uint32_t)std::min<uint64_t>((vecs + 255) / 256, 8 * cus), 1, 1, 256, g);
+  return launch(h, bf16 ? h->gemm_bf16_reduce : h->gemm_f32_reduce,
+                (uint32_t)std::min<uint64_t>((vecs + 255) / 256, 8 * cus), 1, 1, 256, g);
 }
 
 BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, const void *bias, BwppMatmulParams p,
@@ -1130,15 +1150,18 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
   // BWPP_GEMM_BN=384 asks.
   const bool wide_ok = bf16 && !ta && vec && (!use_bias || aligned16(bias)) && p.M % BM == 0 && p.K % BK == 0 &&
                        p.N % 8 == 0 && h->gemm_waves == 8 && 384ull * 2ull * std::max(lda, ldb) < (1ull << 31);
-  // bf16 ring kernels for any M, N and K, where the model below finds them
-  // faster than the full tiles (whose knobs, when set, ask for those).
-  if (bf16 && p.K >= 128 && h->gemm_ring != 0 && (h->gemm_ring > 0 || (h->gemm_bn == 0 && h->gemm_waves == 8))) {
+  // bf16: the kernels for any M, N and K, where their model finds them faster
+  // than the full tiles (0.0272 us per K and round of 256 x 256 tiles, 4096^3
+  // in 115 us; 0.041 of 256 x 384), whose knobs, when set, ask for those.
+  // Below K = 128 the ring does not pay for its prologue.
+  const bool any = h->gemm_ring != 0 && (h->gemm_ring > 0 || (h->gemm_bn == 0 && h->gemm_waves == 8));
+  bool done = false;
+  if (bf16 && any && p.K >= 128) {
     double full_us = 1e300;
     const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
     if (full) full_us = 4.0 + 0.0272 * p.K * (double)((tiles + cus - 1) / cus);
     else if (wide_ok) full_us = 4.0 + 0.041 * p.K * (double)(((uint64_t)g.tiles_m * ((p.N + 383) / 384) + cus - 1) / cus);
-    bool done = false;
-    s = ring_dispatch(h, g, ta, tb, full_us, done);
+    s = ring_dispatch(h, g, true, ta, tb, full_us, done);
     if (s != BWPP_HIP_OK || done) return s;
   }
   if (wide_ok && (h->gemm_bn == 384 || (h->gemm_bn == 0 && p.N % BN != 0))) {
@@ -1206,6 +1229,11 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
         }
       }
     }
+    if (mode == 1 && h->gemm_ring != 0) {
+      // Small products: smaller tiles, one launch (256^3 10.0 -> 4.9 us).
+      s = ring_dispatch(h, g, false, ta, tb, best + 2.0, done);
+      if (s != BWPP_HIP_OK || done) return s;
+    }
     const int ring4 = bestKind == 2;
     if (bestS > 1) {
       if ((s = ensure_ws(h, (size_t)bestS * p.M * p.N * sizeof(float))) != BWPP_HIP_OK) return s;
@@ -1220,6 +1248,10 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
       return launch(h, h->gemm_f32_reduce, (uint32_t)grid, 1, 1, 256, g);
     }
     if (bestKind) return launch(h, h->gemm_f32p[ring4][ta][tb][0], (uint32_t)tiles, 1, 1, 256, g);
+  }
+  if (!bf16 && !full && h->gemm_ring != 0) {
+    s = ring_dispatch(h, g, false, ta, tb, 1e300, done);
+    if (s != BWPP_HIP_OK || done) return s;
   }
   return launch(h, h->gemm[bf16 ? 1 : 0][ta][tb][full ? 1 : 0], (uint32_t)tiles, 1, 1, 256, g);
 }
