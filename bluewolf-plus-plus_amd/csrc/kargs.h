@@ -93,6 +93,12 @@ typedef struct {
   void *dst;
   uint32_t ld_dst;
   uint32_t items; /* persistent flash forward: (slice, query tile) items */
+  /* Few queries (decoding): the keys of a slice in ksplit ranges of kchunk;
+   * with ksplit > 1, range s of slice b leaves its sums of p v
+   * ([M][vdim]) at part_o + (b ksplit + s) M vdim and per query the pair
+   * (exponent offset, sum of p) at part_ml + 2 (b ksplit + s) M. */
+  uint32_t ksplit, kchunk;
+  float *part_o, *part_ml;
 } BwppAttnArgs;
 
 /* Attention operand copies between the caller's strided bf16 layout

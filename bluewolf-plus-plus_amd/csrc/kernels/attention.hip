@@ -1249,6 +1249,296 @@ __device__ __forceinline__ void attn_bf16_small(const BwppAttnArgs &a) {
   }
 }
 
+// -------------------------------------------------- bf16, at most 32 queries
+// Decoding: a few queries against a long cache, bound by reading K and V
+// once (4 flop per byte and query).  A block of 4 waves owns one slice and a
+// range of its keys; every wave holds all the queries as the MFMA "B" operand
+// and streams key tiles of 32 of its own (every fourth of the block's)
+// through a DMA ring of its own, so the waves never wait for one another:
+// 16 KiB of K and V per wave in flight while the previous tile is multiplied.
+// The waves' (offset, sum, O) triples meet in LDS at the end, and those of a
+// split slice in bwpp_attn_dec_combine.  P enters the second product as two
+// bf16 terms (see above).  B8 H32 M1 N4095 d128: 256-query tiles, one block
+// per slice 116-144 us, this 94 us (537 MB at 5.7 TB/s); B1 H32 M1 N8192 172
+// -> 27 (split 8 ways).
+//
+// Tiles with masked keys look for non-finite V elements; where one is found
+// the tile's sums are formed element by element over visible keys only.
+template <int D, bool CAUSAL>
+__device__ __forceinline__ void attn_bf16_dec(const BwppAttnArgs &a) {
+  using T = AttnTile<D>;
+  constexpr int NW = 4, kKeys = 32, KS = D / 16, DB = D / 32;
+  constexpr int kTile = kKeys * T::kRowB, kStage = 2 * kTile;
+  constexpr int kStages = 32768 / kStage;      // 32 KiB per wave
+  constexpr int kDma = kTile / 1024;           // DMA instructions per K (or V) tile
+  constexpr int kCld = D + 4;                  // merge: [wave][32 queries][D + 4] floats
+  static_assert(kStages >= 2 && NW * 32 * kCld * 4 <= NW * kStages * kStage, "merge reuses the rings");
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[NW * kStages * kStage];
+  __shared__ float ps[NW][kKeys][33];          // a tile's probabilities (non-finite V only)
+  __shared__ float mls[NW][32][2];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const uint32_t bh = blockIdx.x / a.ksplit, sp = blockIdx.x % a.ksplit;
+  const uint32_t b = bh / a.heads, h = bh % a.heads;
+  const uint16_t *Q = static_cast<const uint16_t *>(a.q) + b * a.q_bs + h * a.q_hs;
+  const uint16_t *K = static_cast<const uint16_t *>(a.k) + b * a.k_bs + h * a.k_hs;
+  const uint16_t *V = static_cast<const uint16_t *>(a.v) + b * a.v_bs + h * a.v_hs;
+  const int64_t diag = (int64_t)a.N - (int64_t)a.M;  // key n visible to query m iff n <= m + diag
+  const uint32_t lq = (uint32_t)(lane & 31), lh = (uint32_t)(lane >> 5);
+
+  // Keys of this block: [kbeg, kend), kbeg a multiple of 32.
+  const uint32_t kbeg = sp * a.kchunk, kend = min(a.N, kbeg + a.kchunk);
+  const uint32_t ntile = kbeg < kend ? (kend - kbeg + kKeys - 1) / kKeys : 0u;
+  const uint32_t nmine = ntile > (uint32_t)wave ? (ntile - (uint32_t)wave + NW - 1) / NW : 0u;
+
+  bf16x8_t qf[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (lq < a.M) v = *reinterpret_cast<const uint4 *>(Q + (size_t)lq * a.ldq + 16 * ks + 8 * lh);
+    qf[ks] = __builtin_bit_cast(bf16x8_t, v);
+  }
+  wait_vmcnt<0>();  // no load of the compiler's outstanding beside the DMA
+
+  unsigned char *ring = smem + wave * (kStages * kStage);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)ring;
+  uint32_t dma_row[kDma], dma_kcol[kDma], dma_vcol[kDma];
+#pragma unroll
+  for (int i = 0; i < kDma; ++i) {
+    const uint32_t q = (uint32_t)i * 64u + (uint32_t)lane, r = q / T::kSlots, pc = q % T::kSlots;
+    dma_row[i] = r;
+    dma_kcol[i] = 8u * (pc ^ T::k_swz(r));
+    dma_vcol[i] = 8u * (pc ^ T::v_swz(r));
+  }
+  static_assert(D / 8 == T::kSlots, "every slot of a row is in use");
+  // Tile j of this wave: keys from kbeg + 32 (4 j + wave); rows past N
+  // re-read row N - 1 (masked below).
+  auto issue = [&](uint32_t j) {
+    const uint32_t k0 = kbeg + kKeys * (NW * j + (uint32_t)wave), st = lds0 + (j % kStages) * kStage;
+#pragma unroll
+    for (int i = 0; i < kDma; ++i) {
+      const uint32_t key = min(k0 + dma_row[i], a.N - 1);
+      g2lds16_so(K, 2u * (key * a.ldk + dma_kcol[i]), st + (uint32_t)i * 1024u);
+      g2lds16_so(V, 2u * (key * a.ldv + dma_vcol[i]), st + kTile + (uint32_t)i * 1024u);
+    }
+  };
+
+  f32x16_t o[DB];
+#pragma unroll
+  for (int d = 0; d < DB; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[d][r] = 0.0f;
+  float mrow = -INFINITY, lrow = 0.0f;
+  const float c = a.scale_log2;
+  const uint32_t grp = (uint32_t)((lane >> 4) & 3), L = (uint32_t)(lane & 15);
+  uint32_t koff[KS], voff[DB];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) koff[ks] = lq * T::kRowB + 16u * ((2u * ks + lh) ^ T::k_swz(lq));
+  {
+    const uint32_t kbase = 4u * (grp >> 1) + (L >> 2);
+#pragma unroll
+    for (int d = 0; d < DB; ++d) {
+      const uint32_t col = 32u * d + 16u * (grp & 1u) + 4u * (L & 3u);
+      voff[d] = kTile + kbase * T::kRowB + 16u * ((col >> 3) ^ T::v_swz(kbase)) + (col & 7u) * 2u;
+    }
+  }
+
+#pragma unroll
+  for (int j = 0; j < kStages - 1; ++j)
+    if ((uint32_t)j < nmine) issue((uint32_t)j);
+  for (uint32_t j = 0; j < nmine; ++j) {
+    const uint32_t k0 = kbeg + kKeys * (NW * j + (uint32_t)wave);
+    const uint32_t younger = min(nmine - 1 - j, (uint32_t)(kStages - 2));
+    if (kStages >= 4 && younger >= 2) wait_vmcnt<(kStages >= 4 ? 4 * kDma : 0)>();
+    else if (kStages >= 3 && younger >= 1) wait_vmcnt<(kStages >= 3 ? 2 * kDma : 0)>();
+    else wait_vmcnt<0>();
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): done reading the stage that is refilled now
+    if (j + kStages - 1 < nmine) issue(j + kStages - 1);
+    const unsigned char *st = ring + __builtin_amdgcn_readfirstlane((j % kStages) * kStage);
+    f32x16_t s;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] = 0.0f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+          __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4 *>(st + koff[ks])), qf[ks], s, 0, 0, 0);
+    // Key of register r: k0 + 4 lh + 8 (r >> 2) + (r & 3); visible below lim.
+    const bool masked = k0 + kKeys > kend || (CAUSAL && (int64_t)k0 + kKeys - 1 > diag);  // wave-uniform
+    int64_t lim64 = (int64_t)kend - (int64_t)(k0 + 4u * lh);
+    if (CAUSAL) lim64 = min(lim64, (int64_t)lq + diag + 1 - (int64_t)(k0 + 4u * lh));
+    const int lim = (int)(lim64 < -1 ? -1 : (lim64 > kKeys ? kKeys : lim64));
+    if (masked) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[r] = 8 * (r >> 2) + (r & 3) < lim ? s[r] : -INFINITY;
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    {
+      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) * c;
+    }
+    float alpha = 1.0f;
+    if (mx > mrow + kLazy) {
+      alpha = __builtin_amdgcn_exp2f(mrow - mx);  // 0 when mrow is -inf
+      mrow = mx;
+    }
+    const float muse = mrow == -INFINITY ? 0.0f : mrow;
+    float sum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -muse));
+      s[r] = p;
+      sum += p;
+    }
+    {
+      const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+      sum = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    lrow = lrow * alpha + sum;
+    if (__ballot(alpha != 1.0f)) {
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+    }
+    v8s_t vv[2][DB];
+#pragma unroll
+    for (int kq = 0; kq < 2; ++kq)
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        const unsigned char *p = st + voff[d] + 16u * kq * T::kRowB;
+        const v4s_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)p);
+        const v4s_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t *)(p + 8u * T::kRowB));
+        vv[kq][d] = v8s_t{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      }
+    bool plain = true;
+    if (masked) {
+      u16x2_t big = {0, 0};
+#pragma unroll
+      for (int kq = 0; kq < 2; ++kq)
+#pragma unroll
+        for (int d = 0; d < DB; ++d) big = max_abs_bf16(big, vv[kq][d]);
+      plain = __ballot(big[0] >= 0x7f80u || big[1] >= 0x7f80u) == 0;
+    }
+    if (plain) {
+#pragma unroll
+      for (int kq = 0; kq < 2; ++kq) {
+        bf16x8_t ph, pl;
+        split_bf16x8(&s, 8 * kq, ph, pl);
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vv[kq][d]), ph, o[d], 0, 0, 0);
+          o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, vv[kq][d]), pl, o[d], 0, 0, 0);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ps[wave][8 * (r >> 2) + 4 * lh + (r & 3)][lq] = s[r];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const int64_t vis = lim64 + 4 * (int64_t)lh;  // keys of the tile that this lane's query sees
+      for (int key = 0; key < kKeys; ++key) {
+        const float p = ps[wave][key][lq];
+        const unsigned char *vr = st + kTile + (uint32_t)key * T::kRowB;
+        if (key < vis) {
+#pragma unroll
+          for (int d = 0; d < DB; ++d)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+              const uint32_t col = 32u * d + 8u * (r >> 2) + 4u * lh + (r & 3);
+              const uint16_t *e = reinterpret_cast<const uint16_t *>(
+                  vr + 16u * ((col >> 3) ^ T::v_swz((uint32_t)key)) + 2u * (col & 7u));
+              o[d][r] += p * bf16_bits_to_f32(*e);
+            }
+        }
+      }
+    }
+  }
+
+  // The four waves' triples: O (this lane's query, d = 32 db + 8 (r >> 2) +
+  // 4 lh + (r & 3)) and (offset, sum).
+  __syncthreads();
+  float *os = reinterpret_cast<float *>(smem) + wave * (32 * kCld);
+#pragma unroll
+  for (int d = 0; d < DB; ++d)
+#pragma unroll
+    for (int q4 = 0; q4 < 4; ++q4)
+      *reinterpret_cast<float4 *>(os + lq * kCld + 32 * d + 8 * q4 + 4 * (int)lh) =
+          make_float4(o[d][4 * q4], o[d][4 * q4 + 1], o[d][4 * q4 + 2], o[d][4 * q4 + 3]);
+  if (lh == 0) {
+    mls[wave][lq][0] = mrow;
+    mls[wave][lq][1] = lrow;
+  }
+  __syncthreads();
+  uint16_t *O = static_cast<uint16_t *>(a.o) + b * a.o_bs + h * a.o_hs;
+  for (uint32_t i = threadIdx.x; i < a.M * (D / 4); i += 64 * NW) {
+    const uint32_t q = i / (D / 4), d4 = 4u * (i % (D / 4));
+    float m = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) m = fmaxf(m, mls[w][q][0]);
+    float l = 0.0f;
+    float4 t = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float mw = mls[w][q][0];
+      // No key seen (offset -inf): sums of 0 (or NaN, kept).
+      const float f = mw == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(mw - m);
+      const float4 u = *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(smem) + (w * 32 + q) * kCld + d4);
+      l += mls[w][q][1] * f;
+      t.x += u.x * f, t.y += u.y * f, t.z += u.z * f, t.w += u.w * f;
+    }
+    if (a.ksplit > 1) {
+      const size_t row = (size_t)blockIdx.x * a.M + q;
+      *reinterpret_cast<float4 *>(a.part_o + row * D + d4) = t;
+      if (d4 == 0) {
+        a.part_ml[2 * row] = m;
+        a.part_ml[2 * row + 1] = l;
+      }
+      continue;
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    *reinterpret_cast<uint2 *>(O + (size_t)q * a.ldo + d4) =
+        make_uint2(pack_bf16x2(t.x * inv, t.y * inv), pack_bf16x2(t.z * inv, t.w * inv));
+    if (a.lse && d4 == 0)
+      a.lse[(size_t)bh * a.M + q] =
+          l > 0.0f ? __builtin_fmaf(m == -INFINITY ? 0.0f : m, 0.69314718055994531f, logf(l)) : -INFINITY;
+  }
+}
+
+// Merges the ksplit partial triples of a slice's queries: a thread per four
+// d of one query.
+template <class T>
+__device__ __forceinline__ void attn_dec_combine(const BwppAttnArgs &a, uint32_t slices) {
+  const uint32_t D = a.vdim, n4 = D / 4;
+  const uint64_t total = (uint64_t)slices * a.M * n4;
+  for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < total; i += (uint64_t)gridDim.x * 256u) {
+    const uint32_t d4 = 4u * (uint32_t)(i % n4), q = (uint32_t)(i / n4 % a.M), bh = (uint32_t)(i / n4 / a.M);
+    const size_t row0 = (size_t)bh * a.ksplit * a.M + q;
+    float m = -INFINITY;
+    for (uint32_t s = 0; s < a.ksplit; ++s) m = fmaxf(m, a.part_ml[2 * (row0 + (size_t)s * a.M)]);
+    float l = 0.0f;
+    float4 t = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 4
+    for (uint32_t s = 0; s < a.ksplit; ++s) {
+      const size_t row = row0 + (size_t)s * a.M;
+      const float mw = a.part_ml[2 * row];
+      const float f = mw == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(mw - m);
+      const float4 u = *reinterpret_cast<const float4 *>(a.part_o + row * D + d4);
+      l += a.part_ml[2 * row + 1] * f;
+      t.x += u.x * f, t.y += u.y * f, t.z += u.z * f, t.w += u.w * f;
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    T *O = static_cast<T *>(a.o) + bh / a.heads * a.o_bs + bh % a.heads * a.o_hs + (size_t)q * a.ldo + d4;
+    st_elem(O, t.x * inv), st_elem(O + 1, t.y * inv), st_elem(O + 2, t.z * inv), st_elem(O + 3, t.w * inv);
+    if (a.lse && d4 == 0)
+      a.lse[(size_t)bh * a.M + q] =
+          l > 0.0f ? __builtin_fmaf(m == -INFINITY ? 0.0f : m, 0.69314718055994531f, logf(l)) : -INFINITY;
+  }
+}
+
 // ------------------------------------------------------- backward (generic)
 // O = softmax(scale Q K^T [mask]) V.  With the saved lse (natural-log
 // log-sum-exp per query) the probabilities are recomputed as
@@ -1451,6 +1741,20 @@ BWPP_ATTN_BWD(bwpp_attn_bwd_bf16_causal, uint16_t, true)
 BWPP_ATTN_SMALL(32, 4)
 BWPP_ATTN_SMALL(64, 3)
 BWPP_ATTN_SMALL(96, 2)
+
+#define BWPP_ATTN_DEC(D)                                                                       \
+  extern "C" __global__ __launch_bounds__(256) void bwpp_attn_bf16_dec_d##D(const BwppAttnArgs a) { \
+    attn_bf16_dec<D, false>(a);                                                                \
+  }                                                                                            \
+  extern "C" __global__ __launch_bounds__(256) void bwpp_attn_bf16_dec_d##D##_causal(          \
+      const BwppAttnArgs a) {                                                                  \
+    attn_bf16_dec<D, true>(a);                                                                 \
+  }
+BWPP_ATTN_DEC(64)
+BWPP_ATTN_DEC(128)
+extern "C" __global__ __launch_bounds__(256) void bwpp_attn_dec_combine_bf16(const BwppAttnArgs a) {
+  attn_dec_combine<uint16_t>(a, a.items);
+}
 
 // Generic path entry points, one per storage type x mask.
 #define BWPP_ATTN_GENERIC(NAME, T, CAUSAL)                                                  \

@@ -112,6 +112,9 @@ struct BwppHip {
   hipFunction_t attn_flash[2] = {};       // bf16, d = 128: [causal]
   hipFunction_t attn_flash_p[2] = {};     // bf16, d = 128, persistent (one block per CU): [causal]
   hipFunction_t attn_bf16_small[3][2] = {};  // bf16, d = 32 / 64 / 96: [d / 32 - 1][causal]
+  hipFunction_t attn_bf16_dec[2][2] = {};    // bf16, at most 32 queries, d = 64 / 128: [d128][causal]
+  hipFunction_t attn_dec_combine[2] = {};    // [bf16]
+  uint32_t attn_dec = 1;                     // BWPP_ATTN_DEC=0: off
   // BWPP_ATTN_FLASH_PERSIST: bit c set = persistent kernel when causal == c
   // (default unmasked only: causal C4 321.5 against 321.6 us, B2 H16 S4096
   // N 4096 +0.8 %, only B16 H16 S1024 -4.6 %).
@@ -285,6 +288,7 @@ BwppHipStatus resolve_all(BwppHip *h) {
       {"bwpp_col_maxgrad", &h->col_maxgrad},         {"bwpp_col_mask", &h->col_mask},
       {"bwpp_silu_grad", &h->silu_grad},             {"bwpp_softmax_grad", &h->softmax_grad},
       {"bwpp_gemm_bf16_splitk_reduce", &h->gemm_bf16_reduce},
+      {"bwpp_attn_dec_combine_bf16", &h->attn_dec_combine[1]},
       {"bwpp_rmsnorm_grad", &h->rmsnorm_grad},       {"bwpp_col_partials_sum", &h->col_partials_sum},
       {"bwpp_reduce_sum_rows", &h->reduce_sum_rows}, {"bwpp_reduce_sum_cols", &h->reduce_sum_cols},
       {"bwpp_mean_square_part", &h->mean_square_part}, {"bwpp_mean_square_final", &h->mean_square_final},
@@ -367,6 +371,10 @@ BwppHipStatus resolve_all(BwppHip *h) {
       return s;
     if ((s = resolve(h, std::string("bwpp_attn_generic_bf16") + cs, &h->attn_generic[1][causal])) != BWPP_HIP_OK)
       return s;
+    for (int d128 = 0; d128 < 2; ++d128)
+      if ((s = resolve(h, std::string("bwpp_attn_bf16_dec_d") + (d128 ? "128" : "64") + cs,
+                       &h->attn_bf16_dec[d128][causal])) != BWPP_HIP_OK)
+        return s;
     for (int i = 0; i < 3; ++i)
       if ((s = resolve(h, "bwpp_attn_bf16_d" + std::to_string(32 * (i + 1)) + cs, &h->attn_bf16_small[i][causal])) !=
           BWPP_HIP_OK)
@@ -615,6 +623,7 @@ BwppHipStatus bwpp_hip_create(BwppHip **out, int device, const char *code_object
     }
   }
   if (const char *sk = getenv("BWPP_GEMM_SPLITK")) h->gemm_splitk = atoi(sk) != 0 ? 1u : 0u;
+  if (const char *dc = getenv("BWPP_ATTN_DEC")) h->attn_dec = atoi(dc) != 0 ? 1u : 0u;
   if (const char *zz = getenv("BWPP_ATTN_ZIGZAG")) h->attn_zigzag = atoi(zz) != 0 ? 1u : 0u;
   if (const char *fp = getenv("BWPP_GEMM_F32_PIPE")) h->gemm_f32_pipe = (uint32_t)std::min(std::max(atoi(fp), 0), 3);
   if (const char *w8 = getenv("BWPP_ATTN_BWD_W8")) h->attn_w8_mask = (uint32_t)strtoul(w8, nullptr, 10) & 3u;
@@ -1381,6 +1390,25 @@ int attn_bf16_bwd_variant(const BwppAttentionParams &p, const BwppAttnArgs &g, f
 
 constexpr uint32_t kAttnWaves = 4;  // waves (32 rows each) per block of the MFMA attention kernels
 
+// Few queries: `slices` slices of N keys over blocks of one per CU (their
+// LDS rings fill it).  The number of key ranges that leaves the fewest keys
+// to the busiest CU, each at least 512 keys; a split costs a combine launch
+// and its partials, about the time of 256 keys on a CU.
+void dec_ranges(const BwppHip *h, uint64_t slices, uint32_t N, uint32_t &S, uint32_t &chunk) {
+  const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
+  uint64_t best = ~0ull;
+  for (uint32_t want = 1; want <= 64 && (want == 1 || N / want >= 512); ++want) {
+    const uint32_t c = (uint32_t)((((uint64_t)N + want - 1) / want + 31) / 32 * 32);
+    const uint32_t s = (uint32_t)(((uint64_t)N + c - 1) / c);
+    const uint64_t cost = (slices * s + cus - 1) / cus * c + (s > 1 ? 256 : 0);
+    if (cost < best) {
+      best = cost;
+      S = s;
+      chunk = c;
+    }
+  }
+}
+
 BwppHipStatus attn_forward(BwppHip *h, const void *q, const void *k, const void *v, void *o, float *lse,
                            const BwppAttentionParams &p) {
   BwppHipStatus s = enter(h);
@@ -1403,6 +1431,29 @@ BwppHipStatus attn_forward(BwppHip *h, const void *q, const void *k, const void 
                     // K / V byte offsets inside a slice are 32-bit in the kernels
                     (uint64_t)(p.N - 1) * g.ldk + p.K < (1ull << 31) &&
                     (uint64_t)(p.N - 1) * g.ldv + p.D < (1ull << 31);
+  // At most 32 queries, which are one wave's: the waves split the keys.  Up
+  // to 128 keys at d = 64 many slices per CU suit the smaller blocks better
+  // (B16 H32 M1 N100: 6.6 us against 7.0).
+  if (mfma && p.M <= 32 && (p.K == 128 || (p.K == 64 && (p.N > 128 || slices <= (uint64_t)h->cus))) && h->attn_dec &&
+      slices <= 0x7fffffffull) {
+    g.scale = scale;
+    g.scale_log2 = scale * 1.4426950408889634f;
+    g.lse = lse;
+    dec_ranges(h, slices, p.N, g.ksplit, g.kchunk);
+    if (slices * g.ksplit > 0x7fffffffull) g.ksplit = 1;
+    if (g.ksplit > 1) {
+      const uint64_t rows = slices * g.ksplit * p.M;
+      g.part_o = static_cast<float *>(split_scratch(h, (size_t)(rows * (p.D + 2) * 4)));
+      g.part_ml = g.part_o + rows * p.D;
+      if (!g.part_o) g.ksplit = 1;
+    }
+    if (g.ksplit == 1) g.kchunk = (p.N + 31) / 32 * 32;
+    g.items = (uint32_t)slices;
+    s = launch(h, h->attn_bf16_dec[p.K / 64 - 1][causal], (uint32_t)(slices * g.ksplit), 1, 1, 256, g);
+    if (s != BWPP_HIP_OK || g.ksplit == 1) return s;
+    const uint64_t vecs = slices * p.M * (p.D / 4);
+    return launch(h, h->attn_dec_combine[1], (uint32_t)std::min<uint64_t>((vecs + 255) / 256, 2048), 1, 1, 256, g);
+  }
   if (mfma && p.K < 128) {
     g.scale = scale;
     g.scale_log2 = scale * 1.4426950408889634f;

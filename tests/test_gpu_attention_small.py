@@ -43,7 +43,7 @@ def _forward(be, q, k, v, scale, causal, pad=0):
 
 
 @pytest.mark.parametrize("D", [32, 64, 96])
-@pytest.mark.parametrize("B,H,M,N,pad", [(1, 1, 1, 1, 0), (2, 4, 128, 64, 0), (1, 3, 127, 129, 8), (1, 2, 129, 65, 0),
+@pytest.mark.parametrize("B,H,M,N,pad", [(1, 1, 33, 1, 0), (2, 4, 128, 64, 0), (1, 3, 127, 129, 8), (1, 2, 129, 65, 0),
                                          (2, 1, 33, 1000, 16), (1, 1, 513, 200, 0), (1, 2, 300, 300, 0)])
 @pytest.mark.parametrize("causal", [False, True])
 def test_small_head_dims(be, oracle, D, B, H, M, N, pad, causal):
