@@ -92,7 +92,8 @@ typedef struct {
    * query count rounded up to 128. */
   void *dst;
   uint32_t ld_dst;
-  uint32_t items; /* persistent flash forward: (slice, query tile) items */
+  uint32_t items; /* persistent flash forward: (slice, query tile) items;
+                     few queries: slices; generic path: rows per block */
   /* Few queries (decoding): the keys of a slice in ksplit ranges of kchunk;
    * with ksplit > 1, range s of slice b leaves its sums of p v
    * ([M][vdim]) at part_o + (b ksplit + s) M vdim and per query the pair

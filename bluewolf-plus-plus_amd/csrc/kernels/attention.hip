@@ -66,6 +66,11 @@ __device__ __forceinline__ void split_bf16x8(const f32x16_t *s, int r0, bf16x8_t
   lo = __builtin_bit_cast(bf16x8_t, make_uint4(l[0], l[1], l[2], l[3]));
 }
 
+// m ln 2 + ln l, ln 2 in two terms (its rounding would show in the last bit).
+__device__ __forceinline__ float lse_of(float m, float l) {
+  return __builtin_fmaf(m, 0.693147182f, __builtin_fmaf(m, -1.90465421e-9f, logf(l)));
+}
+
 // Running maximum of |v| as bit patterns, two bf16 lanes at a time (0x7f80
 // and above: infinity or NaN).
 __device__ __forceinline__ u16x2_t max_abs_bf16(u16x2_t m, v8s_t v) {
@@ -858,9 +863,9 @@ __device__ __forceinline__ void attn_bf16_d128(const BwppAttnArgs &a) {
 // bwpp_cpu_ref.c:110-113) with an online max/sum over chunks of 64 keys.
 // A wave processes one query at a time: lanes split the keys for the
 // scores (one key per lane per chunk), the probabilities go through LDS,
-// and lanes split d for the weighted sum of V.  4 waves per block, 16
-// queries per block.
-constexpr int kGenQ = 16;
+// and lanes split d for the weighted sum of V.  4 waves per block, a.items
+// rows (queries, or keys in the dK / dV pass) per block: 16, or one per wave
+// where 16 would leave CUs idle.
 constexpr int kGenMaxDim = 512;
 
 template <class T>
@@ -876,6 +881,51 @@ __device__ __forceinline__ void st_elem(T *p, float v) {
     *reinterpret_cast<uint16_t *>(p) = f32_to_bf16_bits(v);
   else
     *p = v;
+}
+
+// acc + sum over k of q[k] * row[k], in k order.  The row comes in 16-byte
+// loads (at any address), several in flight: element loads, one row per lane,
+// were what bound these kernels (forward and backward of B2 H16 S58 d96
+// bf16 271 -> 29 us, of fp32 B3 H4 S127 d96 963 -> 91, of bf16 B1 H4 S800 d96
+// 5616 -> 235; the same bits).
+template <class T>
+__device__ __forceinline__ float dot_row(const float *q, const T *row, uint32_t n, float acc) {
+  constexpr uint32_t W = 16 / sizeof(T);
+  typedef T vec_t __attribute__((ext_vector_type(W), aligned(sizeof(T))));
+  uint32_t k = 0;
+#pragma unroll 4
+  for (; k + W <= n; k += W) {
+    const vec_t v = *reinterpret_cast<const vec_t *>(row + k);
+#pragma unroll
+    for (uint32_t e = 0; e < W; ++e) {
+      const T x = v[e];
+      acc += q[k + e] * ld_elem(&x);
+    }
+  }
+  for (; k < n; ++k) acc += q[k] * ld_elem(row + k);
+  return acc;
+}
+
+// acc[j] += w[t] * row t's element 64 j + lane, rows in order t = 0 .. cnt -
+// 1, eight rows' loads in flight.
+template <class T, int DPL>
+__device__ __forceinline__ void axpy_rows(float (&acc)[DPL], const float *w, const T *rows, uint32_t ld, uint32_t cnt,
+                                          uint32_t n, int lane) {
+#pragma unroll
+  for (int j = 0; j < DPL; ++j) {
+    const uint32_t d = (uint32_t)lane + 64u * j;
+    if (64u * j >= n) break;  // uniform
+    if (d >= n) continue;
+    uint32_t t = 0;
+    for (; t + 8 <= cnt; t += 8) {
+      T x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = rows[(size_t)(t + i) * ld + d];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[j] += w[t + i] * ld_elem(&x[i]);
+    }
+    for (; t < cnt; ++t) acc[j] += w[t] * ld_elem(rows + (size_t)t * ld + d);
+  }
 }
 
 // One query by one wave.  qs: [>= kdim] floats, ps: [64] floats of LDS of
@@ -907,10 +957,7 @@ __device__ __forceinline__ void attn_generic_query(const BwppAttnArgs &a, uint32
     const uint32_t n = n0 + (uint32_t)lane;
     float s = -INFINITY;
     if (n < kend) {
-      const T *kr = K + (size_t)n * a.ldk;
-      float acc = 0.0f;
-      for (uint32_t k = 0; k < Kd; ++k) acc += qs[k] * ld_elem(kr + k);
-      s = acc * scale;
+      s = dot_row(qs, K + (size_t)n * a.ldk, Kd, 0.0f) * scale;
     }
     const float cm = wave_max(s);
     const float mnew = fmaxf(m, cm);
@@ -927,15 +974,7 @@ __device__ __forceinline__ void attn_generic_query(const BwppAttnArgs &a, uint32
     const uint32_t cnt = min(64u, kend - n0);
 #pragma unroll
     for (int j = 0; j < DPL; ++j) o[j] *= alpha;
-    for (uint32_t t = 0; t < cnt; ++t) {
-      const float pn = ps[t];
-      const T *vr = V + (size_t)(n0 + t) * a.ldv;
-#pragma unroll
-      for (int j = 0; j < DPL; ++j) {
-        const uint32_t d = (uint32_t)lane + 64u * j;
-        if (d < Dv) o[j] += pn * ld_elem(vr + d);
-      }
-    }
+    axpy_rows<T, DPL>(o, ps, V + (size_t)n0 * a.ldv, a.ldv, cnt, Dv, lane);
     __builtin_amdgcn_wave_barrier();
   }
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
@@ -956,8 +995,8 @@ __device__ __forceinline__ void attn_generic(const BwppAttnArgs &a) {
   const uint32_t nbh = gridDim.x / a.q_tiles;
   const uint32_t qt = a.q_tiles - 1 - blockIdx.x / nbh;
   const uint32_t bh = blockIdx.x % nbh;
-  for (uint32_t qq = (uint32_t)wave; qq < kGenQ; qq += kWaves) {
-    const uint32_t qi = qt * kGenQ + qq;
+  for (uint32_t qq = (uint32_t)wave; qq < a.items; qq += kWaves) {
+    const uint32_t qi = qt * a.items + qq;
     if (qi >= a.M) break;  // wave-uniform
     attn_generic_query<T, CAUSAL, kGenMaxDim / 64>(a, bh, qi, a.scale_log2 /* the plain scale on this path */, qs[wave],
                                                   ps[wave]);
@@ -1223,7 +1262,7 @@ __device__ __forceinline__ void attn_bf16_small(const BwppAttnArgs &a) {
   if (redo) return;
   if (a.lse && lh == 0 && qi < a.M)
     a.lse[(size_t)bh * a.M + qi] =
-        lrow > 0.0f ? __builtin_fmaf(mrow == -INFINITY ? 0.0f : mrow, 0.69314718055994531f, logf(lrow)) : -INFINITY;
+        lrow > 0.0f ? lse_of(mrow == -INFINITY ? 0.0f : mrow, lrow) : -INFINITY;
   uint16_t *os = reinterpret_cast<uint16_t *>(smem) + (size_t)wave * kQW * (T::kRowB / 2);
   const float inv = lrow > 0.0f ? 1.0f / lrow : 0.0f;
 #pragma unroll
@@ -1504,7 +1543,7 @@ __device__ __forceinline__ void attn_bf16_dec(const BwppAttnArgs &a) {
         make_uint2(pack_bf16x2(t.x * inv, t.y * inv), pack_bf16x2(t.z * inv, t.w * inv));
     if (a.lse && d4 == 0)
       a.lse[(size_t)bh * a.M + q] =
-          l > 0.0f ? __builtin_fmaf(m == -INFINITY ? 0.0f : m, 0.69314718055994531f, logf(l)) : -INFINITY;
+          l > 0.0f ? lse_of(m == -INFINITY ? 0.0f : m, l) : -INFINITY;
   }
 }
 
@@ -1535,7 +1574,7 @@ __device__ __forceinline__ void attn_dec_combine(const BwppAttnArgs &a, uint32_t
     st_elem(O, t.x * inv), st_elem(O + 1, t.y * inv), st_elem(O + 2, t.z * inv), st_elem(O + 3, t.w * inv);
     if (a.lse && d4 == 0)
       a.lse[(size_t)bh * a.M + q] =
-          l > 0.0f ? __builtin_fmaf(m == -INFINITY ? 0.0f : m, 0.69314718055994531f, logf(l)) : -INFINITY;
+          l > 0.0f ? lse_of(m == -INFINITY ? 0.0f : m, l) : -INFINITY;
   }
 }
 
@@ -1569,8 +1608,8 @@ __device__ __forceinline__ void attn_bwd_dq(const BwppAttnArgs &a) {
   const float scale = a.scale_log2;  // the plain scale on this path
   constexpr int DPL = kGenMaxDim / 64;
 
-  for (uint32_t qq = (uint32_t)wave; qq < kGenQ; qq += kWaves) {
-    const uint32_t qi = qt * kGenQ + qq;
+  for (uint32_t qq = (uint32_t)wave; qq < a.items; qq += kWaves) {
+    const uint32_t qi = qt * a.items + qq;
     if (qi >= a.M) break;  // wave-uniform
     for (uint32_t k = (uint32_t)lane; k < Kd; k += 64) qs[wave][k] = ld_elem(Q + (size_t)qi * a.ldq + k);
     float dsum = 0.0f;
@@ -1595,11 +1634,8 @@ __device__ __forceinline__ void attn_bwd_dq(const BwppAttnArgs &a) {
       const uint32_t n = n0 + (uint32_t)lane;
       float ds = 0.0f;
       if (n < kend) {
-        const T *kr = K + (size_t)n * a.ldk;
-        const T *vr = V + (size_t)n * a.ldv;
-        float s = 0.0f, dp = 0.0f;
-        for (uint32_t k = 0; k < Kd; ++k) s += qs[wave][k] * ld_elem(kr + k);
-        for (uint32_t d = 0; d < Dv; ++d) dp += gs[wave][d] * ld_elem(vr + d);
+        const float s = dot_row(qs[wave], K + (size_t)n * a.ldk, Kd, 0.0f);
+        const float dp = dot_row(gs[wave], V + (size_t)n * a.ldv, Dv, 0.0f);
         const float p = expf(s * scale - lse);
         ds = p * (dp - dsum);
       }
@@ -1609,15 +1645,7 @@ __device__ __forceinline__ void attn_bwd_dq(const BwppAttnArgs &a) {
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       const uint32_t cnt = min(64u, kend - n0);
-      for (uint32_t t = 0; t < cnt; ++t) {
-        const float dsn = ps[wave][t];
-        const T *kr = K + (size_t)(n0 + t) * a.ldk;
-#pragma unroll
-        for (int j = 0; j < DPL; ++j) {
-          const uint32_t k = (uint32_t)lane + 64u * j;
-          if (k < Kd) acc[j] += dsn * ld_elem(kr + k);
-        }
-      }
+      axpy_rows<T, DPL>(acc, ps[wave], K + (size_t)n0 * a.ldk, a.ldk, cnt, Kd, lane);
       __builtin_amdgcn_wave_barrier();
     }
 #pragma unroll
@@ -1653,8 +1681,8 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwppAttnArgs &a) {
   const float scale = a.scale_log2;
   constexpr int DPL = kGenMaxDim / 64;
 
-  for (uint32_t kk = (uint32_t)wave; kk < kGenQ; kk += kWaves) {
-    const uint32_t n = kt * kGenQ + kk;
+  for (uint32_t kk = (uint32_t)wave; kk < a.items; kk += kWaves) {
+    const uint32_t n = kt * a.items + kk;
     if (n >= a.N) break;  // wave-uniform
     for (uint32_t k = (uint32_t)lane; k < Kd; k += 64) ks[wave][k] = ld_elem(K + (size_t)n * a.ldk + k);
     for (uint32_t d = (uint32_t)lane; d < Dv; d += 64) vs[wave][d] = ld_elem(V + (size_t)n * a.ldv + d);
@@ -1672,11 +1700,8 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwppAttnArgs &a) {
       const uint32_t m = m0 + (uint32_t)lane;
       float p = 0.0f, ds = 0.0f;
       if (m < a.M) {
-        const T *qr = Q + (size_t)m * a.ldq;
-        const T *gr = dO + (size_t)m * a.ldo;
-        float s = 0.0f, dp = 0.0f;
-        for (uint32_t k = 0; k < Kd; ++k) s += ld_elem(qr + k) * ks[wave][k];
-        for (uint32_t d = 0; d < Dv; ++d) dp += ld_elem(gr + d) * vs[wave][d];
+        const float s = dot_row(ks[wave], Q + (size_t)m * a.ldq, Kd, 0.0f);
+        const float dp = dot_row(vs[wave], dO + (size_t)m * a.ldo, Dv, 0.0f);
         p = expf(s * scale - lse[m]);
         ds = p * (dp - dsum[m]);
       }
@@ -1687,17 +1712,8 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwppAttnArgs &a) {
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       const uint32_t cnt = min(64u, a.M - m0);
-      for (uint32_t t = 0; t < cnt; ++t) {
-        const float pm = pp[wave][t], dm = dd[wave][t];
-        const T *qr = Q + (size_t)(m0 + t) * a.ldq;
-        const T *gr = dO + (size_t)(m0 + t) * a.ldo;
-#pragma unroll
-        for (int j = 0; j < DPL; ++j) {
-          const uint32_t c = (uint32_t)lane + 64u * j;
-          if (c < Kd) gk[j] += dm * ld_elem(qr + c);
-          if (c < Dv) gv[j] += pm * ld_elem(gr + c);
-        }
-      }
+      axpy_rows<T, DPL>(gk, dd[wave], Q + (size_t)m0 * a.ldq, a.ldq, cnt, Kd, lane);
+      axpy_rows<T, DPL>(gv, pp[wave], dO + (size_t)m0 * a.ldo, a.ldo, cnt, Dv, lane);
       __builtin_amdgcn_wave_barrier();
     }
 #pragma unroll

@@ -91,21 +91,21 @@ __device__ __forceinline__ void wave_argmax(float &v, uint32_t &i) {
 
 // 128-bit global accesses at any 4-byte address (what the hardware asks of
 // a dwordx4), non-temporal for data streamed exactly once.
-typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x4a __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ float4 load_nt4(const float *p) {
-  const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(p));
+  const f32x4a t = __builtin_nontemporal_load(reinterpret_cast<const f32x4a *>(p));
   return make_float4(t.x, t.y, t.z, t.w);
 }
 __device__ __forceinline__ void store_nt4(float *p, const float4 &o) {
-  const f32x4 t = {o.x, o.y, o.z, o.w};
-  __builtin_nontemporal_store(t, reinterpret_cast<f32x4 *>(p));
+  const f32x4a t = {o.x, o.y, o.z, o.w};
+  __builtin_nontemporal_store(t, reinterpret_cast<f32x4a *>(p));
 }
 __device__ __forceinline__ void store4(float *p, const float4 &o) {
-  const f32x4 t = {o.x, o.y, o.z, o.w};
-  *reinterpret_cast<f32x4 *>(p) = t;
+  const f32x4a t = {o.x, o.y, o.z, o.w};
+  *reinterpret_cast<f32x4a *>(p) = t;
 }
 __device__ __forceinline__ float4 load4(const float *p) {
-  const f32x4 t = *reinterpret_cast<const f32x4 *>(p);
+  const f32x4a t = *reinterpret_cast<const f32x4a *>(p);
   return make_float4(t.x, t.y, t.z, t.w);
 }
 

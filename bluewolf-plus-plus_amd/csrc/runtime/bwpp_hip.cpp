@@ -1390,6 +1390,13 @@ int attn_bf16_bwd_variant(const BwppAttentionParams &p, const BwppAttnArgs &g, f
 
 constexpr uint32_t kAttnWaves = 4;  // waves (32 rows each) per block of the MFMA attention kernels
 
+// Rows per block of the generic attention kernels: 16 (four a wave), or one
+// a wave until there are eight blocks per CU.
+uint32_t generic_rows(const BwppHip *h, uint64_t slices, uint32_t rows) {
+  const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
+  return slices * (((uint64_t)rows + 15) / 16) >= 8 * cus ? 16u : 4u;
+}
+
 // Few queries: `slices` slices of N keys over blocks of one per CU (their
 // LDS rings fill it).  The number of key ranges that leaves the fewest keys
 // to the busiest CU, each at least 512 keys; a split costs a combine launch
@@ -1490,7 +1497,8 @@ BwppHipStatus attn_forward(BwppHip *h, const void *q, const void *k, const void 
   }
   g.scale_log2 = scale;
   g.lse = lse;
-  g.q_tiles = (p.M + 15) / 16;
+  g.items = generic_rows(h, slices, p.M);
+  g.q_tiles = (uint32_t)(((uint64_t)p.M + g.items - 1) / g.items);
   const uint64_t grid = slices * g.q_tiles;
   if (grid > 0x7fffffffull) return fail(h, BWPP_HIP_ERR_UNSUPPORTED, "attention: grid too large");
   return launch(h, h->attn_generic[bf16 ? 1 : 0][causal], (uint32_t)grid, 1, 1, 256, g);
@@ -1752,13 +1760,15 @@ BwppHipStatus attn_grad_impl(BwppHip *h, const void *q, const void *k, const voi
     return conv(dv32, dv, p.N, g.ldv, g.v_bs, g.v_hs, true);
   }
   if (p.M > 0) {
-    g.q_tiles = (p.M + 15) / 16;
+    g.items = generic_rows(h, slices, p.M);
+    g.q_tiles = (uint32_t)(((uint64_t)p.M + g.items - 1) / g.items);
     const uint64_t grid = slices * g.q_tiles;
     if (grid > 0x7fffffffull) return fail(h, BWPP_HIP_ERR_UNSUPPORTED, "attention_grad: grid too large");
     if ((s = launch(h, h->attn_bwd_dq[bf][causal], (uint32_t)grid, 1, 1, 256, g)) != BWPP_HIP_OK) return s;
   }
   if (p.N > 0) {
-    g.q_tiles = (p.N + 15) / 16;  // key tiles
+    g.items = generic_rows(h, slices, p.N);
+    g.q_tiles = (uint32_t)(((uint64_t)p.N + g.items - 1) / g.items);  // key tiles
     const uint64_t grid = slices * g.q_tiles;
     if (grid > 0x7fffffffull) return fail(h, BWPP_HIP_ERR_UNSUPPORTED, "attention_grad: grid too large");
     if ((s = launch(h, h->attn_bwd_dkdv[bf][causal], (uint32_t)grid, 1, 1, 256, g)) != BWPP_HIP_OK) return s;
