@@ -1771,6 +1771,9 @@ BWPP_ATTN_DEC(128)
 extern "C" __global__ __launch_bounds__(256) void bwpp_attn_dec_combine_bf16(const BwppAttnArgs a) {
   attn_dec_combine<uint16_t>(a, a.items);
 }
+extern "C" __global__ __launch_bounds__(256) void bwpp_attn_dec_combine_f32(const BwppAttnArgs a) {
+  attn_dec_combine<float>(a, a.items);
+}
 
 // Generic path entry points, one per storage type x mask.
 #define BWPP_ATTN_GENERIC(NAME, T, CAUSAL)                                                  \

@@ -280,6 +280,141 @@ __device__ __forceinline__ void attn_fwd(const BwppAttnArgs &a) {
   }
 }
 
+// --------------------------------------------- forward, at most 32 queries
+// Decoding: a few queries against a long cache, bound by reading K and V
+// once.  A block of 4 waves owns one slice and a range of its keys (ksplit
+// ranges of kchunk); every wave holds all the queries and takes every fourth
+// 32-key tile of the range, its operands straight from memory in the MFMA
+// layouts: a lane's K operand is half a row (16-byte loads), its V operand
+// one column of a key pair (128 contiguous bytes per half-wave).  No LDS and
+// no barrier until the end: V is in flight during the scores and the next
+// tile's K during the second product.  The waves' (maximum, sum, O) triples
+// meet in LDS, those of a split slice in bwpp_attn_dec_combine_f32.  B4 H8 M1
+// N8000 d128: 32 blocks with three of four waves idle 1105 us, this 50
+// us (262 MB at 5.3 TB/s; B8 H32 N4095 619 -> 181).
+template <int D, bool CAUSAL>
+__device__ __forceinline__ void attn_dec(const BwppAttnArgs &a) {
+  constexpr int ST = D + 4;
+  __shared__ __attribute__((aligned(16))) float os[kW][32][ST];
+  __shared__ float ml[kW][32][2];
+  const int lane = (int)threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int li = lane & 31, hi = lane >> 5;
+  const uint32_t bh = blockIdx.x / a.ksplit, sp = blockIdx.x % a.ksplit;
+  const uint32_t b = bh / a.heads, h = bh % a.heads;
+  const float *Q = static_cast<const float *>(a.q) + b * a.q_bs + h * a.q_hs;
+  const float *K = static_cast<const float *>(a.k) + b * a.k_bs + h * a.k_hs;
+  const float *V = static_cast<const float *>(a.v) + b * a.v_bs + h * a.v_hs;
+  const int64_t diag = (int64_t)a.N - (int64_t)a.M;
+  const uint32_t kbeg = sp * a.kchunk, kend = min(a.N, kbeg + a.kchunk);
+  const uint32_t ntile = kbeg < kend ? (kend - kbeg + kR - 1) / kR : 0u;
+  const uint32_t nmine = ntile > (uint32_t)wave ? (ntile - (uint32_t)wave + kW - 1) / kW : 0u;
+
+  float qreg[D / 2], kreg[D / 2];
+  load_half_row<D>(qreg, Q, a.ldq, (uint32_t)li, a.M, hi);
+  f32x16 o[D / 32];
+#pragma unroll
+  for (int blk = 0; blk < D / 32; ++blk) o[blk] = f32x16{};
+  float mrun = -INFINITY, lsum = 0.0f;
+  const float c = a.scale_log2;
+  auto tile_key = [&](uint32_t j) { return kbeg + kR * (kW * j + (uint32_t)wave); };
+  // Rows past the cache re-read its last one (masked below).
+  auto load_k = [&](uint32_t j) {
+    const uint32_t row = min(tile_key(j) + (uint32_t)li, a.N - 1u);
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(K + (size_t)row * a.ldk + hi * (D / 2));
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) {
+      const f32x4 v = src[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) kreg[4 * i + e] = v[e];
+    }
+  };
+  if (nmine > 0) load_k(0);
+  for (uint32_t j = 0; j < nmine; ++j) {
+    const uint32_t k0 = tile_key(j);
+    float v[16][D / 32];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float *src = V + (size_t)min(k0 + (uint32_t)acc_row(r, hi), a.N - 1u) * a.ldv + li;
+#pragma unroll
+      for (int blk = 0; blk < D / 32; ++blk) v[r][blk] = src[32 * blk];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // V's loads ahead of the scores
+    f32x16 s = {};
+#pragma unroll
+    for (int i = 0; i < D / 2; ++i) s = mfma(kreg[i], qreg[i], s);
+    __builtin_amdgcn_sched_barrier(0);
+    if (j + 1 < nmine) load_k(j + 1);
+    __builtin_amdgcn_sched_barrier(0);  // the next K's ahead of the softmax and the second product
+#pragma unroll
+    for (int r = 0; r < 16; ++r) s[r] *= c;
+    if (k0 + kR > kend || (CAUSAL && (int64_t)k0 + kR - 1 > diag)) {  // wave-uniform
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const uint32_t key = k0 + (uint32_t)acc_row(r, hi);
+        if (key >= kend || (CAUSAL && (int64_t)key > (int64_t)li + diag)) s[r] = -INFINITY;
+#pragma unroll
+        for (int blk = 0; blk < D / 32; ++blk) v[r][blk] = key < kend ? v[r][blk] : 0.0f;
+      }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    mx = max32(mx);
+    const float mnew = fmaxf(mrun, mx);
+    const float mu = mnew == -INFINITY ? 0.0f : mnew;
+    const float alpha = __builtin_amdgcn_exp2f(mrun - mu);
+    float ps = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = __builtin_amdgcn_exp2f(s[r] - mu);
+      ps += s[r];
+    }
+    lsum = lsum * alpha + ps;
+    mrun = mnew;
+#pragma unroll
+    for (int blk = 0; blk < D / 32; ++blk) o[blk] *= alpha;
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+#pragma unroll
+      for (int blk = 0; blk < D / 32; ++blk) o[blk] = mfma(v[r][blk], s[r], o[blk]);
+  }
+  const float ltot = sum32(lsum);
+  store_t<D>(&os[wave][0][0], ST, (uint32_t)li, o, 1.0f, hi);
+  if (hi == 0) {
+    ml[wave][li][0] = mrun;
+    ml[wave][li][1] = ltot;
+  }
+  __syncthreads();
+  float *O = static_cast<float *>(a.o) + b * a.o_bs + h * a.o_hs;
+  for (uint32_t i = threadIdx.x; i < a.M * (D / 4); i += 64 * kW) {
+    const uint32_t q = i / (D / 4), d4 = 4u * (i % (D / 4));
+    float m = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kW; ++w) m = fmaxf(m, ml[w][q][0]);
+    float l = 0.0f;
+    f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < kW; ++w) {
+      const float mw = ml[w][q][0];
+      const float f = mw == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(mw - m);  // no key seen: sums of 0 (or NaN, kept)
+      l += ml[w][q][1] * f;
+      t += *reinterpret_cast<const f32x4 *>(&os[w][q][d4]) * f;
+    }
+    if (a.ksplit > 1) {
+      const size_t row = (size_t)blockIdx.x * a.M + q;
+      *reinterpret_cast<f32x4 *>(a.part_o + row * D + d4) = t;
+      if (d4 == 0) {
+        a.part_ml[2 * row] = m;
+        a.part_ml[2 * row + 1] = l;
+      }
+      continue;
+    }
+    *reinterpret_cast<f32x4 *>(O + (size_t)q * a.ldo + d4) = t * (l > 0.0f ? 1.0f / l : 0.0f);
+    if (a.lse && d4 == 0) a.lse[(size_t)bh * a.M + q] = l > 0.0f ? (m + log2f(l)) * kLn2 : -INFINITY;
+  }
+}
+
 // ---------------------------------------------------------------- backward
 // D_m = rowsum(dO * O) of query row qi (greg: the lane's half of dO's row):
 // each lane half sums its D / 2 products in order, then the halves add.
@@ -634,6 +769,20 @@ __device__ __forceinline__ void attn_bwd_dkdv(const BwppAttnArgs &a) {
 }
 
 }  // namespace
+
+#define BWPP_ATTN_F32_DEC(D)                                                                         \
+  extern "C" __global__ __attribute__((amdgpu_flat_work_group_size(256, 256),                        \
+                                       amdgpu_waves_per_eu(1, 1))) void                              \
+      bwpp_attn_f32_dec_d##D(const BwppAttnArgs a) {                                                 \
+    attn_dec<D, false>(a);                                                                           \
+  }                                                                                                  \
+  extern "C" __global__ __attribute__((amdgpu_flat_work_group_size(256, 256),                        \
+                                       amdgpu_waves_per_eu(1, 1))) void                              \
+      bwpp_attn_f32_dec_d##D##_causal(const BwppAttnArgs a) {                                        \
+    attn_dec<D, true>(a);                                                                            \
+  }
+BWPP_ATTN_F32_DEC(64)
+BWPP_ATTN_F32_DEC(128)
 
 #define BWPP_ATTN_F32(D, CAUSAL, SUFFIX)                                                                    \
   extern "C" __global__ __launch_bounds__(64 * kW) void bwpp_attn_f32_mfma_d##D##SUFFIX(const BwppAttnArgs a) { \

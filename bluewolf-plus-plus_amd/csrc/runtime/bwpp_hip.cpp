@@ -112,7 +112,7 @@ struct BwppHip {
   hipFunction_t attn_flash[2] = {};       // bf16, d = 128: [causal]
   hipFunction_t attn_flash_p[2] = {};     // bf16, d = 128, persistent (one block per CU): [causal]
   hipFunction_t attn_bf16_small[3][2] = {};  // bf16, d = 32 / 64 / 96: [d / 32 - 1][causal]
-  hipFunction_t attn_bf16_dec[2][2] = {};    // bf16, at most 32 queries, d = 64 / 128: [d128][causal]
+  hipFunction_t attn_dec_k[2][2][2] = {};    // at most 32 queries, d = 64 / 128: [bf16][d128][causal]
   hipFunction_t attn_dec_combine[2] = {};    // [bf16]
   uint32_t attn_dec = 1;                     // BWPP_ATTN_DEC=0: off
   // BWPP_ATTN_FLASH_PERSIST: bit c set = persistent kernel when causal == c
@@ -289,6 +289,7 @@ BwppHipStatus resolve_all(BwppHip *h) {
       {"bwpp_silu_grad", &h->silu_grad},             {"bwpp_softmax_grad", &h->softmax_grad},
       {"bwpp_gemm_bf16_splitk_reduce", &h->gemm_bf16_reduce},
       {"bwpp_attn_dec_combine_bf16", &h->attn_dec_combine[1]},
+      {"bwpp_attn_dec_combine_f32", &h->attn_dec_combine[0]},
       {"bwpp_rmsnorm_grad", &h->rmsnorm_grad},       {"bwpp_col_partials_sum", &h->col_partials_sum},
       {"bwpp_reduce_sum_rows", &h->reduce_sum_rows}, {"bwpp_reduce_sum_cols", &h->reduce_sum_cols},
       {"bwpp_mean_square_part", &h->mean_square_part}, {"bwpp_mean_square_final", &h->mean_square_final},
@@ -371,9 +372,9 @@ BwppHipStatus resolve_all(BwppHip *h) {
       return s;
     if ((s = resolve(h, std::string("bwpp_attn_generic_bf16") + cs, &h->attn_generic[1][causal])) != BWPP_HIP_OK)
       return s;
-    for (int d128 = 0; d128 < 2; ++d128)
-      if ((s = resolve(h, std::string("bwpp_attn_bf16_dec_d") + (d128 ? "128" : "64") + cs,
-                       &h->attn_bf16_dec[d128][causal])) != BWPP_HIP_OK)
+    for (int i = 0; i < 4; ++i)
+      if ((s = resolve(h, std::string(i / 2 ? "bwpp_attn_bf16_dec_d" : "bwpp_attn_f32_dec_d") + (i % 2 ? "128" : "64") + cs,
+                       &h->attn_dec_k[i / 2][i % 2][causal])) != BWPP_HIP_OK)
         return s;
     for (int i = 0; i < 3; ++i)
       if ((s = resolve(h, "bwpp_attn_bf16_d" + std::to_string(32 * (i + 1)) + cs, &h->attn_bf16_small[i][causal])) !=
@@ -1439,10 +1440,11 @@ BwppHipStatus attn_forward(BwppHip *h, const void *q, const void *k, const void 
                     (uint64_t)(p.N - 1) * g.ldk + p.K < (1ull << 31) &&
                     (uint64_t)(p.N - 1) * g.ldv + p.D < (1ull << 31);
   // At most 32 queries, which are one wave's: the waves split the keys.  Up
-  // to 128 keys at d = 64 many slices per CU suit the smaller blocks better
-  // (B16 H32 M1 N100: 6.6 us against 7.0).
-  if (mfma && p.M <= 32 && (p.K == 128 || (p.K == 64 && (p.N > 128 || slices <= (uint64_t)h->cus))) && h->attn_dec &&
-      slices <= 0x7fffffffull) {
+  // to 128 bf16 keys at d = 64 many slices per CU suit the smaller blocks
+  // better (B16 H32 M1 N100: 6.6 us against 7.0).
+  const int f32v = attn_f32_variant(p, g, scale, {q, k, v, o});
+  const bool dec_bf16 = mfma && (p.K == 128 || (p.K == 64 && (p.N > 128 || slices <= (uint64_t)h->cus)));
+  if (h->attn_dec && p.M <= 32 && (dec_bf16 || (f32v >= 0 && p.N > 0)) && slices <= 0x7fffffffull) {
     g.scale = scale;
     g.scale_log2 = scale * 1.4426950408889634f;
     g.lse = lse;
@@ -1454,12 +1456,13 @@ BwppHipStatus attn_forward(BwppHip *h, const void *q, const void *k, const void 
       g.part_ml = g.part_o + rows * p.D;
       if (!g.part_o) g.ksplit = 1;
     }
-    if (g.ksplit == 1) g.kchunk = (p.N + 31) / 32 * 32;
+    if (g.ksplit == 1) g.kchunk = (uint32_t)std::min<uint64_t>(((uint64_t)p.N + 31) / 32 * 32, 0xffffffffull);
     g.items = (uint32_t)slices;
-    s = launch(h, h->attn_bf16_dec[p.K / 64 - 1][causal], (uint32_t)(slices * g.ksplit), 1, 1, 256, g);
+    s = launch(h, h->attn_dec_k[bf16 ? 1 : 0][p.K / 64 - 1][causal], (uint32_t)(slices * g.ksplit), 1, 1, 256, g);
     if (s != BWPP_HIP_OK || g.ksplit == 1) return s;
     const uint64_t vecs = slices * p.M * (p.D / 4);
-    return launch(h, h->attn_dec_combine[1], (uint32_t)std::min<uint64_t>((vecs + 255) / 256, 2048), 1, 1, 256, g);
+    return launch(h, h->attn_dec_combine[bf16 ? 1 : 0], (uint32_t)std::min<uint64_t>((vecs + 255) / 256, 2048), 1, 1,
+                  256, g);
   }
   if (mfma && p.K < 128) {
     g.scale = scale;
@@ -1484,7 +1487,6 @@ BwppHipStatus attn_forward(BwppHip *h, const void *q, const void *k, const void 
     }
     return launch(h, h->attn_flash[causal], (uint32_t)grid, 1, 1, 512, g);
   }
-  const int f32v = attn_f32_variant(p, g, scale, {q, k, v, o});
   if (f32v >= 0) {
     g.scale = scale;
     g.scale_log2 = scale * 1.4426950408889634f;

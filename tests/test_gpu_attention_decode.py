@@ -111,3 +111,42 @@ def test_caller_capture():
     finally:
         torch.cuda.synchronize()
         h.close()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,M,N,pad", [(1, 1, 1, 1, 0), (1, 2, 1, 31, 0), (2, 2, 3, 33, 4), (1, 1, 32, 32, 0),
+                                         (1, 2, 32, 100, 0), (2, 1, 17, 9, 0), (1, 1, 5, 4133, 4), (1, 300, 1, 70, 0)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_decode_f32(be, oracle, D, B, H, M, N, pad, causal):
+    """The fp32 kernel; bar 1e-5 of the largest result (sums of up to 4133
+    terms in a dozen partial sums, 2^-24 each)."""
+    import torch
+    q, k, v = (synth.normal((B, H, r, D), M + N, i) for i, r in enumerate((M, N, N)))
+    ld, scale = D + pad, D ** -0.5
+
+    def rows(t):
+        r = torch.full(t.shape[:3] + (ld,), 3.0, device="cuda")
+        r[..., :D] = torch.from_numpy(t).cuda()
+        return r
+
+    o = torch.full((B, H, M, ld), 5.0, device="cuda")
+    lse = torch.full((B, H, M), 5.0, device="cuda")
+    prm = bwpp.AttentionParams(M=M, N=N, K=D, D=D, ldq=ld, ldk=ld, ldv=ld, ldo=ld, batch=B, heads=H, scale=scale,
+                               causal=int(causal))
+    be.dispatch_attention_lse(rows(q), rows(k), rows(v), o, lse, prm)
+    torch.cuda.synchronize()
+    split = be.last_kernel == "bwpp_attn_dec_combine_f32"
+    assert be.recent_kernel(1 if split else 0) == f"bwpp_attn_f32_dec_d{D}" + ("_causal" if causal else "")
+    assert split == (N >= 1024)
+    assert bool((o[..., D:] == 5.0).all())
+    assert rel_max_err(o[..., :D].cpu().numpy(), oracle.attention_bh(q, k, v, scale, causal)) <= 1e-5
+    want, got = oracle.attention_lse(q, k, scale, causal), lse.cpu().numpy()
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isfinite(got), fin)
+    assert np.all(np.abs(got[fin] - want[fin]) <= 1e-5 * np.maximum(1.0, np.abs(want[fin])))
+    if M == 1:  # an infinity at the last key, whose row the padding re-reads
+        vi = v.copy()
+        vi[..., N - 1, 3] = np.inf
+        be.dispatch_attention(rows(q), rows(k), rows(vi), o, prm)
+        torch.cuda.synchronize()
+        assert bool(torch.isposinf(o[..., 0, 3]).all()) and bool(torch.isfinite(o[..., 0, 4:D]).all())
