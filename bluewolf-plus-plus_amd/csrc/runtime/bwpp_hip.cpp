@@ -994,24 +994,25 @@ namespace {
 // modelled time of a full-tile kernel that could run, is less (done stays
 // false, as where the operands are too small for their 16-byte chunks).
 // Per K element, n blocks on a CU take lat + (n - 1) inc us; every launch
-// costs 4 us with its prologue and epilogue, a split 3.5 us and its partial
-// planes' traffic at 7 TB/s (they stay in the Infinity Cache), and no product
-// runs faster than its operands arrive (5.6 TB/s).  Fitted on MI355X to 26
-// bf16 products from 9 x 9 x 200 to 4095 x 8191 x 2048 and 16 fp32 ones from 5
-// x 7 x 9 to 2048^3, all transposes, S = 1 .. 8; the choice is within 15 % of
-// the best of all tiles and splits on each.  M x N x K: bf16 16 x 11008 x 4096
-// 210 us on the 256 x 256 edge tile, 18.2 so; 1337 x 3000 x 1024 94 -> 17.5;
-// 512 x 1024 x 1024 25.5 (full tiles) -> 6.5; 4000^3, B transposed, 189 ->
-// 134; 4095 x 8191 x 2048, odd rows, 1085 -> 170.  fp32 256^3 10.0 (split full
+// costs 4 us with its prologue and epilogue and each further block of a CU
+// `more`, a split 3.5 us and its partial planes' traffic at 7 TB/s (they stay
+// in the Infinity Cache), and no product runs faster than its operands arrive
+// (5.6 TB/s).  Fitted on MI355X to 30 bf16 products from 9 x 9 x 200 to 4095
+// x 8191 x 2048 and 16 fp32 ones from 5 x 7 x 9 to 2048^3, all transposes, S =
+// 1 .. 8; the choice is within 15 % of the best of all tiles and splits on
+// each.  M x N x K: bf16 16 x 11008 x 4096 210 us on the 256 x 256 edge tile,
+// 18.2 so; 1337 x 3000 x 1024 94 -> 17.5; 512 x 1024 x 1024 25.5 (full tiles)
+// -> 6.5; 4000 x 4000 x 96 45.6 -> 13.9; 4000^3, B transposed, 189 -> 134;
+// 4095 x 8191 x 2048, odd rows, 1085 -> 170.  fp32 256^3 10.0 (split full
 // tiles) -> 4.9; 777 x 2043 x 1021 122 -> 52; 32 x 384 x 5823 528 -> 14.
 BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool bf16, bool ta, bool tb, double full_us, bool &done) {
   struct Cost {
-    double lat, inc;
+    double lat, inc, more;
   };
   static const Cost kBf16[2][kRingNCfg] = {  // [through registers]
-      {{0.0039, 0.0045}, {0.0046, 0.0037}, {0.0085, 0.0055}, {0.0114, 0.0085}, {0.0158, 0.0158}},
-      {{0.0085, 0.0031}, {0.0088, 0.0042}, {0.0146, 0.0060}, {0.0185, 0.0105}, {0.0275, 0.0180}}};
-  static const Cost kF32[kAnyNCfg] = {{0.0082, 0.0066}, {0.0225, 0.0210}, {0.0780, 0.0580}};
+      {{0.0039, 0.0032, 1.5}, {0.0046, 0.0031, 0.6}, {0.0085, 0.0046, 0.9}, {0.0114, 0.0074, 1.4}, {0.0158, 0.0145, 2.5}},
+      {{0.0085, 0.0021, 1.5}, {0.0088, 0.0040, 0.6}, {0.0146, 0.0056, 0.9}, {0.0185, 0.0099, 1.4}, {0.0275, 0.0165, 2.5}}};
+  static const Cost kF32[kAnyNCfg] = {{0.0082, 0.0060, 0.8}, {0.0225, 0.0205, 1.0}, {0.0780, 0.0570, 2.5}};
   constexpr uint32_t kQuantum = 128;  // K ranges in multiples of the deepest stage
   const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
   const uint32_t chunk = bf16 ? 8u : 4u, es = bf16 ? 2u : 4u;
@@ -1042,7 +1043,9 @@ BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool bf16, bool ta, bool
       if (S != want && !forced) continue;
       if (tiles * S > 0x7fffffffull || (S > 1 && (!h->gemm_splitk || plane * S > kSplitBytes))) continue;
       const double n = (double)((tiles * S + cus - 1) / cus);
-      double us = std::max(4.0 + (double)std::min(kchunk, g.K) * (costs[c].lat + (n - 1.0) * costs[c].inc), mem);
+      double us = 4.0 + (n - 1.0) * costs[c].more +
+                  (double)std::min(kchunk, g.K) * (costs[c].lat + (n - 1.0) * costs[c].inc);
+      us = std::max(us, mem);
       if (S > 1) us += 3.5 + 2.0 * (double)plane * S / 7e6;
       if (us < best_us) {
         best = c;
@@ -1119,8 +1122,10 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
   }
 
   // Full-tile kernels: bf16 256 x 256 with K in steps of 32 (pipelined),
-  // fp32 128 x 128 with K in steps of 32; anything else takes the guarded
-  // edge kernels.
+  // fp32 128 x 128 with K in steps of 32.  Other products take the kernels for
+  // any M, N and K (ring_dispatch); the guarded edge kernels are left what
+  // those cannot load (operands shorter than a 16-byte chunk) and up to K = 64
+  // the 256-row bf16 products below.
   const uint32_t BM = bf16 ? 256 : 128, BN = bf16 ? 256 : 128, BK = 32;
   const uint32_t vecw = bf16 ? 8 : 4;  // elements per 16 bytes
   const bool vec = aligned16(a) && aligned16(b) && aligned16(c) && lda % vecw == 0 && ldb % vecw == 0 &&
@@ -1163,10 +1168,12 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
   // bf16: the kernels for any M, N and K, where their model finds them faster
   // than the full tiles (0.0272 us per K and round of 256 x 256 tiles, 4096^3
   // in 115 us; 0.041 of 256 x 384), whose knobs, when set, ask for those.
-  // Below K = 128 the ring does not pay for its prologue.
+  // Up to K = 64 whole 256-row tiles keep the 256-wide kernels, the documented
+  // choice there (512 x 1000 x 64 15.6 us, 4.3 with 64 x 64 ring tiles); other
+  // row counts do not (1 x 64 x 64 33 us on the edge kernel, 4.9 so).
   const bool any = h->gemm_ring != 0 && (h->gemm_ring > 0 || (h->gemm_bn == 0 && h->gemm_waves == 8));
   bool done = false;
-  if (bf16 && any && p.K >= 128) {
+  if (bf16 && any && (p.K > 64 || p.M % BM != 0 || h->gemm_ring > 0)) {
     double full_us = 1e300;
     const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
     if (full) full_us = 4.0 + 0.0272 * p.K * (double)((tiles + cus - 1) / cus);

@@ -74,10 +74,12 @@ def test_every_tile(monkeypatch, tile, ta, tb):
 
 
 @pytest.mark.parametrize("M,N,K,tb", [(16, 1024, 2048, 0), (1, 4096, 512, 1), (300, 77, 4100, 0), (2, 5, 300, 0),
-                                      (3, 7, 1000, 1)])
+                                      (3, 7, 1000, 1), (1, 64, 64, 0), (300, 264, 8, 1), (2000, 64, 100, 0),
+                                      (33, 40, 31, 0), (255, 1000, 127, 1), (9, 13, 7, 0)])
 def test_chosen(be, M, N, K, tb):
     """The default choice, and the fewest columns (N < 8, B row-major: the
-    guarded edge kernel)."""
+    guarded edge kernel), and K from the edge kernel's 7 to less than one K
+    stage."""
     _check(be, M, N, K, 0, tb, 0, 0, 3)
 
 
