@@ -155,7 +155,8 @@ struct BwppHip {
   bool split_used = false;         // work on the current stream may use it
   hipEvent_t split_ev = nullptr;   // recorded behind the last use when the stream changed ...
   bool split_wait = false;         // ... which the next use waits for
-  bool plan_capture = false;  // bwpp_hip_plan_capture is recording this handle's launches
+  bool plan_capture = false;  // bwpp_hip_plan_capture is recording this handle's launches ...
+  bool plan_split = false;    // ... and some of them use the split scratch
   // Device address of this device's scratch array (bwpp_scratch.hip), for
   // the allocation-free entry point; NULL with scratch_why set if the
   // lookup failed.
@@ -203,14 +204,24 @@ BwppHipStatus bwpp_hip_set_error(BwppHip *h, BwppHipStatus s, const char *fmt, .
 
 const void *bwpp_hip_workspace(const BwppHip *h) { return h ? h->ws : nullptr; }
 
-void bwpp_hip_set_plan_capture(BwppHip *h, bool on) { h->plan_capture = on; }
+bool bwpp_hip_set_plan_capture(BwppHip *h, bool on) {
+  h->plan_capture = on;
+  const bool used = h->plan_split;
+  h->plan_split = false;
+  return used;
+}
 
-void bwpp_hip_split_enter(BwppHip *h) {
+bool bwpp_hip_split_enter(BwppHip *h) {
+  if (h->split_off) return false;
   if (h->split_wait) {
-    (void)hipStreamWaitEvent(h->stream, h->split_ev, 0);
+    if (hipStreamWaitEvent(h->stream, h->split_ev, 0) != hipSuccess) {  // not ordered: not now
+      (void)hipGetLastError();
+      return false;
+    }
     h->split_wait = false;
   }
   h->split_used = h->split != nullptr;
+  return true;
 }
 
 namespace {
@@ -225,7 +236,7 @@ void split_leave(BwppHip *h) {
   bool ok = hipStreamIsCapturing(h->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
   if (ok && !h->split_ev) ok = hipEventCreateWithFlags(&h->split_ev, hipEventDisableTiming) == hipSuccess;
   if (ok) ok = hipEventRecord(h->split_ev, h->stream) == hipSuccess;
-  if (!ok) {  // that use cannot be ordered from here: no further use
+  if (!ok) {  // that use cannot be ordered from here: no further use, by recorded plans either
     (void)hipGetLastError();
     h->split_off = true;
   }
@@ -420,10 +431,14 @@ constexpr size_t kSplitBytes = 64u << 20;
 // capture that the caller records itself (such a graph may be replayed on
 // any stream beside this handle's other work, which the scratch does not
 // allow; a plan's graph is replayed on the handle's stream, after one eager
-// run, which has allocated it).
+// run, which has allocated it), or a use on another stream that cannot be
+// waited for (a plan that was recorded with the scratch then runs eagerly).
 void *split_scratch(BwppHip *h, size_t bytes) {
   if (bytes > kSplitBytes || h->split_off) return nullptr;
-  if (h->plan_capture) return h->split;
+  if (h->plan_capture) {
+    h->plan_split |= h->split != nullptr;
+    return h->split;
+  }
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(h->stream, &st) != hipSuccess) {
     (void)hipGetLastError();
@@ -435,8 +450,7 @@ void *split_scratch(BwppHip *h, size_t bytes) {
     h->split = nullptr;
     h->split_off = true;
   }
-  if (h->split) bwpp_hip_split_enter(h);
-  return h->split;
+  return h->split && bwpp_hip_split_enter(h) ? h->split : nullptr;
 }
 
 inline bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }

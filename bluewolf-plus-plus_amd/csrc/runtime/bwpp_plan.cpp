@@ -124,6 +124,7 @@ struct BwppHipPlan {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   const void *graph_ws = nullptr;
+  bool graph_split = false;  // its kernels use the handle's split scratch
 };
 
 namespace {
@@ -457,7 +458,7 @@ extern "C" BwppHipStatus bwpp_hip_plan_capture(BwppHipPlan *p) {
     s = run_op(*p, op);
     if (s != BWPP_HIP_OK) break;
   }
-  bwpp_hip_set_plan_capture(p->h, false);
+  p->graph_split = bwpp_hip_set_plan_capture(p->h, false);
   hipGraph_t g = nullptr;
   e = hipStreamEndCapture(st, &g);
   if (s != BWPP_HIP_OK) {
@@ -484,7 +485,10 @@ extern "C" BwppHipStatus bwpp_hip_plan_replay(BwppHipPlan *p) {
     return perr(p, BWPP_HIP_ERR_INVALID_ARG,
                 "the handle's workspace was reallocated after capture (a larger op ran on it): capture again");
   hipStream_t st = static_cast<hipStream_t>(bwpp_hip_get_stream(p->h));
-  bwpp_hip_split_enter(p->h);
+  // A use of the scratch on another stream that cannot be waited for (that
+  // stream was being recorded when the handle left it): run the ops, which
+  // then take their paths without it.
+  if (p->graph_split && !bwpp_hip_split_enter(p->h)) return bwpp_hip_plan_run(p);
   hipError_t e = hipGraphLaunch(p->exec, st);
   if (e != hipSuccess) return perr(p, BWPP_HIP_ERR_HIP, "hipGraphLaunch: %s", hipGetErrorString(e));
   return BWPP_HIP_OK;

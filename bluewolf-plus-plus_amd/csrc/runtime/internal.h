@@ -22,13 +22,15 @@ BwppHipStatus bwpp_hip_set_error(BwppHip *h, BwppHipStatus s, const char *fmt, .
 const void *bwpp_hip_workspace(const BwppHip *h);
 
 // Tells the handle that the plan executor is recording its launches: they
-// keep the paths of an eager run (see split_scratch in bwpp_hip.cpp).
-void bwpp_hip_set_plan_capture(BwppHip *h, bool on);
+// keep the paths of an eager run (see split_scratch in bwpp_hip.cpp).  When
+// the recording ends, returns whether any of them uses the split scratch.
+bool bwpp_hip_set_plan_capture(BwppHip *h, bool on);
 
-// Work that may use the handle's split scratch is about to be queued on its
+// Work that uses the handle's split scratch is about to be queued on its
 // current stream (a replayed plan, or the handle's own launches): waits for
-// the last use on another stream.
-void bwpp_hip_split_enter(BwppHip *h);
+// the last use on another stream.  False where that use cannot be waited
+// for; the scratch must not be used then.
+bool bwpp_hip_split_enter(BwppHip *h);
 
 // Size of the device-resident scratch array of bwpp_scratch.hip, which the
 // allocation-free attention backward uses for its per-query row sums.

@@ -365,6 +365,61 @@ def test_plan_replay_after_workspace_growth():
         h.close()
 
 
+def test_plan_replay_across_streams_with_scratch():
+    """A plan whose graph uses the handle's split scratch (a bf16 product with
+    K split), replayed on other streams than the scratch's last use: the
+    stream change orders the two, and where it cannot (the old stream is being
+    recorded by the caller when the handle leaves it) replay runs the ops
+    without the scratch instead of racing on it.  Bars: the same bits from the
+    graph, the rounding of a bf16 result otherwise."""
+    import torch
+    M, K, N = 8, 4096, 512
+    h = bwpp.HipBackend(0)
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    a, b, bias = (torch.randn(sh, device="cuda", generator=gen).to(torch.bfloat16) for sh in ((M, K), (K, N), (N,)))
+    c, x = torch.zeros(M, N, device="cuda", dtype=torch.bfloat16), torch.ones(64, device="cuda")
+    prm = bwpp.MatmulParams(M, N, K, K, N, N, int(bwpp.DType.BF16), int(bwpp.Epilogue.ADD_SILU), 0, 0)
+    torch.cuda.synchronize()
+
+    def out():
+        return torch.from_numpy(synth.bf16_bits_to_f32(p.host("out", (M, N), np.uint16)))
+
+    h.set_stream(s)
+    p = plan.Plan(h, plan.load_text("matmul_add_silu", M=M, K=K, N=N))
+    try:
+        p.allocate()
+        for n, v in (("a", a), ("b", b), ("bias", bias)):
+            p.bind(n, v)
+        p.capture()
+        split = h.last_kernel
+        assert split == "bwpp_gemm_bf16_splitk_reduce"
+        p.replay()
+        want = out()
+        for st in (t, s, t):  # each use waits for the last one's stream
+            h.dispatch_matmul(a, b, c, bias, prm)
+            h.set_stream(st)
+            p.replay()
+            assert torch.equal(out(), want) and h.last_kernel == split
+        h.set_stream(s)
+        h.dispatch_matmul(a, b, c, bias, prm)
+        assert h.last_kernel == split
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            x.add_(1.0)
+            h.set_stream(t)
+        for _ in range(3):
+            p.replay()
+            assert h.last_kernel != split and h.last_kernel.startswith("bwpp_gemm_bf16r")
+            got = out()
+            assert bool(((got - want).abs() <= 2.0 ** -7 * want.abs() + 1e-3).all())
+    finally:
+        torch.cuda.synchronize()
+        p.close()
+        h.close()
+
+
 def test_plan_capture_needs_a_stream(be):
     import torch
     be.set_stream(torch.cuda.default_stream())
