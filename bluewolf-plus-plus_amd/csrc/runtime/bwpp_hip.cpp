@@ -424,6 +424,15 @@ std::string library_dir() {
   return ".";
 }
 
+// Whether the caller records the handle's stream (or nothing can be asked of
+// it): nothing may be allocated then.
+bool recording(BwppHip *h) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(h->stream, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 constexpr size_t kSplitBytes = 64u << 20;
 
 // `bytes` of the handle's split scratch, or NULL where the caller has to
@@ -439,12 +448,7 @@ void *split_scratch(BwppHip *h, size_t bytes) {
     h->plan_split |= h->split != nullptr;
     return h->split;
   }
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(h->stream, &st) != hipSuccess) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  if (st != hipStreamCaptureStatusNone) return nullptr;
+  if (recording(h)) return nullptr;
   if (!h->split && hipMalloc(&h->split, kSplitBytes) != hipSuccess) {
     (void)hipGetLastError();
     h->split = nullptr;
@@ -1002,11 +1006,20 @@ BwppHipStatus ensure_ws(BwppHip *h, size_t bytes);
 
 namespace {
 
+// Whether the handle has, or can be given, a workspace of `bytes`.
+bool ws_ready(BwppHip *h, size_t bytes) { return h->ws_bytes >= bytes || !recording(h); }
+
 // Kernels for any M, N and K (gemm.hip: gemm_bf16_ring, gemm_f32_any) for a
 // product whose operands are set in g: picks the tile and the number of K
 // ranges S with the least modelled time and launches them unless full_us, the
 // modelled time of a full-tile kernel that could run, is less (done stays
 // false, as where the operands are too small for their 16-byte chunks).
+// Without memory for the partial planes the choice is made again with S = 1
+// only, against full_us too.  The planes lie in the split scratch, or with
+// use_ws in the workspace: fp32 products whose full-tile kernels split through
+// that one, so a graph that the caller records after a warm-up call splits as
+// the eager call does (256 x 256 x 8192 in such a graph: 43 us with split full
+// tiles, 195 with the split's tile run unsplit, 22.7 so).
 // Per K element, n blocks on a CU take lat + (n - 1) inc us; every launch
 // costs 4 us with its prologue and epilogue and each further block of a CU
 // `more`, a split 3.5 us and its partial planes' traffic at 7 TB/s (they stay
@@ -1019,7 +1032,8 @@ namespace {
 // -> 6.5; 4000 x 4000 x 96 45.6 -> 13.9; 4000^3, B transposed, 189 -> 134;
 // 4095 x 8191 x 2048, odd rows, 1085 -> 170.  fp32 256^3 10.0 (split full
 // tiles) -> 4.9; 777 x 2043 x 1021 122 -> 52; 32 x 384 x 5823 528 -> 14.
-BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool bf16, bool ta, bool tb, double full_us, bool &done) {
+BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool bf16, bool ta, bool tb, double full_us, bool use_ws,
+                            bool &done) {
   struct Cost {
     double lat, inc, more;
   };
@@ -1043,34 +1057,47 @@ BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool bf16, bool ta, bool
   const int ncfg = bf16 ? kRingNCfg : kAnyNCfg;
   const uint64_t np = ((uint64_t)g.N + 3) / 4 * 4, plane = (uint64_t)g.M * np * 4;
   const double mem = 4.0 + ((double)g.M * g.K + (double)g.K * g.N + (double)g.M * g.N) * es / 5.6e6;
-  int best = -1;
-  uint32_t bestS = 1;
-  double best_us = forced ? 1e301 : full_us;
-  for (int c = 0; c < ncfg; ++c) {
-    if (forced && c != h->gemm_ring - 1) continue;
-    const RingCfg &r = cfgs[c];
-    const uint64_t tiles = (((uint64_t)g.M + r.bm - 1) / r.bm) * (((uint64_t)g.N + r.bn - 1) / r.bn);
-    for (uint32_t want = 1; want <= 16; ++want) {
-      if (forced && want != h->gemm_ring_split) continue;
-      const uint32_t kchunk = (uint32_t)((((uint64_t)g.K + want - 1) / want + kQuantum - 1) / kQuantum * kQuantum);
-      const uint32_t S = (g.K + kchunk - 1) / kchunk;
-      if (S != want && !forced) continue;
-      if (tiles * S > 0x7fffffffull || (S > 1 && (!h->gemm_splitk || plane * S > kSplitBytes))) continue;
-      const double n = (double)((tiles * S + cus - 1) / cus);
-      double us = 4.0 + (n - 1.0) * costs[c].more +
-                  (double)std::min(kchunk, g.K) * (costs[c].lat + (n - 1.0) * costs[c].inc);
-      us = std::max(us, mem);
-      if (S > 1) us += 3.5 + 2.0 * (double)plane * S / 7e6;
-      if (us < best_us) {
-        best = c;
-        bestS = S;
-        best_us = us;
+  int best;
+  uint32_t bestS;
+  auto search = [&](uint32_t max_s) {
+    best = -1;
+    bestS = 1;
+    double best_us = forced ? 1e301 : full_us;
+    for (int c = 0; c < ncfg; ++c) {
+      if (forced && c != h->gemm_ring - 1) continue;
+      const RingCfg &r = cfgs[c];
+      const uint64_t tiles = (((uint64_t)g.M + r.bm - 1) / r.bm) * (((uint64_t)g.N + r.bn - 1) / r.bn);
+      for (uint32_t want = 1; want <= max_s; ++want) {
+        if (forced && want != std::min(h->gemm_ring_split, max_s)) continue;
+        const uint32_t kchunk = (uint32_t)((((uint64_t)g.K + want - 1) / want + kQuantum - 1) / kQuantum * kQuantum);
+        const uint32_t S = (g.K + kchunk - 1) / kchunk;
+        if (S != want && !forced) continue;
+        if (tiles * S > 0x7fffffffull || (S > 1 && (!h->gemm_splitk || plane * S > kSplitBytes))) continue;
+        const double n = (double)((tiles * S + cus - 1) / cus);
+        double us = 4.0 + (n - 1.0) * costs[c].more +
+                    (double)std::min(kchunk, g.K) * (costs[c].lat + (n - 1.0) * costs[c].inc);
+        us = std::max(us, mem);
+        if (S > 1) us += 3.5 + 2.0 * (double)plane * S / 7e6;
+        if (us < best_us) {
+          best = c;
+          bestS = S;
+          best_us = us;
+        }
       }
+    }
+  };
+  search(16);
+  void *part = nullptr;
+  if (best >= 0 && bestS > 1) {
+    const size_t bytes = (size_t)(plane * bestS);
+    if (!use_ws) part = split_scratch(h, bytes);
+    else if (ws_ready(h, bytes) && ensure_ws(h, bytes) == BWPP_HIP_OK) part = h->ws;
+    if (!part) {
+      h->err.clear();  // no failure of this call
+      search(1);
     }
   }
   if (best < 0) return BWPP_HIP_OK;
-  void *part = bestS > 1 ? split_scratch(h, (size_t)(plane * bestS)) : nullptr;
-  if (!part) bestS = 1;  // this tile without a split
   const RingCfg &r = cfgs[best];
   g.tiles_m = (g.M + r.bm - 1) / r.bm;
   g.tiles_n = (g.N + r.bn - 1) / r.bn;
@@ -1192,7 +1219,7 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
     const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
     if (full) full_us = 4.0 + 0.0272 * p.K * (double)((tiles + cus - 1) / cus);
     else if (wide_ok) full_us = 4.0 + 0.041 * p.K * (double)(((uint64_t)g.tiles_m * ((p.N + 383) / 384) + cus - 1) / cus);
-    s = ring_dispatch(h, g, true, ta, tb, full_us, done);
+    s = ring_dispatch(h, g, true, ta, tb, full_us, false, done);
     if (s != BWPP_HIP_OK || done) return s;
   }
   if (wide_ok && (h->gemm_bn == 384 || (h->gemm_bn == 0 && p.N % BN != 0))) {
@@ -1240,30 +1267,41 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
       if (S > 1) t += (double)(2 * S - 1) * p.M * p.N * 4.0 / 6e6 + 2.0;
       return t;
     };
-    int bestKind = mode == 0 ? 0 : mode == 3 ? 1 : 2;
-    uint64_t bestS = 1;
-    uint32_t bestChunk = p.K;
-    double best = 1e300;
-    for (int kind = 0; kind < 3; ++kind) {
-      if (mode == 0 ? kind != 0 : mode == 1 ? kind == 0 : kind != bestKind) continue;
-      for (uint64_t S = 1; S <= 16 && p.K / S >= BK; ++S) {
-        if (S > 1 && !h->gemm_splitk) break;
-        const uint32_t kchunk = (uint32_t)(((p.K + S - 1) / S + BK - 1) / BK * BK);
-        const uint64_t Se = (p.K + kchunk - 1) / kchunk;
-        if (Se != S) continue;
-        const double c = cost(kind, Se, kchunk);
-        if (c < best) {
-          best = c;
-          bestKind = kind;
-          bestS = Se;
-          bestChunk = kchunk;
+    int bestKind;
+    uint64_t bestS;
+    uint32_t bestChunk;
+    double best;
+    auto search = [&](uint64_t max_s) {
+      bestKind = mode == 0 ? 0 : mode == 3 ? 1 : 2;
+      bestS = 1;
+      bestChunk = p.K;
+      best = 1e300;
+      for (int kind = 0; kind < 3; ++kind) {
+        if (mode == 0 ? kind != 0 : mode == 1 ? kind == 0 : kind != bestKind) continue;
+        for (uint64_t S = 1; S <= max_s && p.K / S >= BK; ++S) {
+          if (S > 1 && !h->gemm_splitk) break;
+          const uint32_t kchunk = (uint32_t)(((p.K + S - 1) / S + BK - 1) / BK * BK);
+          const uint64_t Se = (p.K + kchunk - 1) / kchunk;
+          if (Se != S) continue;
+          const double c = cost(kind, Se, kchunk);
+          if (c < best) {
+            best = c;
+            bestKind = kind;
+            bestS = Se;
+            bestChunk = kchunk;
+          }
         }
       }
-    }
-    if (mode == 1 && h->gemm_ring != 0) {
-      // Small products: smaller tiles, one launch (256^3 10.0 -> 4.9 us).
-      s = ring_dispatch(h, g, false, ta, tb, best + 2.0, done);
-      if (s != BWPP_HIP_OK || done) return s;
+    };
+    // Small products: smaller tiles, one launch (256^3 10.0 -> 4.9 us).
+    auto small = [&] {
+      return mode == 1 && h->gemm_ring != 0 ? ring_dispatch(h, g, false, ta, tb, best + 2.0, true, done) : BWPP_HIP_OK;
+    };
+    search(16);
+    if ((s = small()) != BWPP_HIP_OK || done) return s;
+    if (bestS > 1 && !ws_ready(h, (size_t)bestS * p.M * p.N * sizeof(float))) {
+      search(1);
+      if ((s = small()) != BWPP_HIP_OK || done) return s;
     }
     const int ring4 = bestKind == 2;
     if (bestS > 1) {
@@ -1281,7 +1319,7 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
     if (bestKind) return launch(h, h->gemm_f32p[ring4][ta][tb][0], (uint32_t)tiles, 1, 1, 256, g);
   }
   if (!bf16 && !full && h->gemm_ring != 0) {
-    s = ring_dispatch(h, g, false, ta, tb, 1e300, done);
+    s = ring_dispatch(h, g, false, ta, tb, 1e300, false, done);
     if (s != BWPP_HIP_OK || done) return s;
   }
   return launch(h, h->gemm[bf16 ? 1 : 0][ta][tb][full ? 1 : 0], (uint32_t)tiles, 1, 1, 256, g);

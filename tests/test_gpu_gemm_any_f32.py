@@ -97,3 +97,55 @@ def test_chosen(be, M, N, K, ta, tb):
     (the guarded edge kernel)."""
     for fuse in range(4):
         _check(be, M, N, K, ta, tb, 1, 2, 3, fuse)
+
+
+@pytest.mark.parametrize("warm", [True, False])
+@pytest.mark.parametrize("M,N,K", [(128, 128, 4096), (256, 256, 8192)])
+def test_caller_capture(monkeypatch, M, N, K, warm):
+    """A full-tile size that splits K through the workspace: a graph that the
+    caller records after a warm-up call splits too (the same kernels, the same
+    bits); one recorded on a new handle, which may not allocate, takes the
+    choice of a handle that never splits."""
+    import torch
+
+    def names(h):
+        return [h.recent_kernel(i) for i in (0, 1)]
+
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    a, b = torch.randn(M, K, device="cuda", generator=gen), torch.randn(K, N, device="cuda", generator=gen)
+    e, c = torch.zeros(M, N, device="cuda"), torch.zeros(M, N, device="cuda")
+    p = bwpp.MatmulParams(M, N, K, K, N, N, int(bwpp.DType.F32), 0, 0, 0)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    if not warm:
+        monkeypatch.setenv("BWPP_GEMM_SPLITK", "0")
+    ref = bwpp.HipBackend(0)
+    monkeypatch.delenv("BWPP_GEMM_SPLITK", raising=False)
+    h = ref if warm else bwpp.HipBackend(0)
+    try:
+        ref.set_stream(s)
+        h.set_stream(s)
+        ref.dispatch_matmul(a, b, e, None, p)
+        want = names(ref)
+        assert (want[0] == "bwpp_gemm_f32_splitk_reduce") == warm
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            h.dispatch_matmul(a, b, c, None, p)
+        assert names(h) == want if warm else h.last_kernel == want[0]
+        for _ in range(3):
+            c.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(s):
+                g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c, e)
+            e.zero_()
+            torch.cuda.synchronize()
+            ref.dispatch_matmul(a, b, e, None, p)  # eager work between the replays
+            torch.cuda.synchronize()
+    finally:
+        torch.cuda.synchronize()
+        ref.close()
+        if h is not ref:
+            h.close()

@@ -116,3 +116,44 @@ def test_caller_capture(be):
     finally:
         torch.cuda.synchronize()
         h.close()
+
+
+@pytest.mark.parametrize("M,N,K", [(128, 1024, 4096), (512, 512, 4096)])
+def test_caller_capture_tile(monkeypatch, M, N, K):
+    """A graph the caller records takes the tile that is best without a
+    split, which a handle that never splits chooses, and not the split's."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    a, b = (torch.randn(s, device="cuda", generator=gen).to(torch.bfloat16) for s in ((M, K), (K, N)))
+    c, e = (torch.zeros(M, N, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    p = bwpp.MatmulParams(M, N, K, K, N, N, int(bwpp.DType.BF16), 0, 0, 0)
+    h = bwpp.HipBackend(0)
+    monkeypatch.setenv("BWPP_GEMM_SPLITK", "0")
+    ref = bwpp.HipBackend(0)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    try:
+        h.set_stream(s)
+        ref.set_stream(s)
+        h.dispatch_matmul(a, b, c, None, p)
+        assert h.last_kernel == "bwpp_gemm_bf16_splitk_reduce"
+        ref.dispatch_matmul(a, b, e, None, p)
+        assert ref.last_kernel != h.recent_kernel(1)  # the split's tile is another
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            h.dispatch_matmul(a, b, c, None, p)
+        assert h.last_kernel == ref.last_kernel
+        for _ in range(3):
+            c.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(s):
+                g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c, e)
+            ref.dispatch_matmul(a, b, e, None, p)
+            torch.cuda.synchronize()
+    finally:
+        torch.cuda.synchronize()
+        h.close()
+        ref.close()
