@@ -292,6 +292,10 @@ __device__ __forceinline__ void attn_fwd(const BwppAttnArgs &a) {
 // meet in LDS, those of a split slice in bwpp_attn_dec_combine_f32.  B4 H8 M1
 // N8000 d128: 32 blocks with three of four waves idle 1105 us, this 50
 // us (262 MB at 5.3 TB/s; B8 H32 N4095 619 -> 181).
+//
+// A masked key has p = 0, but 0 * v is NaN for an infinite or NaN v: masked
+// tiles look for such V elements, and where one is found form the tile's sums
+// element by element over visible keys only.
 template <int D, bool CAUSAL>
 __device__ __forceinline__ void attn_dec(const BwppAttnArgs &a) {
   constexpr int ST = D + 4;
@@ -348,13 +352,12 @@ __device__ __forceinline__ void attn_dec(const BwppAttnArgs &a) {
     __builtin_amdgcn_sched_barrier(0);  // the next K's ahead of the softmax and the second product
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] *= c;
-    if (k0 + kR > kend || (CAUSAL && (int64_t)k0 + kR - 1 > diag)) {  // wave-uniform
+    const bool masked = k0 + kR > kend || (CAUSAL && (int64_t)k0 + kR - 1 > diag);  // wave-uniform
+    if (masked) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const uint32_t key = k0 + (uint32_t)acc_row(r, hi);
         if (key >= kend || (CAUSAL && (int64_t)key > (int64_t)li + diag)) s[r] = -INFINITY;
-#pragma unroll
-        for (int blk = 0; blk < D / 32; ++blk) v[r][blk] = key < kend ? v[r][blk] : 0.0f;
       }
     }
     float mx = -INFINITY;
@@ -374,10 +377,45 @@ __device__ __forceinline__ void attn_dec(const BwppAttnArgs &a) {
     mrun = mnew;
 #pragma unroll
     for (int blk = 0; blk < D / 32; ++blk) o[blk] *= alpha;
+    bool plain = true;  // wave-uniform
+    if (masked) {
+      float nan[2] = {0.0f, 0.0f};  // sums of 0 v: 0, or NaN
 #pragma unroll
-    for (int r = 0; r < 16; ++r)
+      for (int r = 0; r < 16; ++r)
 #pragma unroll
-      for (int blk = 0; blk < D / 32; ++blk) o[blk] = mfma(v[r][blk], s[r], o[blk]);
+        for (int blk = 0; blk < D / 32; ++blk) {
+          v[r][blk] = k0 + (uint32_t)acc_row(r, hi) < kend ? v[r][blk] : 0.0f;
+          nan[blk & 1] = __builtin_fmaf(v[r][blk], 0.0f, nan[blk & 1]);
+        }
+      plain = __ballot(nan[0] + nan[1] != 0.0f) == 0;
+    }
+    if (plain) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+#pragma unroll
+        for (int blk = 0; blk < D / 32; ++blk) o[blk] = mfma(v[r][blk], s[r], o[blk]);
+    } else {
+      float(*ps)[ST] = os[wave];  // [key][query]; free until the waves' triples are stored
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ps[acc_row(r, hi)][li] = s[r];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      for (uint32_t key = k0; key < min(k0 + kR, kend); ++key) {
+        const float p = ps[key - k0][li];
+        const float *src = V + (size_t)key * a.ldv + 4 * hi;
+        if (!CAUSAL || (int64_t)key <= (int64_t)li + diag) {
+#pragma unroll
+          for (int blk = 0; blk < D / 32; ++blk)
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) {
+              const f32x4 t = *reinterpret_cast<const f32x4 *>(src + 32 * blk + 8 * r4);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) o[blk][4 * r4 + e] += p * t[e];
+            }
+        }
+      }
+    }
   }
   const float ltot = sum32(lsum);
   store_t<D>(&os[wave][0][0], ST, (uint32_t)li, o, 1.0f, hi);

@@ -150,3 +150,39 @@ def test_decode_f32(be, oracle, D, B, H, M, N, pad, causal):
         be.dispatch_attention(rows(q), rows(k), rows(vi), o, prm)
         torch.cuda.synchronize()
         assert bool(torch.isposinf(o[..., 0, 3]).all()) and bool(torch.isfinite(o[..., 0, 4:D]).all())
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("M,N,causal", [(20, 70, True), (8, 2060, True), (4, 45, False), (32, 32, True)])
+def test_non_finite_values_f32(be, D, M, N, causal):
+    """The same for the fp32 kernel, against the generic path (rows that no
+    16-byte load divides); finite results within 1e-5 of the largest."""
+    import torch
+    H = 3
+    q, k, v = (synth.normal((1, H, r, D), 9, i) for i, r in enumerate((M, N, N)))
+    v[0, 0, N - 1, 5] = np.inf   # seen by the last query only under the mask
+    v[0, 1, N - 3, 7] = -np.inf
+    v[0, 1, N - 3, 8] = np.nan
+    v[0, 2, 3, 60] = np.inf
+
+    def run(ld):
+        def rows(t):
+            r = torch.full(t.shape[:3] + (ld,), 3.0, device="cuda")
+            r[..., :D] = torch.from_numpy(t).cuda()
+            return r
+
+        o = torch.full((1, H, M, ld), 5.0, device="cuda")
+        be.dispatch_attention(rows(q), rows(k), rows(v), o,
+                              bwpp.AttentionParams(M=M, N=N, K=D, D=D, ldq=ld, ldk=ld, ldv=ld, ldo=ld, batch=1, heads=H,
+                                                   scale=D ** -0.5, causal=int(causal)))
+        torch.cuda.synchronize()
+        return o[..., :D].cpu().numpy()
+
+    o, first = run(D), be.recent_kernel(1 if be.last_kernel == "bwpp_attn_dec_combine_f32" else 0)
+    assert first.startswith(f"bwpp_attn_f32_dec_d{D}")
+    g = run(D + 1)
+    assert be.last_kernel.startswith("bwpp_attn_generic_f32")
+    assert np.array_equal(np.isnan(o), np.isnan(g))
+    assert np.array_equal(np.isposinf(o), np.isposinf(g)) and np.array_equal(np.isneginf(o), np.isneginf(g))
+    fin = np.isfinite(g)
+    assert np.all(np.abs(o[fin] - g[fin]) <= 1e-5 * np.abs(g[fin]).max())
