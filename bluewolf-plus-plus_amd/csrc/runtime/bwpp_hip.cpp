@@ -449,10 +449,19 @@ void *split_scratch(BwppHip *h, size_t bytes) {
     return h->split;
   }
   if (recording(h)) return nullptr;
-  if (!h->split && hipMalloc(&h->split, kSplitBytes) != hipSuccess) {
-    (void)hipGetLastError();
-    h->split = nullptr;
-    h->split_off = true;
+  if (!h->split) {
+    // Relaxed: another stream may be recorded meanwhile, by this thread or
+    // another (torch records in the global mode, in which an allocation fails
+    // and spoils the recording).
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const hipError_t e = hipMalloc(&h->split, kSplitBytes);
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      h->split = nullptr;
+      h->split_off = true;
+    }
   }
   return h->split && bwpp_hip_split_enter(h) ? h->split : nullptr;
 }

@@ -157,3 +157,32 @@ def test_caller_capture_tile(monkeypatch, M, N, K):
         torch.cuda.synchronize()
         h.close()
         ref.close()
+
+
+def test_first_split_while_another_stream_is_recorded():
+    """The scratch's one allocation does not disturb a recording (in the mode
+    that forbids allocations to the whole process) on another stream, and the
+    call splits."""
+    import torch
+    M, N, K = 8, 512, 4096
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    a, b = (torch.randn(s, device="cuda", generator=gen).to(torch.bfloat16) for s in ((M, K), (K, N)))
+    c, x = torch.zeros(M, N, device="cuda", dtype=torch.bfloat16), torch.zeros(64, device="cuda")
+    h = bwpp.HipBackend(0)
+    try:
+        h.set_stream(torch.cuda.Stream())
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, capture_error_mode="global"):
+            x.add_(1.0)
+            h.dispatch_matmul(a, b, c, None, bwpp.MatmulParams(M, N, K, K, N, N, int(bwpp.DType.BF16), 0, 0, 0))
+        assert h.last_kernel == "bwpp_gemm_bf16_splitk_reduce"
+        for i in range(3):
+            g.replay()
+            torch.cuda.synchronize()
+            assert bool((x == i + 1).all())
+        want = a.double() @ b.double()
+        assert bool(((c.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-3).all())
+    finally:
+        torch.cuda.synchronize()
+        h.close()
