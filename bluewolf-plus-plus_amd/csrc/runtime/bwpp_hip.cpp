@@ -476,10 +476,16 @@ BwppHipStatus enter(BwppHip *h) {
   return BWPP_HIP_OK;
 }
 
+inline bool launchable(uint64_t blocks, uint32_t threads) { return blocks * threads <= 0xffffffffull; }
+
 template <class Args>
 BwppHipStatus launch(BwppHip *h, hipFunction_t f, uint32_t gx, uint32_t gy, uint32_t gz, uint32_t bx,
                      const Args &args, uint32_t shmem = 0) {
   if (gx == 0 || gy == 0 || gz == 0) return BWPP_HIP_OK;
+  // Threads along x are counted in 32 bits: beyond that a launch runs a part
+  // of its grid and reports success.
+  if (!launchable(gx, bx))
+    return fail(h, BWPP_HIP_ERR_UNSUPPORTED, "launch of %u blocks of %u threads: 2^32 threads or more", gx, bx);
   const auto mt = h->max_threads.find(f);
   if (mt == h->max_threads.end() || bx > mt->second)
     return fail(h, BWPP_HIP_ERR_HIP, "launch of %u threads per block exceeds the kernel's limit (%u)", bx,
@@ -539,18 +545,31 @@ int pick_row_cfg(const BwppHip *h, RowOpId op, uint32_t cols) {
 // grid of 2 blocks per CU (measured best of 1 / 2 / 4 / one per row) so each
 // block reuses its gamma/beta registers over several rows; the others launch
 // one block per row group.
-BwppHipStatus row_dispatch(BwppHip *h, RowOpId op, const BwppRowArgs &a) {
-  if (a.cols < 4) return launch(h, h->row_tiny[op], (uint32_t)(((uint64_t)a.rows + 255) / 256), 1, 1, 256, a);
-  const int c = pick_row_cfg(h, op, a.cols);
-  if (c < 0) return launch(h, h->row_gen[op], a.rows, 1, 1, 256, a);
-  const RowCfg &cfg = kRowCfgs[c];
-  const int full = (a.cols == row_capacity(cfg)) ? 1 : 0;
-  const uint32_t rpb = row_rows_per_block(cfg);
-  uint32_t grid = (a.rows + rpb - 1) / rpb;
+BwppHipStatus row_dispatch(BwppHip *h, RowOpId op, const BwppRowArgs &all) {
+  const int c = all.cols < 4 ? -1 : pick_row_cfg(h, op, all.cols);
+  const uint32_t rpb = all.cols < 4 ? 256u : c < 0 ? 1u : row_rows_per_block(kRowCfgs[c]);
+  const uint32_t block = c < 0 ? 256u : row_block(kRowCfgs[c]);
   uint32_t cap = h->row_grid_cap;
   if (cap == 0 && (op == ROW_RMSNORM || op == ROW_LAYERNORM) && h->cus > 0) cap = 2u * (uint32_t)h->cus;
-  if (cap && grid > cap) grid = cap;
-  return launch(h, h->row_reg[op][c][full], grid, 1, 1, row_block(cfg), a);
+  const hipFunction_t f = all.cols < 4 ? h->row_tiny[op]
+                          : c < 0      ? h->row_gen[op]
+                                       : h->row_reg[op][c][all.cols == row_capacity(kRowCfgs[c]) ? 1 : 0];
+  // One launch up to 2^31 threads (2^25 rows of up to 1024 columns).
+  const uint64_t per_launch = (0x80000000ull / block) * rpb;
+  for (uint64_t r0 = 0; r0 < all.rows; r0 += per_launch) {
+    BwppRowArgs a = all;
+    a.rows = (uint32_t)std::min<uint64_t>(per_launch, all.rows - r0);
+    a.x += r0 * a.ld;
+    if (a.y) a.y += r0 * a.ld;
+    if (a.dy) a.dy += r0;
+    if (a.maxv) a.maxv += r0;
+    if (a.argmax) a.argmax += r0;
+    uint32_t grid = (a.rows + rpb - 1) / rpb;
+    if (c >= 0 && cap && grid > cap) grid = cap;
+    const BwppHipStatus s = launch(h, f, grid, 1, 1, block, a);
+    if (s != BWPP_HIP_OK) return s;
+  }
+  return BWPP_HIP_OK;
 }
 
 inline uint32_t stream_grid(uint32_t rows) { return rows < (1u << 20) ? rows : (1u << 20); }
@@ -576,23 +595,47 @@ uint32_t col_bands(const BwppHip *h, uint32_t rows, uint32_t cols) {
   return (uint32_t)std::min<uint64_t>(std::min<uint64_t>(std::max<uint64_t>(1, want / blocks), by_rows), 512);
 }
 
+// f(a) over at most 2^28 columns at a time: blocks of 256 threads per 64
+// columns, and fewer than 2^32 threads a launch.
+template <class F>
+BwppHipStatus col_pieces(const BwppRowArgs &all, F f) {
+  constexpr uint32_t kPiece = 1u << 28;
+  for (uint64_t c0 = 0; c0 < all.cols; c0 += kPiece) {
+    BwppRowArgs a = all;
+    a.cols = (uint32_t)std::min<uint64_t>(kPiece, all.cols - c0);
+    for (const float **p : {&a.x, &a.dy})
+      if (*p) *p += c0;
+    for (float **p : {&a.y, &a.maxv, &a.part_v})
+      if (*p) *p += c0;
+    if (a.argmax) a.argmax += c0;
+    if (a.idx_in) a.idx_in += c0;
+    const BwppHipStatus s = f(a);
+    if (s != BWPP_HIP_OK) return s;
+  }
+  return BWPP_HIP_OK;
+}
+
 // Column maxima into a.maxv / a.argmax (either may be NULL); `part`: 8 *
 // bands * cols bytes, used when bands > 1.
 BwppHipStatus col_max_launch(BwppHip *h, BwppRowArgs a, uint32_t bands, void *part) {
   a.bands = bands;
   a.part_v = static_cast<float *>(part);
   a.part_i = reinterpret_cast<uint32_t *>(a.part_v + (size_t)bands * a.cols);
-  const uint32_t gx = (uint32_t)(((uint64_t)a.cols + 63) / 64);
-  BwppHipStatus s = launch(h, h->col_max_band, gx, bands, 1, 256, a);
-  if (s != BWPP_HIP_OK || bands == 1) return s;
-  return launch(h, h->col_max_final, gx, 1, 1, 256, a);
+  if (bands > 1) {  // at most 2^17 columns (col_bands)
+    const uint32_t gx = (a.cols + 63) / 64;
+    BwppHipStatus s = launch(h, h->col_max_band, gx, bands, 1, 256, a);
+    return s != BWPP_HIP_OK ? s : launch(h, h->col_max_final, gx, 1, 1, 256, a);
+  }
+  return col_pieces(a, [&](const BwppRowArgs &p) { return launch(h, h->col_max_band, (p.cols + 63) / 64, 1, 1, 256, p); });
 }
 
 BwppHipStatus col_apply_launch(BwppHip *h, hipFunction_t (&f)[2], const BwppRowArgs &a, bool vec) {
-  const uint64_t gx = vec ? ((uint64_t)a.cols + 255) / 256 : ((uint64_t)a.cols + 63) / 64;
-  const uint64_t want = 8ull * (uint64_t)(h->cus > 0 ? h->cus : 256);
-  const uint64_t gy = std::min<uint64_t>(std::max<uint64_t>(1, want / gx), ((uint64_t)a.rows + 15) / 16);
-  return launch(h, f[vec ? 1 : 0], (uint32_t)gx, (uint32_t)gy, 1, 256, a);
+  return col_pieces(a, [&](const BwppRowArgs &p) {
+    const uint64_t gx = vec ? (p.cols + 255) / 256 : (p.cols + 63) / 64;
+    const uint64_t want = 8ull * (uint64_t)(h->cus > 0 ? h->cus : 256);
+    const uint64_t gy = std::min<uint64_t>(std::max<uint64_t>(1, want / gx), ((uint64_t)p.rows + 15) / 16);
+    return launch(h, f[vec ? 1 : 0], (uint32_t)gx, (uint32_t)gy, 1, 256, p);
+  });
 }
 
 }  // namespace
@@ -1081,7 +1124,7 @@ BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool bf16, bool ta, bool
         const uint32_t kchunk = (uint32_t)((((uint64_t)g.K + want - 1) / want + kQuantum - 1) / kQuantum * kQuantum);
         const uint32_t S = (g.K + kchunk - 1) / kchunk;
         if (S != want && !forced) continue;
-        if (tiles * S > 0x7fffffffull || (S > 1 && (!h->gemm_splitk || plane * S > kSplitBytes))) continue;
+        if (!launchable(tiles * S, r.threads) || (S > 1 && (!h->gemm_splitk || plane * S > kSplitBytes))) continue;
         const double n = (double)((tiles * S + cus - 1) / cus);
         double us = 4.0 + (n - 1.0) * costs[c].more +
                     (double)std::min(kchunk, g.K) * (costs[c].lat + (n - 1.0) * costs[c].inc);
@@ -1111,7 +1154,6 @@ BwppHipStatus ring_dispatch(BwppHip *h, BwppGemmArgs g, bool bf16, bool ta, bool
   g.tiles_m = (g.M + r.bm - 1) / r.bm;
   g.tiles_n = (g.N + r.bn - 1) / r.bn;
   const uint64_t tiles = (uint64_t)g.tiles_m * g.tiles_n;
-  if (tiles > 0x7fffffffull) return BWPP_HIP_OK;
   g.ksplit = bestS;
   g.kchunk = bestS > 1 ? (uint32_t)((((uint64_t)g.K + bestS - 1) / bestS + kQuantum - 1) / kQuantum * kQuantum) : g.K;
   g.part = static_cast<float *>(part);
@@ -1945,11 +1987,13 @@ extern "C" BwppHipStatus bwpp_hip_dispatch_softmax_grad(BwppHip *h, const float 
   g.cols = p.cols;
   g.ld = ld;
   const int c = grad_cfg(p.cols, kGradNCfg);
-  if (c < 0) return launch(h, h->softmax_grad, row_grid(h, p.rows), 1, 1, 256, g);
+  const uint32_t rpb = c >= 0 ? row_rows_per_block(kGradCfgs[c]) : 1u;
+  const uint64_t blocks = ((uint64_t)p.rows + rpb - 1) / rpb;
+  // The register kernels hold one group of rows per block: up to 2^26 rows.
+  if (c < 0 || !launchable(blocks, row_block(kGradCfgs[c])))
+    return launch(h, h->softmax_grad, row_grid(h, p.rows), 1, 1, 256, g);
   const bool vec = p.cols % 4 == 0 && ld % 4 == 0 && aligned16(y) && aligned16(dy) && aligned16(dx);
-  const uint32_t rpb = row_rows_per_block(kGradCfgs[c]);
-  return launch(h, h->softmax_grad_reg[c][vec ? 1 : 0], (uint32_t)(((uint64_t)p.rows + rpb - 1) / rpb), 1, 1,
-                row_block(kGradCfgs[c]), g);
+  return launch(h, h->softmax_grad_reg[c][vec ? 1 : 0], (uint32_t)blocks, 1, 1, row_block(kGradCfgs[c]), g);
 }
 
 extern "C" BwppHipStatus bwpp_hip_dispatch_rmsnorm_grad(BwppHip *h, const float *x, const float *gamma,

@@ -108,3 +108,19 @@ def test_axis0_streams_and_capture(oracle):
     finally:
         torch.cuda.synchronize()
         h.close()
+
+
+@pytest.mark.parametrize("cols", [(1 << 30) + 4, (1 << 30) + 5])
+def test_most_columns(be, cols):
+    """More columns than one launch of 64 a block takes (2^32 threads): two
+    rows of 2^30 columns, in pieces."""
+    import torch
+    x = torch.randn(2, cols, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    mv, ix = torch.full((cols,), 9.0, device="cuda"), torch.full((cols,), 9, device="cuda", dtype=torch.int32)
+    p = bwpp.ReduceParams(2, cols, cols, 0)
+    be.dispatch_reduce_max(x, mv, ix, p)
+    assert torch.equal(mv, torch.maximum(x[0], x[1])) and torch.equal(ix, (x[1] > x[0]).int())
+    dx = torch.full_like(x, 9.0)
+    be.dispatch_reduce_max_grad_argmax(None, ix, mv, dx, p)
+    for r in range(2):
+        assert torch.equal(dx[r], torch.where(ix == r, mv, torch.zeros((), device="cuda")))

@@ -149,3 +149,17 @@ def test_caller_capture(monkeypatch, M, N, K, warm):
         ref.close()
         if h is not ref:
             h.close()
+
+
+def test_most_columns(be):
+    """Columns for which 64-wide tiles would be a launch of 2^32 threads."""
+    import torch
+    N, K, step = 1 << 30, 4, 1 << 27
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    a, b = torch.randn(1, K, device="cuda", generator=gen), torch.randn(K, N, device="cuda", generator=gen)
+    c = torch.full((1, N), 7.0, device="cuda")
+    be.dispatch_matmul(a, b, c, None, bwpp.MatmulParams(1, N, K, K, N, N, int(bwpp.DType.F32), 0, 0, 0))
+    assert be.last_kernel.startswith("bwpp_gemm_f32r")
+    for n in range(0, N, step):
+        t = a[0, :, None].double() * b[:, n:n + step].double()
+        assert bool(((c[0, n:n + step].double() - t.sum(0)).abs() <= 2.0 ** -21 * t.abs().sum(0)).all())

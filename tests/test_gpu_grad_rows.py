@@ -90,3 +90,19 @@ def test_reduce_sum_axis0_bands(be, rows, cols, pad):
     # an fp32 sum's error bound, gamma_n of the band and merge sums' depth (< 100 additions)
     bound = 100 * 2.0 ** -24 * np.abs(x.astype(np.float64)).sum(axis=0)
     assert np.all(np.abs(out.cpu().numpy() - want) <= bound)
+
+
+@pytest.mark.parametrize("rows", [(1 << 26) - 4, (1 << 26) + 5])
+def test_softmax_grad_most_rows(be, rows):
+    """The last row count that one launch of four rows a block can take, and
+    the first beyond it (2^32 threads); one column, dx = y (dy - dy y), three
+    roundings."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    y = torch.rand(rows, device="cuda", generator=gen)
+    dy = torch.randn(rows, device="cuda", generator=gen)
+    out = torch.full_like(y, 7.0)
+    be.dispatch_softmax_grad(y, dy, out, bwpp.SoftmaxParams(rows, 1, 1))
+    torch.cuda.synchronize()
+    want = y.double() * (dy.double() - dy.double() * y.double())
+    assert bool(((out.double() - want).abs() <= 3 * 2.0 ** -24 * dy.double().abs()).all())

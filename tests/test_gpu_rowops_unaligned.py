@@ -69,3 +69,22 @@ def test_unaligned_rows(be, oracle, rows, cols, pad, off):
     assert_bits_equal(mv.cpu().numpy(), wm)
     assert np.array_equal(ix.cpu().numpy(), wi)
     _get(xb, rows, cols, ld, off), _get(gb, 1, cols, cols, (off + 1) % 4), _get(bb, 1, cols, cols, (off + 2) % 4)
+
+
+@pytest.mark.parametrize("cols", [2, 4])
+def test_most_rows(be, cols):
+    """More rows than one launch takes at four rows a block (2^32 threads, run
+    in pieces of 2^25 rows); softmax within 1e-5, the others exact."""
+    import torch
+    rows = (1 << 26) + 5
+    x = torch.randn(rows, cols, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    y = torch.full_like(x, GUARD)
+    be.dispatch_softmax(x, y, bwpp.SoftmaxParams(rows, cols, cols))
+    assert bool(((y - torch.softmax(x, dim=1)).abs() <= 1e-5).all())
+    mp = bwpp.ReduceParams(rows, cols, cols, 1)
+    mv, ix = torch.full((rows,), GUARD, device="cuda"), torch.full((rows,), 7, device="cuda", dtype=torch.int32)
+    be.dispatch_reduce_max(x, mv, ix, mp)
+    want, arg = x.max(dim=1)
+    assert torch.equal(mv, want) and torch.equal(x.gather(1, ix.long()[:, None])[:, 0], want)
+    be.dispatch_reduce_max_grad_argmax(x, None, mv, y, mp)
+    assert torch.equal(y, torch.zeros_like(x).scatter_(1, ix.long()[:, None], want[:, None]))
