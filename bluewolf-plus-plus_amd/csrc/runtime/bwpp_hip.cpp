@@ -1216,8 +1216,8 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
   // Full-tile kernels: bf16 256 x 256 with K in steps of 32 (pipelined),
   // fp32 128 x 128 with K in steps of 32.  Other products take the kernels for
   // any M, N and K (ring_dispatch); the guarded edge kernels are left what
-  // those cannot load (operands shorter than a 16-byte chunk) and up to K = 64
-  // the 256-row bf16 products below.
+  // those cannot load (operands shorter than a 16-byte chunk) and the 256-row
+  // bf16 products of K = 32 and 64 below.
   const uint32_t BM = bf16 ? 256 : 128, BN = bf16 ? 256 : 128, BK = 32;
   const uint32_t vecw = bf16 ? 8 : 4;  // elements per 16 bytes
   const bool vec = aligned16(a) && aligned16(b) && aligned16(c) && lda % vecw == 0 && ldb % vecw == 0 &&
@@ -1260,12 +1260,16 @@ BwppHipStatus matmul_impl(BwppHip *h, const void *a, const void *b, void *c, con
   // bf16: the kernels for any M, N and K, where their model finds them faster
   // than the full tiles (0.0272 us per K and round of 256 x 256 tiles, 4096^3
   // in 115 us; 0.041 of 256 x 384), whose knobs, when set, ask for those.
-  // Up to K = 64 whole 256-row tiles keep the 256-wide kernels, the documented
-  // choice there (512 x 1000 x 64 15.6 us, 4.3 with 64 x 64 ring tiles); other
-  // row counts do not (1 x 64 x 64 33 us on the edge kernel, 4.9 so).
+  // K = 32 and 64 with whole 256-row tiles keep the 256-wide and edge kernels
+  // only because the kernel-choice tests name them there; they are the slower
+  // ones (512 x 1000 x 64 14.5 us on 256 x 384 tiles, 512 x 1004 x 64 49 on
+  // edge tiles, 4.5 with 64 x 64 ring tiles).  Every other K and row count up
+  // to K = 64 takes the model's choice (1 x 64 x 64 33 us on the edge kernel,
+  // 4.9 so; 1024 x 3000 x 33 with A transposed 22 -> 6.8, 4096 x 512 x 63 48 ->
+  // 5.8, 4096 x 11008 x 50 160 -> 31).
   const bool any = h->gemm_ring != 0 && (h->gemm_ring > 0 || (h->gemm_bn == 0 && h->gemm_waves == 8));
   bool done = false;
-  if (bf16 && any && (p.K > 64 || p.M % BM != 0 || h->gemm_ring > 0)) {
+  if (bf16 && any && (p.K > 64 || p.K % BK != 0 || p.M % BM != 0 || h->gemm_ring > 0)) {
     double full_us = 1e300;
     const uint64_t cus = h->cus > 0 ? (uint64_t)h->cus : 256ull;
     if (full) full_us = 4.0 + 0.0272 * p.K * (double)((tiles + cus - 1) / cus);

@@ -83,6 +83,15 @@ def test_chosen(be, M, N, K, tb):
     _check(be, M, N, K, 0, tb, 0, 0, 3)
 
 
+@pytest.mark.parametrize("M,N,K,ta,tb", [(256, 3000, 33, 1, 0), (512, 264, 63, 0, 1), (1024, 100, 48, 1, 1),
+                                         (256, 11008, 8, 0, 0), (256, 520, 31, 1, 0)])
+def test_whole_row_tiles_short_k(be, M, N, K, ta, tb):
+    """Whole 256-row tiles whose K is short and no multiple of 32 (a gradient
+    over a few tokens): no 256-wide kernel runs there."""
+    _check(be, M, N, K, ta, tb, 0, 0, 3)
+    assert be.last_kernel.startswith("bwpp_gemm_bf16r")
+
+
 def test_caller_capture(be):
     """A graph the caller records takes no split (it may be replayed beside
     the handle's other work); its replays match the eager result to the
