@@ -176,9 +176,23 @@ BwppHipStatus bwpp_hip_create(BwppHip **out, int device,
                               const char *code_object_dir);
 void bwpp_hip_destroy(BwppHip *h);
 /* Stream for subsequent launches (a hipStream_t); NULL = the null stream.
- * The handle's workspace (split-K partials, attention-backward row sums,
- * column partials) is ordered on the handle's stream: when the stream
- * changes, the new stream first waits for the work queued on the old one. */
+ * The handle's workspace (split-K partials of fp32 products, attention-
+ * backward row sums, column partials) is ordered on the handle's stream: when
+ * the stream changes, the new stream first waits for the work queued on the
+ * old one.
+ *
+ * Besides the workspace a handle has one scratch of 64 MiB, allocated by the
+ * first call that splits its work through it (bf16 and ragged fp32 products
+ * over K, attention with at most 32 queries over the keys, reduce_max and its
+ * mask and gradient over rows) and kept until bwpp_hip_destroy.  Calls without
+ * it take other kernels or no split, with the same results up to the order of
+ * sums: where it cannot be allocated, and in a graph that the caller records,
+ * which may run beside this handle's other work (plans recorded by
+ * bwpp_hip_plan_capture do use it).  A use of it on another stream waits for
+ * the last one; changing the stream while the old one is being recorded
+ * leaves no way to wait, and the handle then goes on without the scratch.
+ * A graph that the caller records addresses the workspace as it then is: run
+ * the calls once before, and record again after a call that needs more. */
 BwppHipStatus bwpp_hip_set_stream(BwppHip *h, void *hip_stream);
 void *bwpp_hip_get_stream(const BwppHip *h);
 /* Waits for all work on the handle's stream. */
@@ -379,10 +393,15 @@ BwppHipStatus bwpp_hip_dispatch_attention(BwppHip *h, const void *q,
  * for the backward below.  No reference counterpart (the reference
  * differentiates attention through its decomposed graph ops,
  * graph_ir.c:1722-1733, 1529-1583).  The same kernels as the plain forward
- * run: bf16 with K = D = 128 and 16-byte rows (pointers, leading dims and
- * slice strides in multiples of 8 elements) takes the bf16 flash kernel;
- * fp32 with K = D = 64 or 128 and 16-byte rows takes the fp32 matrix-core
- * kernel; anything else the generic kernel. */
+ * run: bf16 with K = D = 32, 64, 96 or 128, 16-byte rows (pointers, leading
+ * dims and slice strides in multiples of 8 elements) and a positive scale
+ * takes the bf16 matrix-core kernels; fp32 with K = D = 64 or 128 and 16-byte
+ * rows the fp32 ones; both have kernels of their own for at most 32 queries
+ * (K = D = 64 or 128); anything else takes the generic kernel.  A key that a
+ * query does not see has weight 0.  With more than 32 queries the fp32
+ * matrix-core kernel and the bf16 one for K = D = 128 multiply V by that
+ * weight, so there an infinite or NaN V at a hidden key can turn a query of
+ * the same tile into NaN; the other kernels leave hidden keys out. */
 BwppHipStatus bwpp_hip_dispatch_attention_lse(BwppHip *h, const void *q,
                                               const void *k, const void *v,
                                               void *o, float *lse,
@@ -543,7 +562,9 @@ BwppHipStatus bwpp_hip_plan_run(BwppHipPlan *plan);
  * afterwards drops the graph; capture again. */
 BwppHipStatus bwpp_hip_plan_capture(BwppHipPlan *plan);
 /* Launches the captured graph on the handle's current stream (INVALID_ARG
- * when there is none).  Results equal bwpp_hip_plan_run's. */
+ * when there is none).  Results equal bwpp_hip_plan_run's.  Where the graph
+ * uses the handle's scratch and its last use cannot be waited for (see
+ * bwpp_hip_set_stream), runs the plan's launches instead. */
 BwppHipStatus bwpp_hip_plan_replay(BwppHipPlan *plan);
 /* Memory-plan report in mem_plan.c:176-193's layout plus byte sizes, arena
  * offsets and the total; returns the bytes needed including the NUL. */
