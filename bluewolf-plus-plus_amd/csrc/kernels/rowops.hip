@@ -46,7 +46,10 @@ constexpr uint32_t kNoIndex = 0xFFFFFFFFu;
 
 // Cross-wave steps of the row reductions.  A block holds 4/WPR rows
 // (WPR < 4) or one row of WPR waves; waves w0 .. w0+WPR-1 share a row.
-template <int WPR>
+// PAIRS: the waves' sums are added in pairs, as the multi-pass fallback adds
+// them: rows of any length are as exact as there (softmax's scale at 5003
+// columns 0.79 x 2^-24 rms, 0.96 with the eight added one after another).
+template <int WPR, bool PAIRS = false>
 __device__ __forceinline__ float row_sum(float v, float *red) {
   v = wave_sum(v);
   if constexpr (WPR > 1) {
@@ -54,9 +57,20 @@ __device__ __forceinline__ float row_sum(float v, float *red) {
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[w] = v;
     __syncthreads();
-    v = red[w0];
+    if constexpr (PAIRS) {
+      float p[WPR];
 #pragma unroll
-    for (int i = 1; i < WPR; ++i) v += red[w0 + i];
+      for (int i = 0; i < WPR; ++i) p[i] = red[w0 + i];
+#pragma unroll
+      for (int n = WPR / 2; n > 0; n /= 2)
+#pragma unroll
+        for (int i = 0; i < n; ++i) p[i] = p[2 * i] + p[2 * i + 1];
+      v = p[0];
+    } else {
+      v = red[w0];
+#pragma unroll
+      for (int i = 1; i < WPR; ++i) v += red[w0 + i];
+    }
   }
   return v;
 }
@@ -238,7 +252,7 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
           for (int e = 0; e < 4; ++e) s += own(j, e) ? get(v[j], e) : 0.0f;
         }
       }
-      s = row_sum<WPR>(s, redf);
+      s = row_sum<WPR, !FULL>(s, redf);
       const float inv = s > 0.0f ? 1.0f / s : 0.0f;
 #pragma unroll
       for (int j = 0; j < VPT; ++j)
@@ -263,7 +277,7 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
         } else {
           // Other rows: the row's mean first (a second reduction costs less
           // than merging unequal counts, which divides at every step).
-          mu = row_sum<WPR>(s, redf) / (float)cols;
+          mu = row_sum<WPR, true>(s, redf) / (float)cols;
         }
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
@@ -274,7 +288,7 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
           }
         }
         if constexpr (FULL) row_chan_equal<WPR>(n, mu, m2, redf);
-        else m2 = row_sum<WPR>(m2, redf);
+        else m2 = row_sum<WPR, true>(m2, redf);
         mean = mu;
         ss = m2;
       } else {
@@ -282,7 +296,7 @@ __device__ __forceinline__ void row_reg(const BwppRowArgs &a) {
         for (int j = 0; j < VPT; ++j)
           ss += (mine(j, 0, v[j].x * v[j].x) + mine(j, 1, v[j].y * v[j].y)) +
                 (mine(j, 2, v[j].z * v[j].z) + mine(j, 3, v[j].w * v[j].w));
-        ss = row_sum<WPR>(ss, redf);
+        ss = row_sum<WPR, !FULL>(ss, redf);
       }
       const float inv = 1.0f / sqrtf(ss / (float)cols + a.eps);
 #pragma unroll

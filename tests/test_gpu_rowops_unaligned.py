@@ -88,3 +88,20 @@ def test_most_rows(be, cols):
     assert torch.equal(mv, want) and torch.equal(x.gather(1, ix.long()[:, None])[:, 0], want)
     be.dispatch_reduce_max_grad_argmax(x, None, mv, y, mp)
     assert torch.equal(y, torch.zeros_like(x).scatter_(1, ix.long()[:, None], want[:, None]))
+
+
+@pytest.mark.parametrize("rows,cols", [(4000, 1921), (4000, 4095), (4000, 5003), (2000, 9001)])
+def test_softmax_scale_error(be, rows, cols):
+    """The rounding of a row's sum (its common factor: the row's outputs add
+    up to 1 but for that) where 4 and 8 waves share a row.  Rounded additions
+    of the whole sum's size: 1 + 1/2 + 1/4 for eight waves in pairs, about 1/4
+    in the lanes, and the reciprocal: 3.0, and sqrt(3.0) 2^-24 / sqrt(3) over
+    the mean mantissa (1.25) is 0.80 x 2^-24; eight waves one after another
+    make it 4.4, 0.97.  The bar lies between, ten deviations of the estimate
+    from the first."""
+    import torch
+    x = torch.randn(rows, cols, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))
+    y = torch.empty_like(x)
+    be.dispatch_softmax(x, y, bwpp.SoftmaxParams(rows, cols, cols))
+    rms = float((y.double().sum(dim=1) - 1).pow(2).mean().sqrt())
+    assert rms <= (0.88 if cols > 4096 else 0.83) * 2.0 ** -24
